@@ -122,6 +122,7 @@ struct fcfd_ctx {
     double *phiB, *phiS;       // ping-pong phi buffers / stage start copy
     double *l1, *l2;           // stored RK stage sources
     double *s2, *s3, *s0;      // reinit work: lambda numerator/denominator, frozen sign
+    unsigned *band;            // reinit work: counters and lists of the tiles that hold interface-band cells
     double *cx, *cy, *cz;      // CCD second-derivative scratch / cross-derivative temp
     double *dsu, *dsv, *dsw;   // viscous + body force source (sec_part1..3), once per step
     double *un, *vn, *wn;      // predictor output buffer (ping-pong with u, v, w)
@@ -254,6 +255,90 @@ __device__ __forceinline__ double block_max256(double v, double *sh4) {
     return m;
 }
 
+// Tiles of 256 cells that hold cells of the interface band, listed by a
+// reinitialisation stage for its band pass: NXCD lists of `cap` entries, a
+// block appending to list (block id % NXCD), with a counter per stage and
+// list (one counter would serialise the appends).  A list can hold every
+// block that appends to it.  The order of a list does not matter: every band
+// cell is independent of the others.
+struct BandList {
+    unsigned *cnt;    // [3 stages][NXCD]
+    unsigned *tile;   // [NXCD][cap]
+    unsigned cap;
+    // list the calling block's tile when any of its threads holds a band cell
+    __device__ __forceinline__ void append(int stage, int hold, unsigned id) const {
+        hold = __syncthreads_or(hold);
+        if (hold && threadIdx.x + threadIdx.y == 0) {
+            const unsigned q = (blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)) % NXCD;
+            tile[q * cap + atomicAdd(&cnt[stage * NXCD + q], 1u)] = id;
+        }
+    }
+    __device__ __forceinline__ unsigned total(int stage) const {
+        unsigned n = 0;
+#pragma unroll
+        for (unsigned q = 0; q < NXCD; ++q) n += cnt[stage * NXCD + q];
+        return n;
+    }
+    // entry `at` of the lists taken end to end
+    __device__ __forceinline__ unsigned entry(int stage, unsigned at) const {
+        for (unsigned q = 0; q < NXCD; ++q) {
+            const unsigned n = cnt[stage * NXCD + q];
+            if (at < n) return tile[q * cap + at];
+            at -= n;
+        }
+        return 0;
+    }
+    // all counters of the lists (of one stage): by the first block of a launch
+    __device__ __forceinline__ void clear() const {
+        const unsigned t = threadIdx.x + threadIdx.y * blockDim.x;
+        if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && t < 3 * NXCD) cnt[t] = 0u;
+    }
+    __device__ __forceinline__ void clear(int stage) const {
+        const unsigned t = threadIdx.x + threadIdx.y * blockDim.x;
+        if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && t < NXCD) cnt[stage * NXCD + t] = 0u;
+    }
+};
+
+// the band cells of up to BAND_TILES listed tiles (entries first .. of
+// `total`), collected by a 256-thread block so that it can work on them with
+// full waves: cell[0 .. n) = slot * 256 + thread slot within the tile.
+// cell_of(tile, thread slot, i, j, k) places a cell (false: none there),
+// inside(phi) is the band test.
+constexpr int BAND_TILES = 8;
+struct BandCells {
+    unsigned tile[BAND_TILES];
+    unsigned short cell[BAND_TILES * 256];
+    int n;
+};
+template <typename CellOf, typename Inside>
+__device__ __forceinline__ void band_collect(BandCells &sh, const BandList &band, int stage, unsigned first,
+                                             unsigned total, const double *__restrict__ phi, const Geom &G,
+                                             CellOf cell_of, Inside inside) {
+    const int t = threadIdx.x + threadIdx.y * blockDim.x;
+    if (t < BAND_TILES) sh.tile[t] = band.entry(stage, first + t);
+    if (t == 0) sh.n = 0;
+    __syncthreads();
+    double p[BAND_TILES];
+    unsigned have = 0;
+#pragma unroll
+    for (int s = 0; s < BAND_TILES; ++s) {
+        int i, j, k;
+        const bool in = cell_of(sh.tile[s], t, i, j, k) && first + s < total;
+        p[s] = phi[in ? G.id(i, j, k) : G.id(0, 0, 0)];
+        have |= in ? 1u << s : 0u;
+    }
+#pragma unroll
+    for (int s = 0; s < BAND_TILES; ++s) {
+        const bool held = ((have >> s) & 1u) && inside(p[s]);
+        const unsigned long long m = __ballot(held);
+        int base = 0;
+        if (t % WAVE == 0 && m) base = atomicAdd(&sh.n, __popcll(m));
+        base = __shfl(base, 0, WAVE);
+        if (held) sh.cell[base + __popcll(m & ((1ull << (t % WAVE)) - 1ull))] = (unsigned short)(s * 256 + t);
+    }
+    __syncthreads();
+}
+
 // device flag words: [0] unused, [1] reinit done, [2] reinit pseudo-step
 // count, [3] max |grad phi| bits; [FLAG_SHARD0, +NSHARD) per-block max slots.
 // A batched stack holds one such block of FLAG_STRIDE words per case.
@@ -270,6 +355,13 @@ template <int DIM>
 __device__ __forceinline__ int case_of(int k) { return DIM == 2 ? k : 0; }
 
 // launch helpers --------------------------------------------------------
+// 256-thread block for rows of w threads: 64 x 4, or 32 x 8 where that
+// leaves fewer lanes idle past the row end (140 cells: 160 instead of 192
+// threads per row; 70 pairs: 96 instead of 128)
+inline dim3 tile_rows(int w) {
+    const long p64 = (w + 63) / 64 * 64L, p32 = (w + 31) / 32 * 32L;
+    return p32 < p64 ? dim3(32, 8) : dim3(64, 4);
+}
 inline dim3 tile_blk(const fcfd_ctx *c, int kernel) { return dim3(c->tile[kernel][0], c->tile[kernel][1]); }
 // interior cell (i, j, k) of a one-dimensional launch over the nx * ny * nz
 // interior cells in memory order (x fastest; no idle lanes at the row ends
@@ -314,6 +406,17 @@ inline dim3 grid_flat(const Geom &G, int blk) {
 
 inline dim3 grid_interior(const Geom &G, dim3 blk) {
     return dim3((G.nx + blk.x - 1) / blk.x, (G.ny + blk.y - 1) / blk.y, G.nz);
+}
+
+// the band lists of a launch of ntiles 256-thread blocks (the context holds
+// room for the larger of its tiled and its flat launch over the interior)
+inline BandList band_lists(const fcfd_ctx *c, long ntiles) {
+    return BandList{c->band, c->band + 3 * NXCD, (unsigned)((ntiles + NXCD - 1) / NXCD)};
+}
+// blocks that share the listed tiles: up to 4 per CU
+inline dim3 band_grid(const fcfd_ctx *c, long ntiles) {
+    const long n = (ntiles + BAND_TILES - 1) / BAND_TILES, most = 4L * c->ncu;
+    return dim3((unsigned)(n < most ? n : most));
 }
 
 // kernels implemented in the .hip files (host wrappers)

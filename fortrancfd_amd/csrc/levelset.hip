@@ -646,259 +646,260 @@ int ls_advect_f32(fcfd_ctx *c, float *phi, const float *nu, const float *nv, con
 }
 
 // ------------------------------------------------------------- reinit
-// Pass A of one reinitialisation stage: backward differences of phi with
-// the bc() ghost copy as clamped indices (redis_gradient :219-233), one-sided
-// WENO5 values, EPS = 1e-10 (wenojs_flux :295-339), Godunov |grad phi| by the
-// frozen sign (:262-291), then the lambda numerator/denominator terms
-// (redis_lambda :366-380; 2D: lambda = delta, 3D: density weighted).
-template <int DIM>
-__global__ void __launch_bounds__(256) k_redis_a(const double *__restrict__ phi, const double *__restrict__ S0,
-                                                 double *__restrict__ grad, double *__restrict__ s2,
-                                                 double *__restrict__ s3, const unsigned long long *__restrict__ done,
-                                                 Geom G, double w, double r12, int btn) {
-    int bx_, by_, bz_;
-    xcd_block(bx_, by_, bz_);
-    const int i = bx_ * blockDim.x + threadIdx.x, j = by_ * blockDim.y + threadIdx.y, k = bz_;
-    if (done && done[(long)case_of<DIM>(k) * FLAG_STRIDE + 1]) return;
-    if (i >= G.nx || j >= G.ny) return;
-    const long id = G.id(i, j, k);
-    const int n[3] = {G.nx, G.ny, G.nz};
-    const int pos[3] = {i, j, k};
-    const long st[3] = {1, G.sx, G.sxy};
-    const double ih[3] = {1.0 / G.dx, 1.0 / G.dy, 1.0 / G.dz};
-    double sel[3];
-    // phi at pos-4 .. pos+3 of the three lines, all loads before any branch
-    // (pos-4 is clamped to the outermost ghost layer; that value is never
-    // selected below)
-    double gw[3][8];
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-        gw[d][0] = phi[id + (long)(max(pos[d] - 4, -3) - pos[d]) * st[d]];
-#pragma unroll
-        for (int r = 1; r < 8; ++r) gw[d][r] = phi[id + (long)(r - 4) * st[d]];
-    }
-    const bool pos_sign = S0[id] >= 0.0;
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-        // D-phi at pos-3 .. pos+3, ghost entries copying the boundary one:
-        // nr[m] = D(clamp(pos - 3 + m, 0, n - 1)) = dw[clamp(m, 3 - pos, n + 2 - pos)]
-        // with dw[m] = D(pos - 3 + m) the window's neighbour differences
-        double nr[7];
-#pragma unroll
-        for (int m = 0; m < 7; ++m) nr[m] = (gw[d][m + 1] - gw[d][m]) * ih[d];
-        if (pos[d] < 3 || pos[d] > n[d] - 4) clamp_window(nr, 3 - pos[d], n[d] + 2 - pos[d]);
-        const double EPS = 1.0e-10;
-        double fm = weno_left(nr[1], nr[2], nr[3], nr[4], nr[5], EPS);   // tdata%s2
-        double fp = weno_right(nr[2], nr[3], nr[4], nr[5], nr[6], EPS);  // tdata%s1
-        if (pos_sign) sel[d] = fmax(-fmin(fp, 0.0), fmax(fm, 0.0));
-        else sel[d] = fmax(fmax(fp, 0.0), -fmin(fm, 0.0));
-    }
-    double g = DIM == 3 ? sqrt(sel[0] * sel[0] + sel[1] * sel[1] + sel[2] * sel[2])
-                        : sqrt(sel[0] * sel[0] + sel[1] * sel[1]);
-    grad[id] = g;
-    if (btn != 0) {
-        double hh, dd;
-        lsfun(phi[id], w, hh, dd);
-        double lam = DIM == 3 ? (2.0 * (1.0 - r12) * hh + r12) * dd : dd;
-        s2[id] = lam * S0[id] * (g - 1.0);
-        s3[id] = g * dd * lam;
+// Interface band of the reinitialisation: the cells where lsfun's delta can
+// be non-zero.  The threshold is tested with the reciprocal width, which may
+// differ from lsfun's quotient by an ulp; a cell at the threshold has
+// delta = 0 either way (1 + cos(pi x) rounds to 0 within ~1e-8 of |x| = 1).
+// NaN counts as inside, as in lsfun.
+__device__ __forceinline__ bool in_band(double phi, double iw) {
+    const double x = phi * iw;
+    return !(x > 1.0 - 1.0e-12) && !(x < -1.0 + 1.0e-12);
+}
+
+// source of one stage and the increment-form SSP-RK3 update (redis_solver
+// :150-208); l1o, l2o the stored sources of the earlier stages
+template <int STAGE>
+__device__ __forceinline__ double redis_update(double p0, double l, double l1o, double l2o, double rdt) {
+    double src;
+    if (STAGE == 0) src = l;
+    else if (STAGE == 1) src = (-3.0 * l1o + l) / 4.0;
+    else src = (-l1o - l2o + 8.0 * l) / 12.0;
+    return p0 - rdt * src;
+}
+
+// max|phi - phi_start| of a block into one of NSHARD slots of the case's
+// flags (reinit stop test :42-54): a single slot would serialise tens of
+// thousands of atomics; the max of non-negative doubles is order
+// independent, compared as bit patterns
+__device__ __forceinline__ void redis_shard_max(double err, double *sh4, unsigned long long *flags) {
+    const double m = block_max256(err, sh4);
+    if (threadIdx.x + threadIdx.y == 0) {
+        const unsigned b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        atomicMax(&flags[FLAG_SHARD0 + b % NSHARD], (unsigned long long)__double_as_longlong(m));
     }
 }
 
-// Pass B: 3^d weighted sums (centre weight 16 in 2D, 51 in 3D, bc() copy as
-// clamped indices), correction s1 (redis_lambda :385-408), stage source and
-// in-place increment-form SSP-RK3 update (redis_solver :150-208).  The last
-// stage also folds max|phi - phi_start| into the flag shards (reinit stop
-// test :42-54).
-template <int DIM>
-__global__ void __launch_bounds__(256) k_redis_b(double *__restrict__ phi, const double *__restrict__ S0,
-                                                 const double *__restrict__ grad, const double *__restrict__ s2,
-                                                 const double *__restrict__ s3, double *__restrict__ l1,
-                                                 double *__restrict__ l2, const double *__restrict__ phis,
-                                                 unsigned long long *__restrict__ flags, Geom G, double w,
-                                                 double rdt, int btn, int stage) {
+constexpr int REDIS_GRADIENT = 3;  // STAGE of the gradient-only pass
+
+// One reinitialisation stage from phi into out (another array: the stencil
+// reads neighbours): backward differences of phi with the bc() ghost copy as
+// clamped indices (redis_gradient :219-233), one-sided WENO5 values,
+// EPS = 1e-10 (wenojs_flux :295-339), Godunov |grad phi| by the frozen sign
+// (:262-291), then the stage source and update.  The mass constraint enters
+// as (a / b) delta with delta = 0 outside the interface band, so every cell
+// outside it is finished here; a band cell only stores |grad phi| and its
+// constraint terms (redis_lambda :366-380; 2D: lambda = delta, 3D: density
+// weighted) and its tile is listed for k_redis_band.  The two-pass form stored
+// three values per cell and read them back: at 256^3 346 + 355 us a stage
+// and a 62 us copy of phi per pseudo step.
+// lo: the lowest index phi is read at, -1 where phi's ghosts are valid
+// (the first stage: phi(-1) may differ from a copy of phi(0)) and 0 for the
+// stage buffers, whose ghosts are not filled; every ghost that bc() would
+// fill reads its clamped cell.
+template <int DIM, int STAGE, bool BTN>
+__global__ void __launch_bounds__(256) k_redis_stage(const double *__restrict__ phi, double *__restrict__ out,
+                                                     const double *__restrict__ S0, double *__restrict__ grad,
+                                                     double *__restrict__ s2, double *__restrict__ s3,
+                                                     double *__restrict__ l1, double *__restrict__ l2,
+                                                     BandList band, unsigned long long *flags, Geom G,
+                                                     double w, double iw, double r12, double rdt, int lo) {
     int bx_, by_, bz_;
-    xcd_block(bx_, by_, bz_);
+    if (DIM == 3) xcd_block_slab(bx_, by_, bz_, 8);
+    else xcd_block(bx_, by_, bz_);
     const int i = bx_ * blockDim.x + threadIdx.x, j = by_ * blockDim.y + threadIdx.y, k = bz_;
     flags += (long)case_of<DIM>(k) * FLAG_STRIDE;   // this case's flag block (a block covers one slice)
-    if (flags[1]) return;
-    bool in = i < G.nx && j < G.ny;
-    double err = 0.0;
-    if (in) {
-        const long id = G.id(i, j, k);
-        double hh, dd;
-        double p0 = phi[id];
-        lsfun(p0, w, hh, dd);
-        double s1 = 0.0;
-        if (btn != 0) {
-            const double wc = DIM == 3 ? 51.0 : 16.0;
-            double a = wc * s2[id], b = wc * s3[id];
-            const int kl = DIM == 3 ? -1 : 0, kh = DIM == 3 ? 1 : 0;
-            for (int kk = kl; kk <= kh; ++kk) {
-                int kq = DIM == 3 ? clampi(k + kk, 0, G.nz - 1) : k;
-                for (int jj = -1; jj <= 1; ++jj) {
-                    int jq = clampi(j + jj, 0, G.ny - 1);
-                    for (int ii = -1; ii <= 1; ++ii) {
-                        int iq = clampi(i + ii, 0, G.nx - 1);
-                        long o = G.id(iq, jq, kq);
-                        a = a + s2[o];
-                        b = b + s3[o];
-                    }
-                }
-            }
-            if (fabs(b) > 1.0e-12) s1 = a / b * dd;
-        }
-        double S = S0[id];
-        double l = (S - s1) * grad[id] - S, src;
-        if (stage == 0) { l1[id] = l; src = l; }
-        else if (stage == 1) { l2[id] = l; src = (-3.0 * l1[id] + l) / 4.0; }
-        else { src = (-l1[id] - l2[id] + 8.0 * l) / 12.0; }
-        double pn = p0 - rdt * src;
-        phi[id] = pn;
-        if (stage == 2) err = fabs(phis[id] - pn);
-    }
-    if (stage == 2) {
-        // block max, then one atomic per block into one of NSHARD slots (a
-        // single slot serialises tens of thousands of atomics); max of
-        // non-negative doubles is order independent, compared as bit patterns
-        __shared__ double sh[4];
-        const double m = block_max256(err, sh);
-        if (threadIdx.x + threadIdx.y == 0) {
-            const unsigned b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-            atomicMax(&flags[FLAG_SHARD0 + b % NSHARD], (unsigned long long)__double_as_longlong(m));
-        }
-    }
-}
-
-// Pass B in 3D, RB_KC planes per thread.  The constraint term is
-// (a / b) delta, and delta = 0 off the interface band, so only band cells
-// (a thin shell, a few % of the cells) read the 3x3x3 sums of s2 and s3,
-// as 3x3 plane sums of planes k-1, k, k+1 (clamped).  Same update as
-// k_redis_b; the sums associate differently (plane by plane), a change of
-// rounding only.  The stage and btn are template arguments so that every
-// load of a plane is issued at the top of its iteration.
-constexpr int RB_KC = 16;
-template <int STAGE, bool BTN>
-__global__ void __launch_bounds__(256) k_redis_b_km(double *__restrict__ phi, const double *__restrict__ S0,
-                                                    const double *__restrict__ grad, const double *__restrict__ s2,
-                                                    const double *__restrict__ s3, double *__restrict__ l1,
-                                                    double *__restrict__ l2, const double *__restrict__ phis,
-                                                    unsigned long long *__restrict__ flags, Geom G, double w,
-                                                    double rdt) {
-    int bx_, by_, bz_;
-    xcd_block(bx_, by_, bz_);
-    const int i = bx_ * blockDim.x + threadIdx.x, j = by_ * blockDim.y + threadIdx.y;
-    const int k0 = bz_ * RB_KC, k1 = min(k0 + RB_KC, G.nz);
-    if (flags[1]) return;
+    if (STAGE != REDIS_GRADIENT && flags[1]) return;
     const bool in = i < G.nx && j < G.ny;
     double err = 0.0;
+    int hold = 0;
     if (in) {
-        const int im = max(i - 1, 0), ip = min(i + 1, G.nx - 1), jm = max(j - 1, 0), jp = min(j + 1, G.ny - 1);
-        const long c0 = G.id(i, j, 0);
-        const long o[9] = {G.id(im, jm, 0) - c0, G.id(i, jm, 0) - c0, G.id(ip, jm, 0) - c0,
-                           G.id(im, j, 0) - c0,  0,                    G.id(ip, j, 0) - c0,
-                           G.id(im, jp, 0) - c0, G.id(i, jp, 0) - c0,  G.id(ip, jp, 0) - c0};
-        auto plane = [&](long c, double &a, double &b) {
-            double t2[9], t3[9];
+        const long id = G.id(i, j, k);
+        const int n[3] = {G.nx, G.ny, G.nz};
+        const int pos[3] = {i, j, k};
+        const long st[3] = {1, G.sx, G.sxy};
+        const double ih[3] = {1.0 / G.dx, 1.0 / G.dy, 1.0 / G.dz};
+        // phi at pos-4 .. pos+3 of the three lines and the cell's other
+        // operands, all loads before any branch
+        double gw[3][8];
 #pragma unroll
-            for (int q = 0; q < 9; ++q) {
-                t2[q] = s2[c + o[q]];
-                t3[q] = s3[c + o[q]];
-            }
-            a = 0.0;
-            b = 0.0;
+        for (int d = 0; d < DIM; ++d)
 #pragma unroll
-            for (int q = 0; q < 9; ++q) {
-                a += t2[q];
-                b += t3[q];
+            for (int r = 0; r < 8; ++r) {
+                const int q = r < 4 ? max(pos[d] + r - 4, lo) : min(pos[d] + r - 4, n[d] - 1);
+                gw[d][r] = phi[id + (long)(q - pos[d]) * st[d]];
             }
-        };
-        long id = G.id(i, j, k0);
-        for (int k = k0; k < k1; ++k, id += G.sxy) {
-            // every load of the plane first
-            const double p0 = phi[id], S = S0[id], gr = grad[id];
-            const double l1o = STAGE >= 1 ? l1[id] : 0.0, l2o = STAGE == 2 ? l2[id] : 0.0;
-            const double pst = STAGE == 2 ? phis[id] : 0.0;
-            double hh, dd;
-            lsfun(p0, w, hh, dd);
-            // the constraint enters as (a / b) delta: only cells of the
-            // interface band (delta != 0) read the 27-point sums
-            double s1 = 0.0;
-            if (BTN && dd != 0.0) {
-                double am, bm, ac, bc, ap = 0.0, bp = 0.0;
-                plane(id - (k > 0 ? G.sxy : 0), am, bm);
-                plane(id, ac, bc);
-                if (k + 1 <= G.nz - 1) plane(id + G.sxy, ap, bp);
-                else { ap = ac; bp = bc; }
-                const double a = 51.0 * s2[id] + am + ac + ap, b = 51.0 * s3[id] + bm + bc + bp;
-                if (fabs(b) > 1.0e-12) s1 = a / b * dd;
+        const double S = S0[id];
+        const double l1o = STAGE == 1 || STAGE == 2 ? l1[id] : 0.0, l2o = STAGE == 2 ? l2[id] : 0.0;
+        const double pst = STAGE == 2 ? out[id] : 0.0;   // the last stage writes over phi_start
+        const double p0 = gw[0][4];
+        const bool pos_sign = S >= 0.0;
+        double sel[3];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            // D-phi at pos-3 .. pos+3, ghost entries copying the boundary one:
+            // nr[m] = D(clamp(pos - 3 + m, 0, n - 1)) = dw[clamp(m, 3 - pos, n + 2 - pos)]
+            // with dw[m] = D(pos - 3 + m) the window's neighbour differences
+            double nr[7];
+#pragma unroll
+            for (int m = 0; m < 7; ++m) nr[m] = (gw[d][m + 1] - gw[d][m]) * ih[d];
+            if (pos[d] < 3 || pos[d] > n[d] - 4) clamp_window(nr, 3 - pos[d], n[d] + 2 - pos[d]);
+            const double EPS = 1.0e-10;
+            double fm = weno_left(nr[1], nr[2], nr[3], nr[4], nr[5], EPS);   // tdata%s2
+            double fp = weno_right(nr[2], nr[3], nr[4], nr[5], nr[6], EPS);  // tdata%s1
+            if (pos_sign) sel[d] = fmax(-fmin(fp, 0.0), fmax(fm, 0.0));
+            else sel[d] = fmax(fmax(fp, 0.0), -fmin(fm, 0.0));
+        }
+        const double g = DIM == 3 ? sqrt(sel[0] * sel[0] + sel[1] * sel[1] + sel[2] * sel[2])
+                                  : sqrt(sel[0] * sel[0] + sel[1] * sel[1]);
+        if (STAGE >= 2) grad[id] = g;   // grad%now holds the last stage's
+        if (STAGE != REDIS_GRADIENT) {
+            if (BTN && in_band(p0, iw)) {
+                double hh, dd;
+                lsfun(p0, w, hh, dd);
+                const double lam = DIM == 3 ? (2.0 * (1.0 - r12) * hh + r12) * dd : dd;
+                grad[id] = g;
+                s2[id] = lam * S * (g - 1.0);
+                s3[id] = g * dd * lam;
+                hold = 1;
+            } else {
+                const double l = S * g - S;
+                const double pn = redis_update<STAGE>(p0, l, l1o, l2o, rdt);
+                if (STAGE == 0) l1[id] = l;
+                if (STAGE == 1) l2[id] = l;
+                out[id] = pn;
+                if (STAGE == 2) err = fabs(pst - pn);
             }
-            const double l = (S - s1) * gr - S;
-            double src;
-            if (STAGE == 0) { l1[id] = l; src = l; }
-            else if (STAGE == 1) { l2[id] = l; src = (-3.0 * l1o + l) / 4.0; }
-            else { src = (-l1o - l2o + 8.0 * l) / 12.0; }
-            const double pn = p0 - rdt * src;
-            phi[id] = pn;
-            if (STAGE == 2) err = fmax(err, fabs(pst - pn));
         }
     }
+    if (BTN && STAGE != REDIS_GRADIENT)
+        band.append(STAGE, hold, (unsigned)bx_ + gridDim.x * ((unsigned)by_ + gridDim.y * (unsigned)bz_));
     if (STAGE == 2) {
         __shared__ double sh[4];
-        const double m = block_max256(err, sh);
-        if (threadIdx.x + threadIdx.y == 0) {
-            const unsigned b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-            atomicMax(&flags[FLAG_SHARD0 + b % NSHARD], (unsigned long long)__double_as_longlong(m));
-        }
+        redis_shard_max(err, sh, flags);
     }
 }
 
-static void launch_redis_b_km(fcfd_ctx *c, dim3 g, dim3 blk, double *phi, const double *grad, int btn, int stage) {
-    const Geom &G = c->G;
-    const double w = c->pr.ls_wid, rdt = c->pr.rdt;
-#define FCFD_RB(S_, B_)                                                                                              \
-    hipLaunchKernelGGL((k_redis_b_km<S_, B_>), g, blk, 0, c->stream, phi, c->s0, grad, c->s2, c->s3, c->l1, c->l2, \
-                       c->phiS, c->flag, G, w, rdt)
-    if (btn) {
-        if (stage == 0) FCFD_RB(0, true);
-        else if (stage == 1) FCFD_RB(1, true);
-        else FCFD_RB(2, true);
-    } else {
-        if (stage == 0) FCFD_RB(0, false);
-        else if (stage == 1) FCFD_RB(1, false);
-        else FCFD_RB(2, false);
+// The band cells of a stage: 3^d weighted sums of the constraint terms
+// (centre weight 16 in 2D, 51 in 3D, bc() copy as clamped indices), the
+// correction (redis_lambda :385-408), source and update as in k_redis_stage.
+// A term outside the band is 0 (its delta is) and is not stored: it is read
+// all the same and not selected, so that the loads of a plane issue together.
+// A block takes BAND_TILES listed tiles at a time (tiles of gx x gy blocks a
+// plane) and works on their band cells with full waves (band_collect): a
+// band is a few cells thick, so about a tenth of a listed tile's lanes hold
+// one.  18 us at 160 x 144 x 200.  One column of 16 planes per thread, tangent to the band,
+// took 350 us at 256^3 for 0.4 % of the cells; one tile per block 53 us at
+// 160 x 144 x 200.
+template <int DIM, int STAGE>
+__global__ void __launch_bounds__(256) k_redis_band(const double *__restrict__ phi, double *__restrict__ out,
+                                                    const double *__restrict__ S0, const double *__restrict__ grad,
+                                                    const double *__restrict__ s2, const double *__restrict__ s3,
+                                                    double *__restrict__ l1, double *__restrict__ l2, BandList band,
+                                                    unsigned long long *flags, Geom G, double w, double iw,
+                                                    double rdt, unsigned gx, unsigned gy) {
+    __shared__ BandCells sh;
+    __shared__ unsigned long long s_err[BAND_TILES];
+    const int t = threadIdx.x + threadIdx.y * blockDim.x;
+    const unsigned total = band.total(STAGE);
+    // cell of thread slot th of listed tile number `tile`
+    auto cell_of = [&](unsigned tile, int th, int &i, int &j, int &k) {
+        const unsigned r = tile / gx, k_ = r / gy;
+        const int tx = th % (int)blockDim.x, ty = th / (int)blockDim.x;
+        i = (int)((tile - r * gx) * blockDim.x) + tx;
+        j = (int)((r - k_ * gy) * blockDim.y) + ty;
+        k = (int)k_;
+        return i < G.nx && j < G.ny;
+    };
+    for (unsigned g = blockIdx.x * BAND_TILES; g < total; g += gridDim.x * BAND_TILES) {
+        if (t < BAND_TILES) s_err[t] = 0ull;
+        band_collect(sh, band, STAGE, g, total, phi, G, cell_of, [&](double p) { return in_band(p, iw); });
+        for (int c = t; c < sh.n; c += 256) {
+            const int slot = sh.cell[c] / 256;
+            int i, j, k;
+            cell_of(sh.tile[slot], sh.cell[c] % 256, i, j, k);
+            const long id = G.id(i, j, k);
+            const double p0 = phi[id];
+            const int is[3] = {max(i - 1, 0), i, min(i + 1, G.nx - 1)};
+            const int js[3] = {max(j - 1, 0), j, min(j + 1, G.ny - 1)};
+            double hh, dd;
+            lsfun(p0, w, hh, dd);
+            double a = (DIM == 3 ? 51.0 : 16.0) * s2[id], b = (DIM == 3 ? 51.0 : 16.0) * s3[id];
+            const double S = S0[id], gr = grad[id];
+            const double l1o = STAGE >= 1 ? l1[id] : 0.0, l2o = STAGE == 2 ? l2[id] : 0.0;
+            const double pst = STAGE == 2 ? out[id] : 0.0;
+#pragma unroll
+            for (int kk = 0; kk < (DIM == 3 ? 3 : 1); ++kk) {
+                const int kq = DIM == 3 ? clampi(k + kk - 1, 0, G.nz - 1) : k;
+                double ph[9], ta[9], tb[9];
+#pragma unroll
+                for (int m = 0; m < 9; ++m) {
+                    const long o = G.id(is[m % 3], js[m / 3], kq);
+                    ph[m] = phi[o];
+                    ta[m] = s2[o];
+                    tb[m] = s3[o];
+                }
+                double pa = 0.0, pb = 0.0;
+#pragma unroll
+                for (int m = 0; m < 9; ++m) {
+                    const bool held = in_band(ph[m], iw);
+                    const double xa = held ? ta[m] : 0.0, xb = held ? tb[m] : 0.0;
+                    if (DIM == 3) {
+                        pa += xa;
+                        pb += xb;
+                    } else {
+                        a = a + xa;
+                        b = b + xb;
+                    }
+                }
+                if (DIM == 3) {
+                    a += pa;
+                    b += pb;
+                }
+            }
+            const double s1 = fabs(b) > 1.0e-12 ? a / b * dd : 0.0;
+            const double l = (S - s1) * gr - S, pn = redis_update<STAGE>(p0, l, l1o, l2o, rdt);
+            if (STAGE == 0) l1[id] = l;
+            if (STAGE == 1) l2[id] = l;
+            out[id] = pn;
+            if (STAGE == 2)   // max of non-negative doubles as bit patterns
+                atomicMax(&s_err[slot], (unsigned long long)__double_as_longlong(fabs(pst - pn)));
+        }
+        __syncthreads();
+        if (STAGE == 2 && t < BAND_TILES && g + t < total) {
+            const int q = case_of<DIM>((int)(sh.tile[t] / gx / gy));
+            atomicMax(&flags[(long)q * FLAG_STRIDE + FLAG_SHARD0 + sh.tile[t] % NSHARD], s_err[t]);
+        }
+        __syncthreads();
     }
-#undef FCFD_RB
 }
 
 // end of one pseudo step: count it, stop when the max over the shards is
-// <= tol, clear the shards (one block of NSHARD threads per case)
-__global__ void __launch_bounds__(NSHARD) k_redis_check(unsigned long long *flags, double tol) {
+// <= tol, clear the shards (one block of NSHARD threads per case); the
+// case's done word also goes to poll[case], pinned host memory, so that the
+// host's poll needs no copy launch.  Clears the band lists' counters.
+__global__ void __launch_bounds__(NSHARD) k_redis_check(unsigned long long *flags, double tol,
+                                                        unsigned long long *poll, BandList band) {
     __shared__ double sh[4];
     flags += (long)blockIdx.x * FLAG_STRIDE;
-    if (flags[1]) return;
     const int t = threadIdx.x;
+    band.clear();
+    if (flags[1]) {
+        if (t == 0) poll[blockIdx.x] = 1ull;
+        return;
+    }
     const double e = __longlong_as_double((long long)flags[FLAG_SHARD0 + t]);
     const double err = block_max256(e, sh);
     flags[FLAG_SHARD0 + t] = 0ull;
     if (t == 0) {
         flags[2] += 1;
         if (err <= tol) flags[1] = 1;
+        poll[blockIdx.x] = err <= tol ? 1ull : 0ull;
     }
 }
 
-__global__ void k_copy_interior(double *__restrict__ dst, const double *__restrict__ src,
-                                const unsigned long long *__restrict__ done, Geom G) {
-    int bx_, by_, bz_;
-    xcd_block(bx_, by_, bz_);
-    const int i = bx_ * blockDim.x + threadIdx.x, j = by_ * blockDim.y + threadIdx.y, k = bz_;
-    if (done && done[(G.dim == 2 ? (long)k : 0L) * FLAG_STRIDE + 1]) return;
-    if (i >= G.nx || j >= G.ny) return;
-    long id = G.id(i, j, k);
-    dst[id] = src[id];
-}
-
-__global__ void k_sign_init(const double *__restrict__ phi, double *__restrict__ S0, Geom G, double w, int btn) {
+__global__ void k_sign_init(const double *__restrict__ phi, double *__restrict__ S0, Geom G, double w, int btn,
+                            BandList band) {
+    band.clear();
     int bx_, by_, bz_;
     xcd_block(bx_, by_, bz_);
     const int i = bx_ * blockDim.x + threadIdx.x, j = by_ * blockDim.y + threadIdx.y, k = bz_;
@@ -937,24 +938,58 @@ __global__ void k_scale_by_flag(double *__restrict__ phi, const unsigned long lo
     phi[id] = phi[id] / gmax;
 }
 
+// one stage: k_redis_stage on every cell, then the listed tiles' band cells
+template <int DIM, int STAGE>
+static int redis_stage(fcfd_ctx *c, dim3 grd, dim3 blk, int btn, const double *in, double *out, int lo) {
+    const Geom &G = c->G;
+    const double w = c->pr.ls_wid, iw = 1.0 / w, r12 = c->pr.rho_12, rdt = c->pr.rdt;
+    double *grad = c->f[FCFD_GRAD];
+    const long nt = (long)grd.x * grd.y * grd.z;
+    const BandList band = band_lists(c, nt);
+    {
+        ProfScope ps_(c, R_REDIS_A);
+        if (btn)
+            hipLaunchKernelGGL((k_redis_stage<DIM, STAGE, true>), grd, blk, 0, c->stream, in, out, c->s0, grad, c->s2,
+                               c->s3, c->l1, c->l2, band, c->flag, G, w, iw, r12, rdt, lo);
+        else
+            hipLaunchKernelGGL((k_redis_stage<DIM, STAGE, false>), grd, blk, 0, c->stream, in, out, c->s0, grad,
+                               c->s2, c->s3, c->l1, c->l2, band, c->flag, G, w, iw, r12, rdt, lo);
+    }
+    FCFD_CHECK(hipGetLastError());
+    if constexpr (STAGE != REDIS_GRADIENT) {
+        if (btn) {
+            ProfScope ps_(c, R_REDIS_B);
+            hipLaunchKernelGGL((k_redis_band<DIM, STAGE>), band_grid(c, nt), blk, 0, c->stream, in, out, c->s0, grad,
+                               c->s2, c->s3, c->l1, c->l2, band, c->flag, G, w, iw, rdt, grd.x, grd.y);
+            FCFD_CHECK(hipGetLastError());
+        }
+    }
+    return FCFD_OK;
+}
+
+template <int DIM>
+static int redis_pseudo_step(fcfd_ctx *c, dim3 grd, dim3 blk, int btn, int lo) {
+    double *phi = c->f[FCFD_PHI];   // phi_start, overwritten by the last stage
+    FCFD_TRY((redis_stage<DIM, 0>(c, grd, blk, btn, phi, c->phiB, lo)));
+    FCFD_TRY((redis_stage<DIM, 1>(c, grd, blk, btn, c->phiB, c->phiS, 0)));
+    return redis_stage<DIM, 2>(c, grd, blk, btn, c->phiS, phi, 0);
+}
+
 int redis(fcfd_ctx *c, int btn, int *iters) {
     const Geom &G = c->G;
-    dim3 blk(64, 4), grd = grid_interior(G, blk);
+    const dim3 blk = tile_rows(G.nx), grd = grid_interior(G, blk);
     double *phi = c->f[FCFD_PHI], *grad = c->f[FCFD_GRAD];
-    const double w = c->pr.ls_wid, r12 = c->pr.rho_12, rdt = c->pr.rdt;
+    const double w = c->pr.ls_wid, rdt = c->pr.rdt;
+    int lo = -1;   // the caller's ghosts until a bc() or a stage has replaced them
     FCFD_CHECK(hipMemsetAsync(c->flag, 0, (size_t)FLAG_STRIDE * c->nb * sizeof(unsigned long long), c->stream));
     // level_set_redis_init / stable (:67-136)
-    hipLaunchKernelGGL(k_sign_init, grd, blk, 0, c->stream, phi, c->s0, G, w, btn);
+    hipLaunchKernelGGL(k_sign_init, grd, blk, 0, c->stream, phi, c->s0, G, w, btn, band_lists(c, 0));
     if (btn == 0) {
-        if (G.dim == 3)
-            hipLaunchKernelGGL(k_redis_a<3>, grd, blk, 0, c->stream, phi, c->s0, grad, c->s2, c->s3, nullptr, G, w,
-                               r12, 0);
-        else
-            hipLaunchKernelGGL(k_redis_a<2>, grd, blk, 0, c->stream, phi, c->s0, grad, c->s2, c->s3, nullptr, G, w,
-                               r12, 0);
+        if (G.dim == 3) FCFD_TRY((redis_stage<3, REDIS_GRADIENT>(c, grd, blk, 0, phi, nullptr, lo)));
+        else FCFD_TRY((redis_stage<2, REDIS_GRADIENT>(c, grd, blk, 0, phi, nullptr, lo)));
         hipLaunchKernelGGL(k_max_interior, grd, blk, 0, c->stream, grad, c->flag, G);
         hipLaunchKernelGGL(k_scale_by_flag, grd, blk, 0, c->stream, phi, c->flag, G);
-        FCFD_TRY(bc_scalar(c, phi));
+        lo = 0;   // the scaled phi's ghosts are bc() copies
     }
     // pseudo-time budget: the reference stops once the accumulated time exceeds
     // timestop (:18-28,54); replay that accumulation to fix the launch count
@@ -975,10 +1010,9 @@ int redis(fcfd_ctx *c, int btn, int *iters) {
         if (nmax > 10000000) return FCFD_ERR_ARG;
     }
     const double tol = G.dim == 3 ? 1.0e-5 : 1.0e-8;
-    const dim3 gkm(grd.x, grd.y, (G.nz + RB_KC - 1) / RB_KC);
     // The stop test runs on the device (k_redis_check); a stopped case's
-    // kernels return at once.  The done words of pseudo-step `it` are copied
-    // to the host behind it, and before step it+2 is queued the host reads
+    // kernels return at once.  The done words of pseudo-step `it` reach the
+    // host behind it, and before step it+2 is queued the host reads
     // them, so it stops queueing once every case has stopped while one step
     // stays queued ahead.  Slots of flag_host past the 4 nb words read below.
     for (int q = 0; q < 2; ++q)
@@ -991,32 +1025,14 @@ int redis(fcfd_ctx *c, int btn, int *iters) {
             for (int q = 0; q < c->nb; ++q) all = all && poll[it & 1][q] != 0ull;
             if (all) break;
         }
-        hipLaunchKernelGGL(k_copy_interior, grd, blk, 0, c->stream, c->phiS, phi, c->flag, G);
-        for (int s = 0; s < 3; ++s) {
-            {
-                ProfScope ps_(c, R_REDIS_A);
-                if (G.dim == 3)
-                    hipLaunchKernelGGL(k_redis_a<3>, grd, blk, 0, c->stream, phi, c->s0, grad, c->s2, c->s3, c->flag,
-                                       G, w, r12, btn);
-                else
-                    hipLaunchKernelGGL(k_redis_a<2>, grd, blk, 0, c->stream, phi, c->s0, grad, c->s2, c->s3, c->flag,
-                                       G, w, r12, btn);
-            }
-            {
-                ProfScope ps_(c, R_REDIS_B);
-                if (G.dim == 3)
-                    launch_redis_b_km(c, gkm, blk, phi, grad, btn, s);
-                else
-                    hipLaunchKernelGGL(k_redis_b<2>, grd, blk, 0, c->stream, phi, c->s0, grad, c->s2, c->s3, c->l1,
-                                       c->l2, c->phiS, c->flag, G, w, rdt, btn, s);
-            }
-            FCFD_CHECK(hipGetLastError());
-            FCFD_TRY(bc_scalar(c, phi));
-        }
-        hipLaunchKernelGGL(k_redis_check, dim3(c->nb), dim3(NSHARD), 0, c->stream, c->flag, tol);
-        FCFD_TRY(gather_to_host(c, poll[it & 1], c->flag + 1, FLAG_STRIDE, 1, c->nb));
+        if (G.dim == 3) FCFD_TRY(redis_pseudo_step<3>(c, grd, blk, btn, it == 0 ? lo : 0));
+        else FCFD_TRY(redis_pseudo_step<2>(c, grd, blk, btn, it == 0 ? lo : 0));
+        hipLaunchKernelGGL(k_redis_check, dim3(c->nb), dim3(NSHARD), 0, c->stream, c->flag, tol, poll[it & 1],
+                           band_lists(c, 0));
+        FCFD_CHECK(hipGetLastError());
         FCFD_CHECK(hipEventRecord(c->redis_ev[it & 1], c->stream));
     }
+    FCFD_TRY(bc_scalar(c, phi));
     // words 0..3 of every case's flag block
     FCFD_TRY(gather_to_host(c, c->flag_host, c->flag, FLAG_STRIDE, 4, c->nb));
     FCFD_CHECK(hipStreamSynchronize(c->stream));

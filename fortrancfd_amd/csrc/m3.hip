@@ -98,8 +98,9 @@ __global__ void k_m3_adv_stage(double *__restrict__ phi, const double *__restric
     }
 }
 
-// sgnf (LS_REDISTANCE.F90:360-376)
-__global__ void k_m3_sign(const double *__restrict__ phi, double *__restrict__ S, Geom G, double w) {
+// sgnf (LS_REDISTANCE.F90:360-376); clears the band lists' counters
+__global__ void k_m3_sign(const double *__restrict__ phi, double *__restrict__ S, Geom G, double w, BandList band) {
+    band.clear();
     int i, j, k;
     if (!cell_of_flat(G, i, j, k)) return;
     const long id = G.id(i, j, k);
@@ -118,15 +119,19 @@ __device__ __forceinline__ double sq(double x) { return x * x; }
 // the one-sided WENO values of the backward differences along a line:
 // F(m) = (T(m) - T(m-1)) / h for interior m, F of a ghost index = F of the
 // nearest interior index (FV_DERI's bc3d); n the line's interior length.
-// The seven values T(i-3 .. i+3) lie inside the 3 ghost layers for every
-// i, and every clamped difference is one of their six neighbour
-// differences: F(clamp(i-2+q)) = d[clamp(q, 2-i, n+1-i)].  So the loads
-// take no branch, the caller issues the three lines of a cell together
-// (m3_line_load), and only the cells within two of a wall remap their
-// differences.
-__device__ __forceinline__ void m3_line_load(const double *__restrict__ T, long id, long st, double (&g)[7]) {
+// The seven values T(i-3 .. i+3) are read at indices clamped to [lo, n-1]
+// (lo as in k_redis_stage: -1 where T's ghosts are valid, else 0), and every
+// clamped difference is one of their six neighbour differences:
+// F(clamp(i-2+q)) = d[clamp(q, 2-i, n+1-i)].  So the loads take no branch,
+// the caller issues the three lines of a cell together (m3_line_load), and
+// only the cells within two of a wall remap their differences.
+__device__ __forceinline__ void m3_line_load(const double *__restrict__ T, long id, long st, int i, int n, int lo,
+                                             double (&g)[7]) {
 #pragma unroll
-    for (int r = 0; r < 7; ++r) g[r] = T[id + (long)(r - 3) * st];
+    for (int r = 0; r < 7; ++r) {
+        const int q = r < 3 ? max(i + r - 3, lo) : min(i + r - 3, n - 1);
+        g[r] = T[id + (long)(q - i) * st];
+    }
 }
 
 __device__ __forceinline__ void m3_line_weno(const double (&g)[7], int i, int n, double ih, double &up, double &um) {
@@ -138,94 +143,138 @@ __device__ __forceinline__ void m3_line_weno(const double (&g)[7], int i, int n,
     up = weno_right(f[1], f[2], f[3], f[4], f[5], kEps);
 }
 
-// GRADFI + the pointwise part of RIS_MASS (LS_REDISTANCE.F90:148-238):
-// |grad T| by Godunov on the WENO values, delta of T, and the constraint
-// terms a = SGN delta (|grad| - 1), b = |grad| delta^2
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4)))
-k_m3_redis_a(const double *__restrict__ T, const double *__restrict__ S, double *__restrict__ Gr,
-                             double *__restrict__ D, double *__restrict__ A, double *__restrict__ B, Geom G, double w) {
-    int i, j, k;
-    if (!cell_of_flat(G, i, j, k)) return;
-    const long id = G.id(i, j, k);
-    double gx[7], gy[7], gz[7];
-    m3_line_load(T, id, 1, gx);
-    m3_line_load(T, id, G.sx, gy);
-    m3_line_load(T, id, G.sxy, gz);
-    const double sg = S[id];
-    double up, um, vp, vm, wp, wm;
-    m3_line_weno(gx, i, G.nx, 1.0 / G.dx, up, um);
-    m3_line_weno(gy, j, G.ny, 1.0 / G.dy, vp, vm);
-    m3_line_weno(gz, k, G.nz, 1.0 / G.dz, wp, wm);
-    double g;
-    if (sg >= 0.0)
-        g = sqrt(sq(fmax(-fmin(up, 0.0), fmax(um, 0.0))) + sq(fmax(-fmin(vp, 0.0), fmax(vm, 0.0))) +
-                 sq(fmax(-fmin(wp, 0.0), fmax(wm, 0.0))));
-    else
-        g = sqrt(sq(fmax(fmax(up, 0.0), -fmin(um, 0.0))) + sq(fmax(fmax(vp, 0.0), -fmin(vm, 0.0))) +
-                 sq(fmax(fmax(wp, 0.0), -fmin(wm, 0.0))));
-    double hp;
-    m3_heav(gx[3], w, hp);
-    Gr[id] = g;
-    D[id] = hp;
-    A[id] = (sg * hp) * (g - 1.0);
-    B[id] = g * sq(hp);
+// the interface band, |T| <= INTERFACE_WIDTH: where m3_heav's delta can be
+// non-zero (NaN counts as inside)
+__device__ __forceinline__ bool m3_in_band(double x, double w) { return !(x > w) && !(x < -w); }
+
+// one RK stage of LS_REDIS (LS_REDISTANCE.F90:68-146)
+template <int STAGE>
+__device__ __forceinline__ double m3_redis_update(double T, double s, double s0, double s1, double rdt) {
+    if (STAGE == 0) return T - rdt * s;
+    if (STAGE == 1) return T - rdt / 4.0 * (-3.0 * s0 + s);
+    return T - rdt / 12.0 * (-s0 - s1 + 8.0 * s);
 }
 
-// RIS_MASS's 27-point constraint (a, b zero-gradient beyond the walls, as
-// bc3d leaves them) and one RK stage of LS_REDIS (LS_REDISTANCE.F90:68-146)
-// on T in place: s = (SGN - C) |grad| - SGN, C = delta (51 a + sum a) /
-// (51 b + sum b).  C enters only where delta != 0, the interface band of
-// |T| <= INTERFACE_WIDTH (well under 1 % of the cells of a bubble problem);
-// elsewhere C = 0 and the cell needs none of the 54 values of a and b, so a
-// thread per cell reads them only in the band (3 x 3 plane sums of planes
-// k-1, k, k+1 in the order of the reference's loop nest).
+// One stage of LS_REDIS from T into out (another array): GRADFI, |grad T| by
+// Godunov on the WENO values (LS_REDISTANCE.F90:148-238), then s = (SGN - C)
+// |grad| - SGN and the update.  C, RIS_MASS's constraint, enters only in the
+// interface band (well under 1 % of the cells of a bubble problem), so every
+// other cell is finished here; a band cell stores |grad|, a = SGN delta
+// (|grad| - 1) and b = |grad| delta^2, and its block is listed for
+// k_m3_redis_band.  `last`: the call's last stage also leaves GRAD and DELTA.
 constexpr int M3_BT = 256;
-__global__ void __launch_bounds__(M3_BT) k_m3_redis_b(double *__restrict__ T, const double *__restrict__ S,
-                                                     const double *__restrict__ Gr, const double *__restrict__ D,
-                                                     const double *__restrict__ A, const double *__restrict__ B,
-                                                     double *__restrict__ s0, double *__restrict__ s1, Geom G,
-                                                     double rdt, int stage) {
+template <int STAGE>
+__global__ void __launch_bounds__(M3_BT) __attribute__((amdgpu_waves_per_eu(1, 4)))
+k_m3_redis_stage(const double *__restrict__ T, double *__restrict__ out, const double *__restrict__ S,
+                 double *__restrict__ Gr, double *__restrict__ D, double *__restrict__ A, double *__restrict__ B,
+                 double *__restrict__ s0, double *__restrict__ s1, BandList band, Geom G, double w, double rdt, int lo,
+                 int last) {
+    band.clear((STAGE + 1) % 3);   // the next stage's list
+    int bx, by, bz, hold = 0;
+    xcd_block(bx, by, bz);
     int i, j, k;
-    if (!cell_of_flat(G, i, j, k)) return;
-    const long id = G.id(i, j, k);
-    const double d = D[id], sg = S[id], g = Gr[id];
-    double c = 0.0;
-    if (d != 0.0) {
-        const int im = clampi(i - 1, 0, G.nx - 1), ip = clampi(i + 1, 0, G.nx - 1);
-        const int jm = clampi(j - 1, 0, G.ny - 1), jp = clampi(j + 1, 0, G.ny - 1);
-        // 3 x 3 sums of a and b over plane kk (clamped), rows j-1, j, j+1
-        auto plane = [&](int kk, double &pa, double &pb) {
-            const int kc = clampi(kk, 0, G.nz - 1);
-            pa = 0.0;
-            pb = 0.0;
-            const int js[3] = {jm, j, jp};
-#pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                const long row = G.id(0, js[r], kc);
-                pa += A[row + im];
-                pa += A[row + i];
-                pa += A[row + ip];
-                pb += B[row + im];
-                pb += B[row + i];
-                pb += B[row + ip];
-            }
-        };
-        double am, bm, ac, bc, ap, bp;
-        plane(k - 1, am, bm);
-        plane(k, ac, bc);
-        plane(k + 1, ap, bp);
-        const double suma = 51.0 * A[id] + (am + ac + ap), sumb = 51.0 * B[id] + (bm + bc + bp);
-        c = (sumb != 0.0 ? suma / sumb : 0.0) * d;
+    if (cell_of_flat(G, i, j, k)) {
+        const long id = G.id(i, j, k);
+        double gx[7], gy[7], gz[7];
+        m3_line_load(T, id, 1, i, G.nx, lo, gx);
+        m3_line_load(T, id, G.sx, j, G.ny, lo, gy);
+        m3_line_load(T, id, G.sxy, k, G.nz, lo, gz);
+        const double sg = S[id], s0o = STAGE >= 1 ? s0[id] : 0.0, s1o = STAGE == 2 ? s1[id] : 0.0;
+        const double T0 = gx[3];
+        double up, um, vp, vm, wp, wm;
+        m3_line_weno(gx, i, G.nx, 1.0 / G.dx, up, um);
+        m3_line_weno(gy, j, G.ny, 1.0 / G.dy, vp, vm);
+        m3_line_weno(gz, k, G.nz, 1.0 / G.dz, wp, wm);
+        double g;
+        if (sg >= 0.0)
+            g = sqrt(sq(fmax(-fmin(up, 0.0), fmax(um, 0.0))) + sq(fmax(-fmin(vp, 0.0), fmax(vm, 0.0))) +
+                     sq(fmax(-fmin(wp, 0.0), fmax(wm, 0.0))));
+        else
+            g = sqrt(sq(fmax(fmax(up, 0.0), -fmin(um, 0.0))) + sq(fmax(fmax(vp, 0.0), -fmin(vm, 0.0))) +
+                     sq(fmax(fmax(wp, 0.0), -fmin(wm, 0.0))));
+        double hp = 0.0;
+        if (m3_in_band(T0, w)) {
+            m3_heav(T0, w, hp);
+            Gr[id] = g;
+            A[id] = (sg * hp) * (g - 1.0);
+            B[id] = g * sq(hp);
+            hold = 1;
+        } else {
+            const double s = sg * g - sg;
+            if (STAGE == 0) s0[id] = s;
+            if (STAGE == 1) s1[id] = s;
+            out[id] = m3_redis_update<STAGE>(T0, s, s0o, s1o, rdt);
+        }
+        if (last) {
+            Gr[id] = g;
+            D[id] = hp;
+        }
     }
-    const double s = (sg - c) * g - sg;
-    if (stage == 0) {
-        s0[id] = s;
-        T[id] = T[id] - rdt * s;
-    } else if (stage == 1) {
-        s1[id] = s;
-        T[id] = T[id] - rdt / 4.0 * (-3.0 * s0[id] + s);
-    } else {
-        T[id] = T[id] - rdt / 12.0 * (-s0[id] - s1[id] + 8.0 * s);
+    band.append(STAGE, hold, (unsigned)bx);
+}
+
+// The band cells of a stage: RIS_MASS's 27-point constraint (a, b
+// zero-gradient beyond the walls, as bc3d leaves them; 0 outside the band),
+// C = delta (51 a + sum a) / (51 b + sum b), in 3 x 3 plane sums of planes
+// k-1, k, k+1 in the order of the reference's loop nest, and the update.
+template <int STAGE>
+__global__ void __launch_bounds__(M3_BT) k_m3_redis_band(const double *__restrict__ T, double *__restrict__ out,
+                                                        const double *__restrict__ S, const double *__restrict__ Gr,
+                                                        const double *__restrict__ A, const double *__restrict__ B,
+                                                        double *__restrict__ s0, double *__restrict__ s1,
+                                                        BandList band, Geom G, double w, double rdt) {
+    __shared__ BandCells sh;
+    const unsigned total = band.total(STAGE), nxy = (unsigned)G.nx * (unsigned)G.ny, n = nxy * (unsigned)G.nz;
+    auto cell_of = [&](unsigned tile, int th, int &i, int &j, int &k) {
+        const unsigned t = tile * M3_BT + th, kk = t / nxy, r = t - kk * nxy, jj = r / (unsigned)G.nx;
+        i = (int)(r - jj * (unsigned)G.nx);
+        j = (int)jj;
+        k = (int)kk;
+        return t < n;
+    };
+    for (unsigned first = blockIdx.x * BAND_TILES; first < total; first += gridDim.x * BAND_TILES) {
+        band_collect(sh, band, STAGE, first, total, T, G, cell_of, [&](double p) { return m3_in_band(p, w); });
+        for (int c = threadIdx.x; c < sh.n; c += M3_BT) {
+            int i, j, k;
+            cell_of(sh.tile[sh.cell[c] / 256], sh.cell[c] % 256, i, j, k);
+            const long id = G.id(i, j, k);
+            const int is[3] = {max(i - 1, 0), i, min(i + 1, G.nx - 1)};
+            const int js[3] = {max(j - 1, 0), j, min(j + 1, G.ny - 1)};
+            const double T0 = T[id], sg = S[id], g = Gr[id], s0o = STAGE >= 1 ? s0[id] : 0.0,
+                         s1o = STAGE == 2 ? s1[id] : 0.0;
+            double d;
+            m3_heav(T0, w, d);
+            double suma = 0.0, sumb = 0.0;
+#pragma unroll
+            for (int kk = 0; kk < 3; ++kk) {
+                const int kc = clampi(k + kk - 1, 0, G.nz - 1);
+                double ph[9], ta[9], tb[9];
+#pragma unroll
+                for (int m = 0; m < 9; ++m) {
+                    const long o = G.id(is[m % 3], js[m / 3], kc);
+                    ph[m] = T[o];
+                    ta[m] = A[o];
+                    tb[m] = B[o];
+                }
+                double pa = 0.0, pb = 0.0;
+#pragma unroll
+                for (int m = 0; m < 9; ++m) {
+                    const bool held = m3_in_band(ph[m], w);
+                    pa += held ? ta[m] : 0.0;
+                    pb += held ? tb[m] : 0.0;
+                }
+                suma += pa;
+                sumb += pb;
+            }
+            suma = 51.0 * A[id] + suma;
+            sumb = 51.0 * B[id] + sumb;
+            const double C = (sumb != 0.0 ? suma / sumb : 0.0) * d;
+            const double s = (sg - (d != 0.0 ? C : 0.0)) * g - sg;
+            if (STAGE == 0) s0[id] = s;
+            if (STAGE == 1) s1[id] = s;
+            out[id] = m3_redis_update<STAGE>(T0, s, s0o, s1o, rdt);
+        }
+        __syncthreads();
     }
 }
 
@@ -552,31 +601,43 @@ static int m3_redis_steps(const fcfd_ctx *c) {
     return n;
 }
 
-// LS_REDISTANCE(T, 1) on T (a ghosted field whose ghosts hold bc3d copies)
+template <int STAGE>
+static int m3_redis_stage(fcfd_ctx *c, const double *in, double *out, int lo, int last) {
+    const Geom &G = c->G;
+    double **F = c->f;
+    const dim3 ga = grid_flat(G, M3_BT);
+    const BandList band = band_lists(c, ga.x);
+    {
+        ProfScope ps_(c, R_REDIS_A);
+        hipLaunchKernelGGL(k_m3_redis_stage<STAGE>, ga, dim3(M3_BT), 0, c->stream, in, out, F[FCFD_SIGN], F[FCFD_GRAD],
+                           F[FCFD_DELTA], c->s2, c->s3, c->l1, c->l2, band, G, c->pr.ls_wid, c->pr.rdt, lo, last);
+        FCFD_CHECK(hipGetLastError());
+    }
+    {
+        ProfScope ps_(c, R_REDIS_B);
+        hipLaunchKernelGGL(k_m3_redis_band<STAGE>, band_grid(c, ga.x), dim3(M3_BT), 0, c->stream, in, out,
+                           F[FCFD_SIGN], F[FCFD_GRAD], c->s2, c->s3, c->l1, c->l2, band, G, c->pr.ls_wid, c->pr.rdt);
+        FCFD_CHECK(hipGetLastError());
+    }
+    return FCFD_OK;
+}
+
+// LS_REDISTANCE(T, 1) on T (a ghosted field whose ghosts hold bc3d copies):
+// the stages go T -> phiB -> phiS -> T
 static int m3_redistance(fcfd_ctx *c, double *T) {
     const Geom &G = c->G;
     double **F = c->f;
     if (!flat_fits(G)) return FCFD_ERR_ARG;
-    hipLaunchKernelGGL(k_m3_sign, grid_flat(G, M3_BT), dim3(M3_BT), 0, c->stream, T, F[FCFD_SIGN], G, c->pr.ls_wid);
+    hipLaunchKernelGGL(k_m3_sign, grid_flat(G, M3_BT), dim3(M3_BT), 0, c->stream, T, F[FCFD_SIGN], G, c->pr.ls_wid,
+                       band_lists(c, 0));
     FCFD_CHECK(hipGetLastError());
-    const dim3 ga = grid_flat(G, M3_BT);
     const int n = m3_redis_steps(c);
-    for (int it = 0; it < n; ++it)
-        for (int s = 0; s < 3; ++s) {
-            {
-                ProfScope ps_(c, R_REDIS_A);
-                hipLaunchKernelGGL(k_m3_redis_a, ga, dim3(M3_BT), 0, c->stream, T, F[FCFD_SIGN], F[FCFD_GRAD],
-                                   F[FCFD_DELTA], c->s2, c->s3, G, c->pr.ls_wid);
-                FCFD_CHECK(hipGetLastError());
-            }
-            {
-                ProfScope ps_(c, R_REDIS_B);
-                hipLaunchKernelGGL(k_m3_redis_b, ga, dim3(M3_BT), 0, c->stream, T, F[FCFD_SIGN], F[FCFD_GRAD],
-                                   F[FCFD_DELTA], c->s2, c->s3, c->l1, c->l2, G, c->pr.rdt, s);
-                FCFD_CHECK(hipGetLastError());
-            }
-            FCFD_TRY(bc_scalar(c, T));
-        }
+    for (int it = 0; it < n; ++it) {
+        FCFD_TRY(m3_redis_stage<0>(c, T, c->phiB, it == 0 ? -1 : 0, 0));
+        FCFD_TRY(m3_redis_stage<1>(c, c->phiB, c->phiS, 0, 0));
+        FCFD_TRY(m3_redis_stage<2>(c, c->phiS, T, 0, it == n - 1));
+    }
+    if (n > 0) FCFD_TRY(bc_scalar(c, T));
     c->diag.redis_iters = n;
     return FCFD_OK;
 }
