@@ -114,7 +114,7 @@ __device__ __forceinline__ double sq(double x) { return x * x; }
 // weno_js (SCHEME_WENO.F90:47-101) at one point is the WENO5-JS pair of
 // weno.h with EPS = 1e-12: the left-biased value from f(i-2..i+2), the
 // right-biased one from f(i-1..i+3), the same smoothness indicators and
-// weights d = (1, 6, 3), normalised there with one division instead of six.
+// weights d = (1, 6, 3), with one reciprocal instead of six divisions.
 
 // the one-sided WENO values of the backward differences along a line:
 // F(m) = (T(m) - T(m-1)) / h for interior m, F of a ghost index = F of the
@@ -139,8 +139,8 @@ __device__ __forceinline__ void m3_line_weno(const double (&g)[7], int i, int n,
 #pragma unroll
     for (int q = 0; q < 6; ++q) f[q] = (g[q + 1] - g[q]) * ih;
     if (i < 2 || i > n - 4) clamp_window(f, 2 - i, n + 1 - i);
-    um = weno_left(f[0], f[1], f[2], f[3], f[4], kEps);
-    up = weno_right(f[1], f[2], f[3], f[4], f[5], kEps);
+    um = weno_left_sum(f[0], f[1], f[2], f[3], f[4], kEps);
+    up = weno_left_sum(f[5], f[4], f[3], f[2], f[1], kEps);   // the right-biased value: mirrored
 }
 
 // the interface band, |T| <= INTERFACE_WIDTH: where m3_heav's delta can be
