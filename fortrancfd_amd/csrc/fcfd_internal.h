@@ -63,6 +63,28 @@ __device__ __forceinline__ void clamp_window(double (&d)[W], int lo, int hi) {
     for (int m = 0; m < W; ++m) d[m] = m < lo ? vlo : (m > hi ? vhi : d[m]);
 }
 
+// The W values of a field's line around a cell, at pos - BELOW .. of the
+// line, indices clamped to [lo, n - 1].  base: the address of the block's
+// first cell (uniform over the block), off: the cell's distance from it.  A
+// wave whose cells all lie inside the line reads at uniform strides from
+// scalar bases (one vector offset for every load of the kernel, where
+// per-lane 64-bit addresses take 4-6 instructions a load); the others clamp
+// lane by lane.
+template <int W, int BELOW>
+__device__ __forceinline__ void line_load(const double *__restrict__ base, unsigned off, long st, int pos, int n,
+                                          int lo, double (&g)[W]) {
+    if (__all(pos - BELOW >= lo && pos + W - 1 - BELOW < n)) {
+#pragma unroll
+        for (int r = 0; r < W; ++r) g[r] = (base + (r - BELOW) * st)[off];
+    } else {
+#pragma unroll
+        for (int r = 0; r < W; ++r) {
+            const int q = r < BELOW ? max(pos + r - BELOW, lo) : min(pos + r - BELOW, n - 1);
+            g[r] = base[(long)off + (long)(q - pos) * st];
+        }
+    }
+}
+
 // One level of the pressure multigrid hierarchy (see mg.hip).
 struct MgLevel {
     int nx, ny, nz;          // cells
@@ -396,6 +418,22 @@ __device__ __forceinline__ void cell_of_index(long t, const Geom &G, int &i, int
         j = (int)(r % G.ny);
         k = (int)(r / G.ny);
     }
+}
+
+// cell_of_flat with the index of the block's first cell (id0, uniform) and
+// the cell's distance from it (cells of a block follow each other in memory)
+__device__ __forceinline__ bool cell_of_flat(const Geom &G, int &i, int &j, int &k, long &id0, unsigned &off) {
+    int bx, by, bz;
+    xcd_block(bx, by, bz);
+    const unsigned nxy = (unsigned)G.nx * (unsigned)G.ny, t0 = (unsigned)bx * blockDim.x, t = t0 + threadIdx.x;
+    const unsigned k0 = t0 / nxy, r0 = t0 - k0 * nxy, j0 = r0 / (unsigned)G.nx;
+    id0 = G.id((int)(r0 - j0 * (unsigned)G.nx), (int)j0, (int)k0);
+    const unsigned kk = t / nxy, r = t - kk * nxy, jj = r / (unsigned)G.nx;
+    i = (int)(r - jj * (unsigned)G.nx);
+    j = (int)jj;
+    k = (int)kk;
+    off = (unsigned)(G.id(i, j, k) - id0);
+    return t < nxy * (unsigned)G.nz;
 }
 
 inline bool flat_fits(const Geom &G) { return (double)G.nx * G.ny * G.nz < 4294967296.0 - 1024.0; }

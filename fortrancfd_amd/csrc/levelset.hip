@@ -679,6 +679,9 @@ __device__ __forceinline__ void redis_shard_max(double err, double *sh4, unsigne
     }
 }
 
+struct Recip {
+    double x, y, z;   // reciprocal spacings
+};
 constexpr int REDIS_GRADIENT = 3;  // STAGE of the gradient-only pass
 
 // One reinitialisation stage from phi into out (another array: the stencil
@@ -702,7 +705,8 @@ __global__ void __launch_bounds__(256) k_redis_stage(const double *__restrict__ 
                                                      double *__restrict__ s2, double *__restrict__ s3,
                                                      double *__restrict__ l1, double *__restrict__ l2,
                                                      BandList band, unsigned long long *flags, Geom G,
-                                                     double w, double iw, double r12, double rdt, int lo) {
+                                                     double w, double iw, double r12, double rdt, Recip ih,
+                                                     int lo) {
     int bx_, by_, bz_;
     if (DIM == 3) xcd_block_slab(bx_, by_, bz_, 8);
     else xcd_block(bx_, by_, bz_);
@@ -713,24 +717,21 @@ __global__ void __launch_bounds__(256) k_redis_stage(const double *__restrict__ 
     double err = 0.0;
     int hold = 0;
     if (in) {
-        const long id = G.id(i, j, k);
+        const long id0 = G.id(bx_ * (int)blockDim.x, by_ * (int)blockDim.y, k);   // the block's first cell
+        const unsigned off = threadIdx.x + threadIdx.y * (unsigned)G.sx;
         const int n[3] = {G.nx, G.ny, G.nz};
         const int pos[3] = {i, j, k};
         const long st[3] = {1, G.sx, G.sxy};
-        const double ih[3] = {1.0 / G.dx, 1.0 / G.dy, 1.0 / G.dz};
+        const double ihd[3] = {ih.x, ih.y, ih.z};
         // phi at pos-4 .. pos+3 of the three lines and the cell's other
-        // operands, all loads before any branch
+        // operands before any branch that depends on them
         double gw[3][8];
 #pragma unroll
-        for (int d = 0; d < DIM; ++d)
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const int q = r < 4 ? max(pos[d] + r - 4, lo) : min(pos[d] + r - 4, n[d] - 1);
-                gw[d][r] = phi[id + (long)(q - pos[d]) * st[d]];
-            }
-        const double S = S0[id];
-        const double l1o = STAGE == 1 || STAGE == 2 ? l1[id] : 0.0, l2o = STAGE == 2 ? l2[id] : 0.0;
-        const double pst = STAGE == 2 ? out[id] : 0.0;   // the last stage writes over phi_start
+        for (int d = 0; d < DIM; ++d) line_load<8, 4>(phi + id0, off, st[d], pos[d], n[d], lo, gw[d]);
+        grad += id0; s2 += id0; s3 += id0; l1 += id0; l2 += id0; out += id0;
+        const double S = (S0 + id0)[off];
+        const double l1o = STAGE == 1 || STAGE == 2 ? l1[off] : 0.0, l2o = STAGE == 2 ? l2[off] : 0.0;
+        const double pst = STAGE == 2 ? out[off] : 0.0;   // the last stage writes over phi_start
         const double p0 = gw[0][4];
         const bool pos_sign = S >= 0.0;
         double sel[3];
@@ -741,7 +742,7 @@ __global__ void __launch_bounds__(256) k_redis_stage(const double *__restrict__ 
             // with dw[m] = D(pos - 3 + m) the window's neighbour differences
             double nr[7];
 #pragma unroll
-            for (int m = 0; m < 7; ++m) nr[m] = (gw[d][m + 1] - gw[d][m]) * ih[d];
+            for (int m = 0; m < 7; ++m) nr[m] = (gw[d][m + 1] - gw[d][m]) * ihd[d];
             if (pos[d] < 3 || pos[d] > n[d] - 4) clamp_window(nr, 3 - pos[d], n[d] + 2 - pos[d]);
             const double EPS = 1.0e-10;
             double fm = weno_left(nr[1], nr[2], nr[3], nr[4], nr[5], EPS);   // tdata%s2
@@ -751,22 +752,22 @@ __global__ void __launch_bounds__(256) k_redis_stage(const double *__restrict__ 
         }
         const double g = DIM == 3 ? sqrt(sel[0] * sel[0] + sel[1] * sel[1] + sel[2] * sel[2])
                                   : sqrt(sel[0] * sel[0] + sel[1] * sel[1]);
-        if (STAGE >= 2) grad[id] = g;   // grad%now holds the last stage's
+        if (STAGE >= 2) grad[off] = g;   // grad%now holds the last stage's
         if (STAGE != REDIS_GRADIENT) {
             if (BTN && in_band(p0, iw)) {
                 double hh, dd;
                 lsfun(p0, w, hh, dd);
                 const double lam = DIM == 3 ? (2.0 * (1.0 - r12) * hh + r12) * dd : dd;
-                grad[id] = g;
-                s2[id] = lam * S * (g - 1.0);
-                s3[id] = g * dd * lam;
+                grad[off] = g;
+                s2[off] = lam * S * (g - 1.0);
+                s3[off] = g * dd * lam;
                 hold = 1;
             } else {
                 const double l = S * g - S;
                 const double pn = redis_update<STAGE>(p0, l, l1o, l2o, rdt);
-                if (STAGE == 0) l1[id] = l;
-                if (STAGE == 1) l2[id] = l;
-                out[id] = pn;
+                if (STAGE == 0) l1[off] = l;
+                if (STAGE == 1) l2[off] = l;
+                out[off] = pn;
                 if (STAGE == 2) err = fabs(pst - pn);
             }
         }
@@ -946,14 +947,15 @@ static int redis_stage(fcfd_ctx *c, dim3 grd, dim3 blk, int btn, const double *i
     double *grad = c->f[FCFD_GRAD];
     const long nt = (long)grd.x * grd.y * grd.z;
     const BandList band = band_lists(c, nt);
+    const Recip ih{1.0 / G.dx, 1.0 / G.dy, 1.0 / G.dz};
     {
         ProfScope ps_(c, R_REDIS_A);
         if (btn)
             hipLaunchKernelGGL((k_redis_stage<DIM, STAGE, true>), grd, blk, 0, c->stream, in, out, c->s0, grad, c->s2,
-                               c->s3, c->l1, c->l2, band, c->flag, G, w, iw, r12, rdt, lo);
+                               c->s3, c->l1, c->l2, band, c->flag, G, w, iw, r12, rdt, ih, lo);
         else
             hipLaunchKernelGGL((k_redis_stage<DIM, STAGE, false>), grd, blk, 0, c->stream, in, out, c->s0, grad,
-                               c->s2, c->s3, c->l1, c->l2, band, c->flag, G, w, iw, r12, rdt, lo);
+                               c->s2, c->s3, c->l1, c->l2, band, c->flag, G, w, iw, r12, rdt, ih, lo);
     }
     FCFD_CHECK(hipGetLastError());
     if constexpr (STAGE != REDIS_GRADIENT) {

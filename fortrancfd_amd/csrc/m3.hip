@@ -120,20 +120,10 @@ __device__ __forceinline__ double sq(double x) { return x * x; }
 // F(m) = (T(m) - T(m-1)) / h for interior m, F of a ghost index = F of the
 // nearest interior index (FV_DERI's bc3d); n the line's interior length.
 // The seven values T(i-3 .. i+3) are read at indices clamped to [lo, n-1]
-// (lo as in k_redis_stage: -1 where T's ghosts are valid, else 0), and every
-// clamped difference is one of their six neighbour differences:
-// F(clamp(i-2+q)) = d[clamp(q, 2-i, n+1-i)].  So the loads take no branch,
-// the caller issues the three lines of a cell together (m3_line_load), and
-// only the cells within two of a wall remap their differences.
-__device__ __forceinline__ void m3_line_load(const double *__restrict__ T, long id, long st, int i, int n, int lo,
-                                             double (&g)[7]) {
-#pragma unroll
-    for (int r = 0; r < 7; ++r) {
-        const int q = r < 3 ? max(i + r - 3, lo) : min(i + r - 3, n - 1);
-        g[r] = T[id + (long)(q - i) * st];
-    }
-}
-
+// (line_load; lo as in k_redis_stage: -1 where T's ghosts are valid, else 0),
+// and every clamped difference is one of their six neighbour differences:
+// F(clamp(i-2+q)) = d[clamp(q, 2-i, n+1-i)]; only the cells within two of a
+// wall remap their differences.
 __device__ __forceinline__ void m3_line_weno(const double (&g)[7], int i, int n, double ih, double &up, double &um) {
     double f[6];
 #pragma unroll
@@ -167,24 +157,26 @@ template <int STAGE>
 __global__ void __launch_bounds__(M3_BT) __attribute__((amdgpu_waves_per_eu(1, 4)))
 k_m3_redis_stage(const double *__restrict__ T, double *__restrict__ out, const double *__restrict__ S,
                  double *__restrict__ Gr, double *__restrict__ D, double *__restrict__ A, double *__restrict__ B,
-                 double *__restrict__ s0, double *__restrict__ s1, BandList band, Geom G, double w, double rdt, int lo,
-                 int last) {
+                 double *__restrict__ s0, double *__restrict__ s1, BandList band, Geom G, double w, double rdt,
+                 double ihx, double ihy, double ihz, int lo, int last) {
     band.clear((STAGE + 1) % 3);   // the next stage's list
     int bx, by, bz, hold = 0;
     xcd_block(bx, by, bz);
     int i, j, k;
-    if (cell_of_flat(G, i, j, k)) {
-        const long id = G.id(i, j, k);
+    long id0;
+    unsigned off;
+    if (cell_of_flat(G, i, j, k, id0, off)) {
         double gx[7], gy[7], gz[7];
-        m3_line_load(T, id, 1, i, G.nx, lo, gx);
-        m3_line_load(T, id, G.sx, j, G.ny, lo, gy);
-        m3_line_load(T, id, G.sxy, k, G.nz, lo, gz);
-        const double sg = S[id], s0o = STAGE >= 1 ? s0[id] : 0.0, s1o = STAGE == 2 ? s1[id] : 0.0;
+        line_load<7, 3>(T + id0, off, 1, i, G.nx, lo, gx);
+        line_load<7, 3>(T + id0, off, G.sx, j, G.ny, lo, gy);
+        line_load<7, 3>(T + id0, off, G.sxy, k, G.nz, lo, gz);
+        out += id0; Gr += id0; D += id0; A += id0; B += id0; s0 += id0; s1 += id0;
+        const double sg = (S + id0)[off], s0o = STAGE >= 1 ? s0[off] : 0.0, s1o = STAGE == 2 ? s1[off] : 0.0;
         const double T0 = gx[3];
         double up, um, vp, vm, wp, wm;
-        m3_line_weno(gx, i, G.nx, 1.0 / G.dx, up, um);
-        m3_line_weno(gy, j, G.ny, 1.0 / G.dy, vp, vm);
-        m3_line_weno(gz, k, G.nz, 1.0 / G.dz, wp, wm);
+        m3_line_weno(gx, i, G.nx, ihx, up, um);
+        m3_line_weno(gy, j, G.ny, ihy, vp, vm);
+        m3_line_weno(gz, k, G.nz, ihz, wp, wm);
         double g;
         if (sg >= 0.0)
             g = sqrt(sq(fmax(-fmin(up, 0.0), fmax(um, 0.0))) + sq(fmax(-fmin(vp, 0.0), fmax(vm, 0.0))) +
@@ -195,19 +187,19 @@ k_m3_redis_stage(const double *__restrict__ T, double *__restrict__ out, const d
         double hp = 0.0;
         if (m3_in_band(T0, w)) {
             m3_heav(T0, w, hp);
-            Gr[id] = g;
-            A[id] = (sg * hp) * (g - 1.0);
-            B[id] = g * sq(hp);
+            Gr[off] = g;
+            A[off] = (sg * hp) * (g - 1.0);
+            B[off] = g * sq(hp);
             hold = 1;
         } else {
             const double s = sg * g - sg;
-            if (STAGE == 0) s0[id] = s;
-            if (STAGE == 1) s1[id] = s;
-            out[id] = m3_redis_update<STAGE>(T0, s, s0o, s1o, rdt);
+            if (STAGE == 0) s0[off] = s;
+            if (STAGE == 1) s1[off] = s;
+            out[off] = m3_redis_update<STAGE>(T0, s, s0o, s1o, rdt);
         }
         if (last) {
-            Gr[id] = g;
-            D[id] = hp;
+            Gr[off] = g;
+            D[off] = hp;
         }
     }
     band.append(STAGE, hold, (unsigned)bx);
@@ -610,7 +602,8 @@ static int m3_redis_stage(fcfd_ctx *c, const double *in, double *out, int lo, in
     {
         ProfScope ps_(c, R_REDIS_A);
         hipLaunchKernelGGL(k_m3_redis_stage<STAGE>, ga, dim3(M3_BT), 0, c->stream, in, out, F[FCFD_SIGN], F[FCFD_GRAD],
-                           F[FCFD_DELTA], c->s2, c->s3, c->l1, c->l2, band, G, c->pr.ls_wid, c->pr.rdt, lo, last);
+                           F[FCFD_DELTA], c->s2, c->s3, c->l1, c->l2, band, G, c->pr.ls_wid, c->pr.rdt, 1.0 / G.dx,
+                           1.0 / G.dy, 1.0 / G.dz, lo, last);
         FCFD_CHECK(hipGetLastError());
     }
     {
