@@ -77,10 +77,23 @@ __device__ __forceinline__ bool local_cell(const BlkDesc &D, int bx, int by, int
     const int lz = D.start[2][bz + 1] - D.start[2][bz];
     const long ex = lx + 2 * D.g, ey = ly + 2 * D.g, ez = lz + 2 * D.gz;
     if (t >= ex * ey * ez) return false;
-    i = (int)(t % ex) - D.g;
-    j = (int)((t / ex) % ey) - D.g;
-    k = (int)(t / (ex * ey)) - D.gz;
+    if (ex * ey * ez < 4294967296L) {   // 32-bit divisions (a 64-bit one is several times longer)
+        const unsigned tt = (unsigned)t, xx = (unsigned)ex, yy = (unsigned)ey, r = tt / xx, kk = r / yy;
+        i = (int)(tt - r * xx) - D.g;
+        j = (int)(r - kk * yy) - D.g;
+        k = (int)kk - D.gz;
+    } else {
+        i = (int)(t % ex) - D.g;
+        j = (int)((t / ex) % ey) - D.g;
+        k = (int)(t / (ex * ey)) - D.gz;
+    }
     return true;
+}
+
+// local (i, j, k) is one of block b's own cells
+__device__ __forceinline__ bool own_cell(const BlkDesc &D, int bx, int by, int bz, int i, int j, int k) {
+    return i >= 0 && i < D.start[0][bx + 1] - D.start[0][bx] && j >= 0 && j < D.start[1][by + 1] - D.start[1][by] &&
+           k >= 0 && k < D.start[2][bz + 1] - D.start[2][bz];
 }
 
 __device__ __forceinline__ long local_id(const BlkDesc &D, int bx, int by, int i, int j, int k) {
@@ -101,13 +114,13 @@ __global__ void __launch_bounds__(256) k_blocks_sync(double *__restrict__ stack,
     int bx, by, bz, i, j, k;
     block_coords(D, bx, by, bz);
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (!local_cell(D, bx, by, bz, t, i, j, k)) return;
+    if (!local_cell(D, bx, by, bz, t, i, j, k) || own_cell(D, bx, by, bz, i, j, k)) return;
     const int X = D.start[0][bx] + i, Y = D.start[1][by] + j, Z = D.start[2][bz] + k;
     int ox, oy, oz, li, lj, lk;
     owner(D, 0, X, ox, li);
     owner(D, 1, Y, oy, lj);
     owner(D, 2, Z, oz, lk);
-    if (ox == bx && oy == by && oz == bz && li == i && lj == j && lk == k) return;   // interior or own physical ghost
+    if (ox == bx && oy == by && oz == bz && li == i && lj == j && lk == k) return;   // own physical ghost
     stack[blk_off(D, bx, by, bz) + t] = stack[blk_off(D, ox, oy, oz) + local_id(D, ox, oy, li, lj, lk)];
 }
 
@@ -210,6 +223,9 @@ struct fcfd_blocks {
     double *a = nullptr, *b = nullptr, *l1 = nullptr, *l2 = nullptr;   // advection scratch stacks
     double *part = nullptr;
     std::vector<double> part_host;
+    int ncu = 0;                   // compute units of the device
+    int len[3] = {0, 0, 0};        // largest block's cells per axis
+    BlockGeom *tab = nullptr;      // device: geometry and offset of every block, x fastest
 };
 
 namespace {
@@ -236,6 +252,22 @@ Geom block_geom(const fcfd_blocks *B, int bx, int by, int bz) {
 }
 
 int stack_scratch(fcfd_blocks *B) {
+    if (!B->tab) {
+        const BlkDesc &D = B->D;
+        std::vector<BlockGeom> h;
+        for (int bz = 0; bz < D.nb[2]; ++bz)
+            for (int by = 0; by < D.nb[1]; ++by)
+                for (int bx = 0; bx < D.nb[0]; ++bx) {
+                    const BlockGeom g{block_geom(B, bx, by, bz), blk_off(D, bx, by, bz)};
+                    B->len[0] = std::max(B->len[0], g.G.nx);
+                    B->len[1] = std::max(B->len[1], g.G.ny);
+                    B->len[2] = std::max(B->len[2], g.G.nz);
+                    h.push_back(g);
+                }
+        FCFD_CHECK(hipDeviceGetAttribute(&B->ncu, hipDeviceAttributeMultiprocessorCount, B->device));
+        FCFD_CHECK(hipMalloc((void **)&B->tab, sizeof(BlockGeom) * h.size()));
+        FCFD_CHECK(hipMemcpy(B->tab, h.data(), sizeof(BlockGeom) * h.size(), hipMemcpyHostToDevice));
+    }
     if (B->a) return FCFD_OK;
     for (double **p : {&B->a, &B->b, &B->l1, &B->l2})
         FCFD_CHECK(hipMalloc((void **)p, sizeof(double) * B->total));
@@ -310,6 +342,7 @@ extern "C" int fcfd_blocks_destroy(fcfd_blocks *B) {
     if (!B) return FCFD_ERR_ARG;
     for (double *p : {B->a, B->b, B->l1, B->l2, B->part})
         if (p) hipFree(p);
+    if (B->tab) hipFree(B->tab);
     delete B;
     return FCFD_OK;
 }
@@ -381,20 +414,15 @@ extern "C" int fcfd_blocks_level_set_rk3_solver(fcfd_blocks *B, double *phi, con
     if (!B || !phi || !nu || !nv || (B->G.dim == 3 && !nw)) return FCFD_ERR_ARG;
     FCFD_TRY(stack_scratch(B));
     hipStream_t st = (hipStream_t)stream;
-    const BlkDesc &D = B->D;
-    // stage inputs and outputs: phi -> a -> b -> phi
+    // stage inputs and outputs: phi -> a -> b -> phi.  A stage reads its
+    // block's cells and, through shared faces, the ghosts that the exchange
+    // fills; physical ghosts (job_bc) are written on the result only.
     const double *in[3] = {phi, B->a, B->b};
     double *out[3] = {B->a, B->b, phi};
     for (int s = 0; s < 3; ++s) {
-        for (int bz = 0; bz < D.nb[2]; ++bz)
-            for (int by = 0; by < D.nb[1]; ++by)
-                for (int bx = 0; bx < D.nb[0]; ++bx) {
-                    const Geom g = block_geom(B, bx, by, bz);
-                    const long o = blk_off(D, bx, by, bz);
-                    FCFD_TRY(ls_adv_stage_geom(st, g, in[s] + o, out[s] + o, nu + o, nv + o, nw ? nw + o : nullptr,
-                                               B->l1 + o, B->l2 + o, B->dt, s));
-                }
-        FCFD_TRY(fcfd_blocks_bc(B, out[s], stream));
+        FCFD_TRY(ls_adv_stage_blocks(st, B->ncu, B->tab, B->nblk, B->G.dim, B->len[0], B->len[1], B->len[2], in[s],
+                                     out[s], nu, nv, nw, B->l1, B->l2, B->dt, s));
+        if (s == 2) FCFD_TRY(fcfd_blocks_bc(B, out[s], stream));
         FCFD_TRY(fcfd_blocks_sync(B, out[s], stream));
     }
     return FCFD_OK;

@@ -305,15 +305,6 @@ static int create_impl(const fcfd_grid *grid, const fcfd_params *params, int nca
         if (rc != FCFD_OK) break;
         rc = alloc_field(p, n);
     }
-    // the reinitialisation's lists of band tiles (256 cells each): 3 x NXCD
-    // counters and room for every block of a launch (a tiled launch has at
-    // least as many blocks as a flat one)
-    {
-        const dim3 blk = tile_rows(G.nx), grd = grid_interior(G, blk);
-        const long nt = (long)grd.x * grd.y * grd.z, words = 3 * NXCD + (nt + NXCD - 1) / NXCD * NXCD;
-        if (rc == FCFD_OK && hipMalloc((void **)&c->band, words * sizeof(unsigned)) != hipSuccess) rc = FCFD_ERR_HIP;
-        if (rc == FCFD_OK && hipMemset(c->band, 0, words * sizeof(unsigned)) != hipSuccess) rc = FCFD_ERR_HIP;
-    }
     // reduction partials: 8 slots x 1024 blocks per case, or two slots per
     // block of an interior launch with 64x4 blocks, whichever is larger
     const long nbc = c->nb;
@@ -323,8 +314,19 @@ static int create_impl(const fcfd_grid *grid, const fcfd_params *params, int nca
         c->red.nblocks = (int)((need + 7) / 8);
     }
     // + 4 slots x 256 second-stage partials per case of the level-0 reductions
-    if (rc == FCFD_OK) rc = alloc_field(&c->red.partial, 8L * c->red.nblocks + 4 * 256 * nbc);
-    if (rc == FCFD_OK) c->red.partial2 = c->red.partial + 8L * c->red.nblocks;
+    // + the reinitialisation's lists of band tiles (256 cells each): 3 x NXCD
+    // counters and room for every block of a launch (a tiled launch has at
+    // least as many blocks as a flat one)
+    {
+        const dim3 blk = tile_rows(G.nx), grd = grid_interior(G, blk);
+        const long nt = (long)grd.x * grd.y * grd.z, words = 3 * NXCD + (nt + NXCD - 1) / NXCD * NXCD;
+        const long np = 8L * c->red.nblocks + 4 * 256 * nbc;
+        if (rc == FCFD_OK) rc = alloc_field(&c->red.partial, np + (words + 1) / 2);
+        if (rc == FCFD_OK) {
+            c->red.partial2 = c->red.partial + 8L * c->red.nblocks;
+            c->band = (unsigned *)(c->red.partial + np);
+        }
+    }
     if (rc == FCFD_OK) rc = alloc_field(&c->red.result, RES_STRIDE * nbc);
     if (rc == FCFD_OK && hipHostMalloc((void **)&c->red.host, 64 * nbc * sizeof(double)) != hipSuccess)
         rc = FCFD_ERR_HIP;
@@ -411,7 +413,6 @@ extern "C" int fcfd_destroy(fcfd_ctx *c) {
     if (c->diag_host) hipHostFree(c->diag_host);
     if (c->cases_dev) hipFree(c->cases_dev);
     if (c->pack) hipFree(c->pack);
-    if (c->band) hipFree(c->band);
     if (c->flag) hipFree(c->flag);
     if (c->flag_host) hipHostFree(c->flag_host);
     for (hipEvent_t e : c->redis_ev)

@@ -63,6 +63,18 @@ __device__ __forceinline__ void clamp_window(double (&d)[W], int lo, int hi) {
     for (int m = 0; m < W; ++m) d[m] = m < lo ? vlo : (m > hi ? vhi : d[m]);
 }
 
+// element at a byte offset from a base that is uniform over the wave: the
+// load takes the base from scalar registers and 32 offset bits per lane (an
+// index would be scaled in 64-bit vector arithmetic for every load)
+template <typename T>
+__device__ __forceinline__ T &at_bytes(T *base, unsigned bytes) {
+    return *(T *)((char *)base + bytes);
+}
+template <typename T>
+__device__ __forceinline__ const T &at_bytes(const T *base, unsigned bytes) {
+    return *(const T *)((const char *)base + bytes);
+}
+
 // The W values of a field's line around a cell, at pos - BELOW .. of the
 // line, indices clamped to [lo, n - 1].  base: the address of the block's
 // first cell (uniform over the block), off: the cell's distance from it.  A
@@ -75,7 +87,7 @@ __device__ __forceinline__ void line_load(const double *__restrict__ base, unsig
                                           int lo, double (&g)[W]) {
     if (__all(pos - BELOW >= lo && pos + W - 1 - BELOW < n)) {
 #pragma unroll
-        for (int r = 0; r < W; ++r) g[r] = (base + (r - BELOW) * st)[off];
+        for (int r = 0; r < W; ++r) g[r] = at_bytes(base + (r - BELOW) * st, off * (unsigned)sizeof(double));
     } else {
 #pragma unroll
         for (int r = 0; r < W; ++r) {
@@ -473,12 +485,20 @@ int ccd_lines_set(fcfd_ctx *c, int set, int dir, const double *f, double *fx, do
 int m3_fields(fcfd_ctx *c);
 int uccd_lines_set(fcfd_ctx *c, int set, int dir, const double *f, const double *u, double *fx, double *fxx);
 int uccd_dir(fcfd_ctx *c, int dir, const double *f, const double *u, double *fx, double *fxx);
-// one WENO5 SSP-RK3 stage of the FP64 advection on the field geometry G
-// (which may carry open faces) with caller pointers, queued on st
 int ls_adv_stage_f32(fcfd_ctx *c, const float *phi, float *phin, const float *nu, const float *nv, const float *nw,
                      float *l1, float *l2, int stage);
-int ls_adv_stage_geom(hipStream_t st, const Geom &G, const double *phi, double *phin, const double *nu,
-                      const double *nv, const double *nw, double *l1, double *l2, double dt, int stage);
+// a block of a multi-block layout: its geometry (with open faces) and its
+// offset in a stack
+struct BlockGeom {
+    Geom G;
+    long off;
+};
+// one WENO5 SSP-RK3 stage on every block of a layout in one launch: tab on
+// the device, nx, ny, nz the largest block's extents; phin's ghosts are not
+// written
+int ls_adv_stage_blocks(hipStream_t st, int ncu, const BlockGeom *tab, int nblk, int dim, int nx, int ny, int nz,
+                        const double *phi, double *phin, const double *nu, const double *nv, const double *nw,
+                        double *l1, double *l2, double dt, int stage);
 int ccd_setup(fcfd_ctx *c);
 int surface_norms(fcfd_ctx *c, const double *phi, int full);
 int curv_kernel(fcfd_ctx *c);

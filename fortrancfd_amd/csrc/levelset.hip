@@ -363,28 +363,42 @@ int mpls(fcfd_ctx *c) {
 }
 
 // ------------------------------------------------------------- advection
-constexpr int LS_KC = 16;   // planes per block of the 3D stage
-
 // One SSP-RK3 stage of level_set_rk3_solver, fused: velocity flux split
 // (source_setup :67-96, with the bc() copy of s1/s2 realised by clamped
 // indices), WENO5-JS faces (:162-219), flux divergence (:145-158) and the
 // increment-form stage update (:13-60), with every face computed once.
 // T = float is the single-precision variant (same operation order, FP32
 // weights of weno.h); the velocity is vs (nu, nv, nw).
-// A block covers a 64 x 4 tile and, in 3D, walks LS_KC planes of it (2D:
-// the block's slice, a case of a batched stack).  Per plane its 256 threads
-// compute the 4 x 65 x-faces and 5 x 64 y-faces of the tile into LDS (580
-// faces where two faces per cell and direction take 1024), then each cell
-// differences them.  The z flux of face k+1/2 is the k-1/2 flux of the next
-// plane, from a 7-plane window of (w, phi) splits carried in registers.  The
-// LDS plane is double buffered, one barrier per plane.  Face value F =
-// WENO_left(s1 at f-2..f+2) + WENO_right(s2 at f-1..f+3) at clamped
+// A block covers a TX x 256/TX tile and, in 3D, walks kc planes of it (2D:
+// the block's slice, a case of a batched stack).  Per plane each thread
+// computes the x-face and the y-face below its cell into LDS, the first TX
+// threads the tile's last row of y-faces and one thread per row the last
+// x-face; then each cell differences them.  The z flux of face k+1/2 is the
+// k-1/2 flux of the next plane, from a 7-plane window of (w, phi) splits
+// carried in registers.  The LDS plane is double buffered, one barrier per
+// plane; what a cell needs besides the faces is loaded before it.  Face value
+// F = WENO_left(s1 at f-2..f+2) + WENO_right(s2 at f-1..f+3) at clamped
 // positions; L sums F(+1/2) - F(-1/2) per direction.
-template <int DIM, typename T>
-__global__ void __launch_bounds__(256) k_ls_adv_stage_kf(const T *__restrict__ phi, T *__restrict__ phin,
-                                                         const T *__restrict__ nu, const T *__restrict__ nv,
-                                                         const T *__restrict__ nw, T *__restrict__ l1,
-                                                         T *__restrict__ l2, Geom G, T dt, T vs, int stage) {
+// With TX = 64 a wave is one row, so a face's six rows (y) or its row (x)
+// have scalar bases and one vector offset.
+//
+// What bounds it: a plane is a chain of memory round trips, the faces one
+// after the other and a barrier, about 5 us; a block's planes are serial, so
+// the walk is only as long as the grid can afford (stage_planes).  434 us at
+// 256^3 (533 with 256 threads striding over the 580 faces at 64-bit
+// addresses), 54 us at 128^3 (83 with 16 planes a block whatever the grid), 30
+// us in FP32 at 101 x 87 x 117 (90).
+template <int DIM, typename T, int TX>
+struct StageLds {
+    T fx[2][256 / TX][TX + 1], fy[2][256 / TX + 1][TX];
+};
+
+template <int DIM, typename T, int TX>
+__device__ __forceinline__ void ls_adv_stage_body(StageLds<DIM, T, TX> &sh, const T *__restrict__ phi,
+                                                  T *__restrict__ phin, const T *__restrict__ nu,
+                                                  const T *__restrict__ nv, const T *__restrict__ nw,
+                                                  T *__restrict__ l1, T *__restrict__ l2, const Geom &G, T dt, T vs,
+                                                  int stage, int kc, int bx_, int by_, int bz_) {
     // Products are fused into adds only within one statement here: the flux
     // splits s1, s2 of the z window are formed in the plane that loads them,
     // and with fusion across statements a face whose splits were formed in
@@ -393,39 +407,37 @@ __global__ void __launch_bounds__(256) k_ls_adv_stage_kf(const T *__restrict__ p
     // wherever a walk starts, which keeps block-by-block runs bit for bit
     // equal to whole-field ones.
 #pragma clang fp contract(on)
-    constexpr int TX = 64, TY = 4, NFX = TY * (TX + 1), NFY = (TY + 1) * TX;
-    __shared__ T fxs[2][TY][TX + 1], fys[2][TY + 1][TX];
-    int bx_, by_, bz_;
-    xcd_block(bx_, by_, bz_);
-    const int tx = threadIdx.x, ty = threadIdx.y, t = ty * TX + tx;
+    constexpr int TY = 256 / TX;
+    const int tx = threadIdx.x, t = threadIdx.y * TX + tx;
+    const int ty = TX == WAVE ? __builtin_amdgcn_readfirstlane(threadIdx.y) : (int)threadIdx.y;
     const int i0 = bx_ * TX, j0 = by_ * TY, i = i0 + tx, j = j0 + ty;
-    // 3D: LS_KC planes per block; 2D: the block's slice (a case of a batched stack)
-    const int k0 = DIM == 3 ? bz_ * LS_KC : bz_, k1 = DIM == 3 ? min(k0 + LS_KC, G.nz) : bz_ + 1;
+    // 3D: kc planes per block; 2D: the block's slice (a case of a batched stack)
+    const int k0 = DIM == 3 ? bz_ * kc : bz_, k1 = DIM == 3 ? min(k0 + kc, G.nz) : bz_ + 1;
+    if (i0 >= G.nx || j0 >= G.ny || k0 >= G.nz) return;   // the whole block
     const bool in = i < G.nx && j < G.ny;
     const int ic = min(i, G.nx - 1), jc = min(j, G.ny - 1);
     const T half = (T)0.5, EPS = (T)1.0e-13;
-    const T hx = (T)G.dx, hy = (T)G.dy, hz = (T)G.dz;
-    // face f + 1/2 of a line: positions clamp(f - 2 + m), m = 0..5, into
-    // [-lo, n - 1 + hi] (lo, hi = 0 on physical faces), at stride st from the
-    // line start a0
-    auto face = [&](const T *__restrict__ vel, long a0, long st, int f, int lo, int hi) -> T {
+    const T rhx = (T)(1.0 / G.dx), rhy = (T)(1.0 / G.dy), rhz = (T)(1.0 / G.dz);
+    const int xlo = -G.ox0, xhi = G.nx - 1 + G.ox1, ylo = -G.oy0, yhi = G.ny - 1 + G.oy1;
+    const int zlo = -G.oz0, zhi = G.nz - 1 + G.oz1;
+    auto flux = [&](const T (&u)[6], const T (&p)[6]) -> T {
         T s1[6], s2[6];
 #pragma unroll
         for (int m = 0; m < 6; ++m) {
-            const long a = a0 + (long)clampi(f - 2 + m, lo, hi) * st;
-            const T u = vs * vel[a], p = phi[a];
-            s1[m] = half * (u + fabs(u)) * p;
-            s2[m] = half * (u - fabs(u)) * p;
+            const T v = vs * u[m];
+            s1[m] = half * (v + fabs(v)) * p[m];
+            s2[m] = half * (v - fabs(v)) * p[m];
         }
         return weno_left(s1[0], s1[1], s1[2], s1[3], s1[4], EPS) + weno_right(s2[1], s2[2], s2[3], s2[4], s2[5], EPS);
     };
+    const unsigned co = (unsigned)(ic + G.g) * (unsigned)sizeof(T);
     // z window of this column: positions clamp(k - 3 + m), m = 0..6
     T s1z[7], s2z[7], Fl = 0;
     if (DIM == 3) {
 #pragma unroll
         for (int m = 0; m < 7; ++m) {
-            const long a = G.id(ic, jc, clampi(k0 - 3 + m, -G.oz0, G.nz - 1 + G.oz1));
-            const T u = vs * nw[a], p = phi[a];
+            const long row = G.id(0, jc, clampi(k0 - 3 + m, zlo, zhi)) - G.g;
+            const T u = vs * at_bytes(nw + row, co), p = at_bytes(phi + row, co);
             s1z[m] = half * (u + fabs(u)) * p;
             s2z[m] = half * (u - fabs(u)) * p;
         }
@@ -434,15 +446,44 @@ __global__ void __launch_bounds__(256) k_ls_adv_stage_kf(const T *__restrict__ p
     }
     for (int k = k0; k < k1; ++k) {
         const int b = k & 1;
-        for (int e = t; e < NFX + NFY; e += TX * TY) {
-            if (e < NFX) {   // x-face i0 - 1 + c + 1/2 of row j0 + r
-                const int r = e / (TX + 1), c = e - r * (TX + 1);
-                fxs[b][r][c] = face(nu, G.id(0, min(j0 + r, G.ny - 1), k), 1, i0 - 1 + c, -G.ox0, G.nx - 1 + G.ox1);
-            } else {         // y-face j0 - 1 + r + 1/2 of column i0 + c
-                const int q = e - NFX, r = q / TX, c = q - r * TX;
-                fys[b][r][c] = face(nv, G.id(min(i0 + c, G.nx - 1), 0, k), G.sx, j0 - 1 + r, -G.oy0,
-                                    G.ny - 1 + G.oy1);
+        // this cell's operands and the z window's next plane, ahead of the faces
+        const long rc = G.id(0, jc, k) - G.g;
+        const T pc = at_bytes(phi + rc, co);
+        const T l1o = stage >= 1 ? at_bytes(l1 + rc, co) : (T)0, l2o = stage == 2 ? at_bytes(l2 + rc, co) : (T)0;
+        T wn = 0, pn = 0;
+        if (DIM == 3) {
+            const long row = G.id(0, jc, clampi(k + 4, zlo, zhi)) - G.g;
+            wn = at_bytes(nw + row, co);
+            pn = at_bytes(phi + row, co);
+        }
+        // the x-face and the y-face below the cell, then the tile's last
+        // y-face row (first TX threads) and last x-faces (TY threads), one
+        // after the other: unrolled, their loads take 198 VGPRs.  A face reads
+        // positions clamp(f - 2 + m) of its line at byte offsets from the
+        // plane's first cell.
+        const long pl = G.id(0, 0, k) - G.g - (long)G.g * G.sx;
+        const T *pp = phi + pl;
+#pragma unroll 1
+        for (int r = 0; r < 3; ++r) {
+            const bool last = r == 2, xf = r == 0 || (last && t >= 128);
+            if (last && !(t < TX || (t >= 128 && t < 128 + TY))) break;
+            const T *vp = (xf ? nu : nv) + pl;
+            const int row = xf ? (last ? min(j0 + t - 128, G.ny - 1) : jc) : 0;
+            const int f = xf ? (last ? i0 + TX - 1 : i - 1) : (last ? j0 + TY - 1 : j - 1);
+            const int lo = xf ? xlo : ylo, hi = xf ? xhi : yhi;
+            const unsigned st = (xf ? 1u : (unsigned)G.sx) * (unsigned)sizeof(T);
+            const unsigned o0 = xf ? (unsigned)((row + G.g) * (int)G.sx + G.g) * (unsigned)sizeof(T)
+                                   : co + (unsigned)(G.g * (int)G.sx) * (unsigned)sizeof(T);
+            T u[6], p[6];
+#pragma unroll
+            for (int m = 0; m < 6; ++m) {
+                const unsigned o = o0 + (unsigned)clampi(f - 2 + m, lo, hi) * st;
+                u[m] = at_bytes(vp, o);
+                p[m] = at_bytes(pp, o);
             }
+            const T F = flux(u, p);
+            if (xf) sh.fx[b][last ? t - 128 : ty][last ? TX : tx] = F;
+            else sh.fy[b][last ? TY : ty][tx] = F;
         }
         __syncthreads();
         // face k + 1/2: gm from s1(k-2..k+2), fp from s2(k-1..k+3)
@@ -451,21 +492,20 @@ __global__ void __launch_bounds__(256) k_ls_adv_stage_kf(const T *__restrict__ p
             Fr = weno_left(s1z[1], s1z[2], s1z[3], s1z[4], s1z[5], EPS) +
                  weno_right(s2z[2], s2z[3], s2z[4], s2z[5], s2z[6], EPS);
         if (in) {
-            const long id = G.id(i, j, k);
-            T L = -(fxs[b][ty][tx + 1] - fxs[b][ty][tx]) / hx;
-            L = L + (-(fys[b][ty + 1][tx] - fys[b][ty][tx]) / hy);
-            if (DIM == 3) L = L + (-(Fr - Fl) / hz);
+            T L = -(sh.fx[b][ty][tx + 1] - sh.fx[b][ty][tx]) * rhx;
+            L = L + (-(sh.fy[b][ty + 1][tx] - sh.fy[b][ty][tx]) * rhy);
+            if (DIM == 3) L = L + (-(Fr - Fl) * rhz);
             T src;
             if (stage == 0) {
-                l1[id] = L;
+                at_bytes(l1 + rc, co) = L;
                 src = L;
             } else if (stage == 1) {
-                l2[id] = L;
-                src = ((T)-3.0 * l1[id] + L) / (T)4.0;
+                at_bytes(l2 + rc, co) = L;
+                src = ((T)-3.0 * l1o + L) * (T)0.25;
             } else {
-                src = (-l1[id] - l2[id] + (T)8.0 * L) / (T)12.0;
+                src = (-l1o - l2o + (T)8.0 * L) / (T)12.0;
             }
-            phin[id] = phi[id] + src * dt;
+            at_bytes(phin + rc, co) = pc + src * dt;
         }
         if (DIM == 3) {
             Fl = Fr;
@@ -475,12 +515,45 @@ __global__ void __launch_bounds__(256) k_ls_adv_stage_kf(const T *__restrict__ p
                 s1z[m] = s1z[m + 1];
                 s2z[m] = s2z[m + 1];
             }
-            const long a = G.id(ic, jc, clampi(k + 4, -G.oz0, G.nz - 1 + G.oz1));
-            const T u = vs * nw[a], p = phi[a];
-            s1z[6] = half * (u + fabs(u)) * p;
-            s2z[6] = half * (u - fabs(u)) * p;
+            const T u = vs * wn;
+            s1z[6] = half * (u + fabs(u)) * pn;
+            s2z[6] = half * (u - fabs(u)) * pn;
         }
     }
+}
+
+template <int DIM, typename T, int TX>
+__global__ void __launch_bounds__(256) k_ls_adv_stage(const T *__restrict__ phi, T *__restrict__ phin,
+                                                      const T *__restrict__ nu, const T *__restrict__ nv,
+                                                      const T *__restrict__ nw, T *__restrict__ l1,
+                                                      T *__restrict__ l2, Geom G, T dt, T vs, int stage, int kc) {
+    __shared__ StageLds<DIM, T, TX> sh;
+    int bx_, by_, bz_;
+    xcd_block(bx_, by_, bz_);
+    ls_adv_stage_body<DIM, T, TX>(sh, phi, phin, nu, nv, nw, l1, l2, G, dt, vs, stage, kc, bx_, by_, bz_);
+}
+
+// the same stage on every block of a multi-block layout in one launch:
+// tab[b] places block b in the stacks; the grid covers the largest block, nz
+// walks per block along z.  (A launch per block of 80 x 75 x 85 cells leaves
+// the chip nearly empty: 75 us each, eight in a row; together 134 us.)
+template <int DIM, int TX>
+__global__ void __launch_bounds__(256) k_ls_adv_stage_blocks(const double *__restrict__ phi,
+                                                             double *__restrict__ phin,
+                                                             const double *__restrict__ nu,
+                                                             const double *__restrict__ nv,
+                                                             const double *__restrict__ nw, double *__restrict__ l1,
+                                                             double *__restrict__ l2,
+                                                             const BlockGeom *__restrict__ tab, double dt, int stage,
+                                                             int kc, int nz) {
+    __shared__ StageLds<DIM, double, TX> sh;
+    int bx_, by_, bz_;
+    xcd_block(bx_, by_, bz_);
+    const int b = bz_ / nz;
+    const Geom G = tab[b].G;
+    const long o = tab[b].off;
+    ls_adv_stage_body<DIM, double, TX>(sh, phi + o, phin + o, nu + o, nv + o, DIM == 3 ? nw + o : nullptr, l1 + o,
+                                       l2 + o, G, dt, 1.0, stage, kc, bx_, by_, bz_ - b * nz);
 }
 
 // One SSP-RK3 stage with the UCCD source L = -(u phi_x + v phi_y + w phi_z)
@@ -514,35 +587,61 @@ __global__ void __launch_bounds__(256) k_ls_uccd_stage(const double *__restrict_
     phin[id] = phi[id] + src * dt;
 }
 
-// launch grid of k_ls_adv_stage_kf: LS_KC planes per block
-static dim3 grid_km(const Geom &G, dim3 blk) {
-    return dim3((G.nx + blk.x - 1) / blk.x, (G.ny + blk.y - 1) / blk.y, (G.nz + LS_KC - 1) / LS_KC);
+// planes a block of the 3D stage walks: 16 (one plane in 17 costs its first
+// z-face and window twice), halved while the launch would leave CUs with
+// fewer than 8 blocks, down to 4
+static int stage_planes(long tiles, int nz, int ncu) {
+    int kc = 16;
+    while (kc > 4 && tiles * ((nz + kc - 1) / kc) < 8L * ncu) kc /= 2;
+    return kc;
+}
+
+template <int DIM, typename T>
+static int launch_stage(hipStream_t st, int ncu, const Geom &G, const T *phi, T *phin, const T *nu, const T *nv,
+                        const T *nw, T *l1, T *l2, T dt, T vs, int stage) {
+    const dim3 blk = tile_rows(G.nx);
+    const dim3 tiles((G.nx + blk.x - 1) / blk.x, (G.ny + blk.y - 1) / blk.y, G.nz);
+    const int kc = DIM == 3 ? stage_planes((long)tiles.x * tiles.y, G.nz, ncu) : 1;
+    const dim3 grd(tiles.x, tiles.y, (G.nz + kc - 1) / kc);
+    if (blk.x == 64)
+        hipLaunchKernelGGL((k_ls_adv_stage<DIM, T, 64>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, G, dt, vs,
+                           stage, kc);
+    else
+        hipLaunchKernelGGL((k_ls_adv_stage<DIM, T, 32>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, G, dt, vs,
+                           stage, kc);
+    FCFD_CHECK(hipGetLastError());
+    return FCFD_OK;
 }
 
 // one WENO5 SSP-RK3 stage from phi into phin with the context's velocity
 // (the stage sources stay in l1/l2 as in ls_advect); no ghost update
 int ls_adv_stage(fcfd_ctx *c, const double *phi, double *phin, int stage) {
-    const Geom &G = c->G;
-    dim3 blk(64, 4), grd = grid_interior(G, blk);
-    if (G.dim == 3)
-        hipLaunchKernelGGL((k_ls_adv_stage_kf<3, double>), grid_km(G, blk), blk, 0, c->stream, phi, phin,
-                           c->f[FCFD_NU], c->f[FCFD_NV], c->f[FCFD_NW], c->l1, c->l2, G, c->pr.dt, c->vscale, stage);
-    else
-        hipLaunchKernelGGL((k_ls_adv_stage_kf<2, double>), grd, blk, 0, c->stream, phi, phin, c->f[FCFD_NU],
-                           c->f[FCFD_NV], nullptr, c->l1, c->l2, G, c->pr.dt, c->vscale, stage);
-    FCFD_CHECK(hipGetLastError());
-    return FCFD_OK;
+    double **F = c->f;
+    if (c->G.dim == 3)
+        return launch_stage<3, double>(c->stream, c->ncu, c->G, phi, phin, F[FCFD_NU], F[FCFD_NV], F[FCFD_NW], c->l1,
+                                       c->l2, c->pr.dt, c->vscale, stage);
+    return launch_stage<2, double>(c->stream, c->ncu, c->G, phi, phin, F[FCFD_NU], F[FCFD_NV], nullptr, c->l1, c->l2,
+                                   c->pr.dt, c->vscale, stage);
 }
 
-int ls_adv_stage_geom(hipStream_t st, const Geom &G, const double *phi, double *phin, const double *nu,
-                      const double *nv, const double *nw, double *l1, double *l2, double dt, int stage) {
-    dim3 blk(64, 4);
-    if (G.dim == 3)
-        hipLaunchKernelGGL((k_ls_adv_stage_kf<3, double>), grid_km(G, blk), blk, 0, st, phi, phin, nu, nv, nw, l1, l2,
-                           G, dt, 1.0, stage);
-    else
-        hipLaunchKernelGGL((k_ls_adv_stage_kf<2, double>), grid_interior(G, blk), blk, 0, st, phi, phin, nu, nv,
-                           nullptr, l1, l2, G, dt, 1.0, stage);
+int ls_adv_stage_blocks(hipStream_t st, int ncu, const BlockGeom *tab, int nblk, int dim, int nx, int ny, int nz,
+                        const double *phi, double *phin, const double *nu, const double *nv, const double *nw,
+                        double *l1, double *l2, double dt, int stage) {
+    const dim3 blk = tile_rows(nx);
+    const dim3 tiles((nx + blk.x - 1) / blk.x, (ny + blk.y - 1) / blk.y);
+    const int kc = dim == 3 ? stage_planes((long)tiles.x * tiles.y * nblk, nz, ncu) : 1, kz = (nz + kc - 1) / kc;
+    const dim3 grd(tiles.x, tiles.y, (unsigned)(nblk * kz));
+#define FCFD_SB(D_, X_)                                                                                         \
+    hipLaunchKernelGGL((k_ls_adv_stage_blocks<D_, X_>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, tab, dt, \
+                       stage, kc, kz)
+    if (dim == 3) {
+        if (blk.x == 64) FCFD_SB(3, 64);
+        else FCFD_SB(3, 32);
+    } else {
+        if (blk.x == 64) FCFD_SB(2, 64);
+        else FCFD_SB(2, 32);
+    }
+#undef FCFD_SB
     FCFD_CHECK(hipGetLastError());
     return FCFD_OK;
 }
@@ -581,18 +680,12 @@ int ls_advect(fcfd_ctx *c) {
     for (int s = 0; s < 3; ++s) {
         {
             ProfScope ps_(c, R_LS_ADV);
-            if (G.dim == 3)
-                hipLaunchKernelGGL((k_ls_adv_stage_kf<3, double>), grid_km(G, blk), blk, 0, c->stream, a, b,
-                                   c->f[FCFD_NU], c->f[FCFD_NV], c->f[FCFD_NW], c->l1, c->l2, G, c->pr.dt, c->vscale,
-                                   s);
-            else
-                hipLaunchKernelGGL((k_ls_adv_stage_kf<2, double>), grd, blk, 0, c->stream, a, b, c->f[FCFD_NU],
-                                   c->f[FCFD_NV], nullptr, c->l1, c->l2, G, c->pr.dt, c->vscale, s);
-            FCFD_CHECK(hipGetLastError());
+            FCFD_TRY(ls_adv_stage(c, a, b, s));
         }
-        FCFD_TRY(bc_scalar(c, b));
         double *t = a; a = b; b = t;
     }
+    // the stages read no ghosts (clamped indices): only the result's are filled
+    FCFD_TRY(bc_scalar(c, a));
     // three stages end in the buffer that was phiB: swap roles
     c->phiB = c->f[FCFD_PHI];
     c->f[FCFD_PHI] = a;
@@ -603,46 +696,27 @@ int ls_advect(fcfd_ctx *c) {
 // velocity times the context's scale); no ghost update
 int ls_adv_stage_f32(fcfd_ctx *c, const float *phi, float *phin, const float *nu, const float *nv, const float *nw,
                      float *l1, float *l2, int stage) {
-    const Geom &G = c->G;
-    dim3 blk(64, 4);
     const float dt = (float)c->pr.dt, vs = (float)c->vscale;
-    if (G.dim == 3)
-        hipLaunchKernelGGL((k_ls_adv_stage_kf<3, float>), grid_km(G, blk), blk, 0, c->stream, phi, phin, nu, nv, nw,
-                           l1, l2, G, dt, vs, stage);
-    else
-        hipLaunchKernelGGL((k_ls_adv_stage_kf<2, float>), grid_interior(G, blk), blk, 0, c->stream, phi, phin, nu,
-                           nv, (const float *)nullptr, l1, l2, G, dt, vs, stage);
-    FCFD_CHECK(hipGetLastError());
-    return FCFD_OK;
+    if (c->G.dim == 3)
+        return launch_stage<3, float>(c->stream, c->ncu, c->G, phi, phin, nu, nv, nw, l1, l2, dt, vs, stage);
+    return launch_stage<2, float>(c->stream, c->ncu, c->G, phi, phin, nu, nv, nullptr, l1, l2, dt, vs, stage);
 }
 
 // One SSP-RK3 step in FP32 of a caller's level set phi with the caller's
 // FP32 cell velocity times the context's scale: stage 0 phi -> B, stage 1
 // B -> C, stage 2 C -> phi (each stage reads its input and writes another
-// array), the zero-gradient ghost copy after each stage as in ls_advect.
+// array, no ghosts), then the zero-gradient ghost copy as in ls_advect.
 int ls_advect_f32(fcfd_ctx *c, float *phi, const float *nu, const float *nv, const float *nw) {
     const Geom &G = c->G;
     if (!c->adv32[0])
         for (int q = 0; q < 4; ++q) FCFD_CHECK(hipMalloc((void **)&c->adv32[q], sizeof(float) * G.ntot));
     float *B = c->adv32[0], *Cb = c->adv32[1], *l1 = c->adv32[2], *l2 = c->adv32[3];
-    dim3 blk(64, 4), grd = grid_interior(G, blk);
-    const float dt = (float)c->pr.dt, vs = (float)c->vscale;
     float *in[3] = {phi, B, Cb}, *out[3] = {B, Cb, phi};
     for (int s = 0; s < 3; ++s) {
-        {
-            ProfScope ps_(c, R_LS_ADV);
-            if (G.dim == 3)
-                hipLaunchKernelGGL((k_ls_adv_stage_kf<3, float>), grid_km(G, blk), blk, 0, c->stream, in[s], out[s], nu,
-                                   nv, nw, l1,
-                                   l2, G, dt, vs, s);
-            else
-                hipLaunchKernelGGL((k_ls_adv_stage_kf<2, float>), grd, blk, 0, c->stream, in[s], out[s], nu, nv,
-                                   (const float *)nullptr, l1, l2, G, dt, vs, s);
-            FCFD_CHECK(hipGetLastError());
-        }
-        FCFD_TRY(bc_scalar_f32(c, out[s]));
+        ProfScope ps_(c, R_LS_ADV);
+        FCFD_TRY(ls_adv_stage_f32(c, in[s], out[s], nu, nv, nw, l1, l2, s));
     }
-    return FCFD_OK;
+    return bc_scalar_f32(c, phi);
 }
 
 // ------------------------------------------------------------- reinit
