@@ -6,6 +6,7 @@ in test_gpu_parity.py); and the multi-block launch on blocks of unequal
 extents, bit for bit the whole-field step."""
 import numpy as np
 import pytest
+import torch   # before the library: both then share one HIP runtime
 
 from cases import bubble, max_rel, node_velocities
 from fortrancfd_amd.types import Case
@@ -41,7 +42,6 @@ def test_stage_tiles(size):
 
 @pytest.mark.parametrize("size,nb", [((67, 11, 13), (2, 2, 3)), ((129, 10, 9), (2, 3, 2)), ((70, 31, 1), (3, 4, 1))])
 def test_blocks_in_one_launch(size, nb):
-    import torch
     from fortrancfd_amd import Solver
     from fortrancfd_amd.blocks import Blocks
     from fortrancfd_amd.types import bc_copy
