@@ -1,5 +1,5 @@
 // adjoint.hip — discrete adjoint of the WENO5 flux-split level-set advection
-// with SSP-RK3 (the forward is k_ls_adv_stage_kf in levelset.hip, following
+// with SSP-RK3 (the forward is k_ls_adv_stage in levelset.hip, following
 // `Two phase flows/newOpenMP/3D+IBM/src/interface_solver/
 // level_set_rk3_solver.f90:1-219`).  There is no counterpart in the
 // reference: this is the differentiation entry point of the path.
@@ -71,7 +71,6 @@ __device__ __forceinline__ void face_adj(const T *s1, const T *s2, T fbar, T *gb
 
 constexpr int ADJ_TX = 64, ADJ_TY = 4;
 constexpr int ADJ_NFX = ADJ_TX + 5;   // x faces i0-3 .. i0+65 of a 64-cell row
-constexpr int ADJ_KC = 16;            // z cells per thread
 
 // x pass: block 64 x 4 cells of one plane; the 69 faces of each row are
 // computed by the row's wave (two passes) into LDS, then each cell gathers
@@ -134,22 +133,24 @@ __global__ void __launch_bounds__(256) k_adj_x(const T *__restrict__ psi, const 
 }
 
 // y and z passes: each thread walks the faces of one line along axis AX
-// (1: y, 2: z) that reach its ADJ_KC cells, keeping the samples of positions
+// (1: y, 2: z) that reach its kc cells, keeping the samples of positions
 // f-2 .. f+3 and the s1 / s2 adjoints of cells f-2 .. f+3 in registers;
 // after face f no later face reaches cell f-2, which is then complete.
-// Threads run along x (coalesced); blockIdx.y picks the other index.
+// Threads run along x (coalesced); blockIdx.y picks the other index.  A
+// face's operands and those of the cell it completes are loaded a face
+// ahead: a walk is a serial chain of faces, each about 210 operations deep.
 template <int AX, typename T>
 __global__ void __launch_bounds__(256) k_adj_walk(const T *__restrict__ psi, const T *__restrict__ vel,
                                                   const T *__restrict__ w, T *__restrict__ out,
-                                                  T *__restrict__ velbar, Geom G, T vs) {
+                                                  T *__restrict__ velbar, Geom G, T vs, int kc) {
     int bx_, by_, bz_;
     xcd_block(bx_, by_, bz_);
     const int i = bx_ * blockDim.x + threadIdx.x, o = by_ * blockDim.y + threadIdx.y;
     const int n = AX == 1 ? G.ny : G.nz;
-    const int k0 = bz_ * ADJ_KC, k1 = min(k0 + ADJ_KC, n);
+    const int k0 = bz_ * kc, k1 = min(k0 + kc, n);
     if (i >= G.nx || o >= (AX == 1 ? G.nz : G.ny)) return;
     const long c0 = AX == 1 ? G.id(i, 0, o) : G.id(i, o, 0), st = AX == 1 ? G.sx : G.sxy;
-    const T h = (T)(AX == 1 ? G.dy : G.dz), half = (T)0.5, zero = (T)0;
+    const T rh = (T)(1.0 / (AX == 1 ? G.dy : G.dz)), half = (T)0.5, zero = (T)0;
     const int fa = max(-1, k0 - 3), fz = min(n - 1, k1 + 1);
     T s1[6], s2[6], acc1[6], acc2[6];
 #pragma unroll
@@ -161,19 +162,30 @@ __global__ void __launch_bounds__(256) k_adj_walk(const T *__restrict__ psi, con
         acc1[m] = zero;
         acc2[m] = zero;
     }
-    auto finish = [&](int c, T s1b, T s2b) {
+    struct Cell {
+        T u, ph, o, vb;
+    };
+    auto load = [&](int c) {   // operands of cell c (off this walk's cells: unused, and another walk may be writing them)
+        const long id = c0 + clampi(c, k0, k1 - 1) * st;
+        return Cell{vs * vel[id], psi[id], out[id], velbar ? velbar[id] : zero};
+    };
+    auto finish = [&](int c, const Cell &q, T s1b, T s2b) {
         const long id = c0 + c * st;
         T pb, vb;
-        adj_cell<T>(s1b, s2b, vs * vel[id], psi[id], vs, pb, vb);
-        out[id] = out[id] + pb;
-        if (velbar) velbar[id] += vb;
+        adj_cell<T>(s1b, s2b, q.u, q.ph, vs, pb, vb);
+        out[id] = q.o + pb;
+        if (velbar) velbar[id] = q.vb + vb;
     };
-    T wl = fa >= 0 ? w[c0 + fa * st] : zero;
+    auto seed = [&](int c) { return c >= 0 && c <= n - 1 ? w[c0 + c * st] : zero; };
+    T wl = seed(fa), wr = seed(fa + 1);
     for (int f = fa; f <= fz; ++f) {
-        const T wr = f + 1 <= n - 1 ? w[c0 + (f + 1) * st] : zero;
-        T gb[5], fb[5];
-        face_adj<T>(s1, s2, (wr - wl) / h, gb, fb);
         const int b = f - 2;   // cell of window slot 0
+        const Cell q = load(b);
+        const T wn = seed(f + 2);
+        const long an = c0 + clampi(f + 4, 0, n - 1) * st;   // position (f+1) + 3
+        const T un = vs * vel[an], pn = psi[an];
+        T gb[5], fb[5];
+        face_adj<T>(s1, s2, (wr - wl) * rh, gb, fb);
         if (f - 2 >= 0 && f + 3 <= n - 1) {
 #pragma unroll
             for (int m = 0; m < 5; ++m) {
@@ -191,7 +203,7 @@ __global__ void __launch_bounds__(256) k_adj_walk(const T *__restrict__ psi, con
                 }
             }
         }
-        if (b >= k0 && b < k1) finish(b, acc1[0], acc2[0]);
+        if (b >= k0 && b < k1) finish(b, q, acc1[0], acc2[0]);
 #pragma unroll
         for (int m = 0; m < 5; ++m) {
             acc1[m] = acc1[m + 1];
@@ -201,20 +213,26 @@ __global__ void __launch_bounds__(256) k_adj_walk(const T *__restrict__ psi, con
         }
         acc1[5] = zero;
         acc2[5] = zero;
-        {
-            const long a = c0 + clampi(f + 4, 0, n - 1) * st;   // position (f+1) + 3
-            const T u = vs * vel[a], ph = psi[a];
-            s1[5] = half * (u + fabs(u)) * ph;
-            s2[5] = half * (u - fabs(u)) * ph;
-        }
+        s1[5] = half * (un + fabs(un)) * pn;
+        s2[5] = half * (un - fabs(un)) * pn;
         wl = wr;
+        wr = wn;
     }
     // at the far wall the last cells complete after the last face
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         const int c = fz - 1 + m;
-        if (c >= k0 && c < k1 && c <= n - 1) finish(c, acc1[m], acc2[m]);
+        if (c >= k0 && c < k1 && c <= n - 1) finish(c, load(c), acc1[m], acc2[m]);
     }
+}
+
+// cells per thread of a walk over lines of n cells, `tiles` blocks of lines:
+// 16 (21 faces for 16 cells), halved while the launch would leave CUs with
+// fewer than 4 blocks (of 16 waves a CU), down to 4 (9 faces for 4 cells)
+static int adj_planes(long tiles, int n, int ncu) {
+    int kc = 16;
+    while (kc > 4 && tiles * ((n + kc - 1) / kc) < 4L * ncu) kc /= 2;
+    return kc;
 }
 
 static int adj_scratch(fcfd_ctx *c) {
@@ -237,15 +255,17 @@ static int adjoint_stages(fcfd_ctx *c, const T *phi, const T *phi1, const T *phi
     const T dt = (T)c->pr.dt, vs = (T)c->vscale;
     // walkers: 64 x 4 threads over (x, z) or (x, y) in 3D, 256 along x in 2D
     const dim3 bw = G.dim == 3 ? dim3(64, 4) : dim3(256, 1);
-    const dim3 gy((G.nx + bw.x - 1) / bw.x, (G.nz + bw.y - 1) / bw.y, (G.ny + ADJ_KC - 1) / ADJ_KC);
-    const dim3 gz((G.nx + bw.x - 1) / bw.x, (G.ny + bw.y - 1) / bw.y, (G.nz + ADJ_KC - 1) / ADJ_KC);
+    const long bx = (G.nx + bw.x - 1) / bw.x, by = (G.nz + bw.y - 1) / bw.y, bz = (G.ny + bw.y - 1) / bw.y;
+    const int ky = adj_planes(bx * by, G.ny, c->ncu), kz = adj_planes(bx * bz, G.nz, c->ncu);
+    const dim3 gy(bx, by, (G.ny + ky - 1) / ky), gz(bx, bz, (G.nz + kz - 1) / kz);
     auto adj = [&](const T *psi, const T *base, T *out) {
         if (G.dim == 3)
             hipLaunchKernelGGL((k_adj_x<3, T>), grd, blk, 0, c->stream, psi, nu, w, base, out, ub, G, vs);
         else
             hipLaunchKernelGGL((k_adj_x<2, T>), grd, blk, 0, c->stream, psi, nu, w, base, out, ub, G, vs);
-        hipLaunchKernelGGL((k_adj_walk<1, T>), gy, bw, 0, c->stream, psi, nv, w, out, vb, G, vs);
-        if (G.dim == 3) hipLaunchKernelGGL((k_adj_walk<2, T>), gz, bw, 0, c->stream, psi, nw, w, out, wb, G, vs);
+        hipLaunchKernelGGL((k_adj_walk<1, T>), gy, bw, 0, c->stream, psi, nv, w, out, vb, G, vs, ky);
+        if (G.dim == 3) 
+            hipLaunchKernelGGL((k_adj_walk<2, T>), gz, bw, 0, c->stream, psi, nw, w, out, wb, G, vs, kz);
     };
     const T one = (T)1, three = (T)3, four = (T)4, eight = (T)8, twelve = (T)12;
     // lambda2 = lambda3 + J(phi2)^T (8 dt/12 lambda3)

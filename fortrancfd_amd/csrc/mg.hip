@@ -1304,15 +1304,19 @@ __global__ void __launch_bounds__(CDENSE) k_coarse_dense(T *__restrict__ eout, c
 // coarse cells with all their children, so the restriction needs no
 // exchange.  FP64 would need twice the registers (spills) and keeps TAIL_MAX.
 //
-// The levels of at most TAIL_MAX cells (TAIL_CPT cells per thread) keep their
-// error in LDS for the whole cycle (ghosted boxes of TAIL_ELDS elements in
-// all, ghosts 0): the owner thread holds the cell's six face coefficients
-// and rhs in registers, loaded from global memory once per down and once per
-// up phase, so a half-sweep waits on LDS instead of on dependent L2 loads.
-// Each level's error is written back at the end of its up phase.
-constexpr int TAIL_MAX = 2048, TAIL_THREADS = 1024, TAIL_LEVELS = 8, TAIL_CPT = TAIL_MAX / TAIL_THREADS;
+// The levels of at most TAIL_MAX cells keep their error in LDS for the whole
+// cycle (ghosted boxes of TAIL_ELDS elements in all, ghosts 0).  A thread
+// owns pairs of neighbouring cells of a row, one of each colour, so that
+// every thread has one cell per pair in every half-sweep; it holds their LDS
+// positions, face coefficients, reciprocal diagonals and rhs in registers,
+// loaded from global memory once per down and once per up phase.  A
+// half-sweep is then seven LDS reads, the update and a barrier.  (With cells
+// dealt out in memory order half of the threads were idle in a half-sweep,
+// and every one recomputed its cells' positions.)  Each level's error is
+// written back at the end of its up phase.
+constexpr int TAIL_MAX = 4096, TAIL_THREADS = 1024, TAIL_LEVELS = 8, TAIL_PAIRS = TAIL_MAX / (2 * TAIL_THREADS);
 constexpr int TAIL_TOP = 8192, TAIL_LDS = 12288, TAIL_SLOTS = TAIL_TOP / TAIL_THREADS;
-constexpr int TAIL_ELDS = 4096;
+constexpr int TAIL_ELDS = 8192;
 
 template <typename T>
 struct TailLevel {
@@ -1335,11 +1339,26 @@ struct TailArgs {
     int eoff[TAIL_LEVELS]; // offset of each such level's ghosted box
 };
 
+// 1 / sc of a Gauss-Seidel update in the cycle's precision (0 off the grid)
+__device__ __forceinline__ float tail_recip(float sc) { return sc > 0.f ? __builtin_amdgcn_rcpf(sc) : 0.f; }
+__device__ __forceinline__ double tail_recip(double sc) { return sc > 0.0 ? 1.0 / sc : 0.0; }
+
+// the pairs of an LDS-resident level owned by a thread: [pair][colour]
+template <typename T>
+struct TailCells {
+    int np;                        // pairs this thread owns
+    int li[TAIL_PAIRS][2];         // position in the level's LDS box
+    T cf[TAIL_PAIRS][2][6];        // face coefficients E W N S T B, as stencil() forms them
+    T rs[TAIL_PAIRS][2];           // reciprocal diagonal; 0 where the pair has no such cell
+    T f[TAIL_PAIRS][2];            // rhs
+};
+
 template <typename T, int DIM>
 __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
     if (A.lv[0].L.skipped()) return;
     __shared__ double red[TAIL_THREADS / WAVE];
-    __shared__ double bvec[CDENSE];
+    constexpr int CPARTS = TAIL_THREADS / CDENSE;
+    __shared__ double bvec[CDENSE], dpart[CPARTS][CDENSE];
     const int t = threadIdx.x;
     // a batched 2D stack runs one workgroup per case on its slice kq; the
     // level layouts describe one slice
@@ -1382,50 +1401,55 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         return (i + 1) + (L.nx + 2) * ((j + 1) + (DIM == 3 ? (L.ny + 2) * (k + 1) : 0));
     };
     auto boxn = [](const Lay &L) { return (L.nx + 2) * (L.ny + 2) * (DIM == 3 ? L.nz + 2 : 1); };
-    // the owner's face coefficients (E W N S T B, as stencil() forms them) and
-    // rhs of its cells c = t + u TAIL_THREADS
-    auto load_regs = [&](const TailLevel<T> &V, T (&cf)[TAIL_CPT][6], T (&fv)[TAIL_CPT]) {
+    // this thread's pairs of a level: pair q = t + u TAIL_THREADS covers cells
+    // 2m, 2m + 1 of a row; the cell of colour c is i = 2m + ((j + k + c) & 1)
+    auto load_cells = [&](const TailLevel<T> &V, TailCells<T> &Q) {
         const Lay &L = V.L;
+        const int mx = (L.nx + 1) / 2, npair = mx * L.ny * L.nz;
+        Q.np = 0;
 #pragma unroll
-        for (int u = 0; u < TAIL_CPT; ++u) {
-            const int c = t + u * TAIL_THREADS;
-            if (c < ncells(L)) {
-                int i, j, k;
-                cell_coords(L, c, i, j, k);
-                const long id = L.id(i, j, k);
-                cf[u][0] = (T)V.bx[id] * (T)V.ih.x;
-                cf[u][1] = (T)V.bx[id - 1] * (T)V.ih.x;
-                cf[u][2] = (T)V.by[id] * (T)V.ih.y;
-                cf[u][3] = (T)V.by[id - L.sx] * (T)V.ih.y;
-                cf[u][4] = DIM == 3 ? (T)V.bz[id] * (T)V.ih.z : (T)0;
-                cf[u][5] = DIM == 3 ? (T)V.bz[id - L.sxy] * (T)V.ih.z : (T)0;
-                fv[u] = V.f[id];
+        for (int u = 0; u < TAIL_PAIRS; ++u) {
+            const int q = t + u * TAIL_THREADS;
+            if (q >= npair) continue;
+            Q.np = u + 1;
+            const int r = q / mx, m = q - r * mx, k = r / L.ny, j = r - k * L.ny;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int i = 2 * m + ((j + k + c) & 1);
+                const long id = L.id(min(i, L.nx - 1), j, k + kq);
+                T *cf = Q.cf[u][c];
+                cf[0] = (T)V.bx[id] * (T)V.ih.x;
+                cf[1] = (T)V.bx[id - 1] * (T)V.ih.x;
+                cf[2] = (T)V.by[id] * (T)V.ih.y;
+                cf[3] = (T)V.by[id - L.sx] * (T)V.ih.y;
+                T sc = cf[0] + cf[1] + cf[2] + cf[3];
+                if (DIM == 3) {
+                    cf[4] = (T)V.bz[id] * (T)V.ih.z;
+                    cf[5] = (T)V.bz[id - L.sxy] * (T)V.ih.z;
+                    sc += cf[4] + cf[5];
+                }
+                Q.f[u][c] = V.f[id];
+                Q.rs[u][c] = i < L.nx ? tail_recip(sc) : (T)0;
+                Q.li[u][c] = lbox(L, i, j, k);   // i = nx: the row's ghost, never changed (rs = 0)
             }
         }
     };
-    // one colour of Gauss-Seidel on an LDS-resident level, stencil()'s order
-    auto gs_lds = [&](const TailLevel<T> &V, T *el, const T (&cf)[TAIL_CPT][6], const T (&fv)[TAIL_CPT],
-                      int color) {
-        const Lay &L = V.L;
+    // sum c (e_nb - e_P) of the pair's cell of colour c, stencil()'s order
+    auto cell_sum = [&](const Lay &L, const T *el, const TailCells<T> &Q, int u, int c) {
+        const int li = Q.li[u][c], bsx = L.nx + 2, bsxy = bsx * (L.ny + 2);
+        const T *cf = Q.cf[u][c];
+        const T ep = el[li];
+        T s = cf[0] * (el[li + 1] - ep) + cf[1] * (el[li - 1] - ep) + cf[2] * (el[li + bsx] - ep) +
+              cf[3] * (el[li - bsx] - ep);
+        if (DIM == 3) s += cf[4] * (el[li + bsxy] - ep) + cf[5] * (el[li - bsxy] - ep);
+        return s;
+    };
+    // one colour of Gauss-Seidel on an LDS-resident level
+    auto gs_lds = [&](const Lay &L, T *el, const TailCells<T> &Q, int color) {
 #pragma unroll
-        for (int u = 0; u < TAIL_CPT; ++u) {
-            const int c = t + u * TAIL_THREADS;
-            if (c >= ncells(L)) continue;
-            int i, j, k;
-            cell_coords(L, c, i, j, k);
-            const int kl = DIM == 3 ? k : 0;
-            if (((i + j + kl) & 1) != color) continue;
-            const int li = lbox(L, i, j, kl), bsx = L.nx + 2, bsxy = bsx * (L.ny + 2);
-            const T ep = el[li];
-            const T vE = el[li + 1], vW = el[li - 1], vN = el[li + bsx], vS = el[li - bsx];
-            T sc = cf[u][0] + cf[u][1] + cf[u][2] + cf[u][3];
-            T sce = cf[u][0] * (vE - ep) + cf[u][1] * (vW - ep) + cf[u][2] * (vN - ep) + cf[u][3] * (vS - ep);
-            if (DIM == 3) {
-                sc += cf[u][4] + cf[u][5];
-                sce += cf[u][4] * (el[li + bsxy] - ep) + cf[u][5] * (el[li - bsxy] - ep);
-            }
-            el[li] = sc > (T)0 ? ep + gs_step<T>(sce - fv[u], sc) : ep;
-        }
+        for (int u = 0; u < TAIL_PAIRS; ++u)
+            if (u < Q.np && Q.rs[u][color] != (T)0)
+                el[Q.li[u][color]] += (cell_sum(L, el, Q, u, color) - Q.f[u][color]) * Q.rs[u][color];
         __syncthreads();
     };
     // ---- top level in LDS + registers (FP32 only; A.top is never set for FP64).
@@ -1544,34 +1568,34 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         const TailLevel<T> &C = A.lv[a + 1];
         const Lay &L = F.L;
         T *el = el_ + A.eoff[a];
-        T cf[TAIL_CPT][6], fv[TAIL_CPT];
+        TailCells<T> Q;
         for (int q = t; q < boxn(L); q += TAIL_THREADS) el[q] = (T)0;
+        load_cells(F, Q);
         __syncthreads();
-        load_regs(F, cf, fv);
         const int n = ncells(L);
-        if (a == a0)   // the first level's error as it was left (later ones start at 0)
+        if (a == a0) {   // the first level's error as it was left (later ones start at 0)
             for (int c = t; c < n; c += TAIL_THREADS) {
                 int i, j, k;
                 cell_coords(L, c, i, j, k);
                 el[lbox(L, i, j, DIM == 3 ? k : 0)] = F.e[L.id(i, j, k)];
             }
-        __syncthreads();
-        for (int s = 0; s < F.nu1; ++s) { gs_lds(F, el, cf, fv, 0); gs_lds(F, el, cf, fv, 1); }
-        // residual of each cell by its owner in apply_A's order, then the
-        // coarse sums over the children in k_resid_restrict's order
-#pragma unroll
-        for (int u = 0; u < TAIL_CPT; ++u) {
-            const int c = t + u * TAIL_THREADS;
-            if (c >= n) continue;
-            int i, j, k;
-            cell_coords(L, c, i, j, k);
-            const int li = lbox(L, i, j, DIM == 3 ? k : 0), bsx = L.nx + 2, bsxy = bsx * (L.ny + 2);
-            const T ep = el[li];
-            T acc = cf[u][0] * (el[li + 1] - ep) + cf[u][1] * (el[li - 1] - ep) + cf[u][2] * (el[li + bsx] - ep) +
-                    cf[u][3] * (el[li - bsx] - ep);
-            if (DIM == 3) acc += cf[u][4] * (el[li + bsxy] - ep) + cf[u][5] * (el[li - bsxy] - ep);
-            rt_[c] = fv[u] - acc;
+            __syncthreads();
         }
+        for (int s = 0; s < F.nu1; ++s) { gs_lds(L, el, Q, 0); gs_lds(L, el, Q, 1); }
+        // residual of each cell by its owner in apply_A's order (at the cell's
+        // interior index), then the coarse sums over the children in
+        // k_resid_restrict's order
+#pragma unroll
+        for (int u = 0; u < TAIL_PAIRS; ++u)
+            if (u < Q.np) {
+                const int q = t + u * TAIL_THREADS, mx = (L.nx + 1) / 2, r = q / mx, m = q - r * mx, k = r / L.ny,
+                          j = r - k * L.ny;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const int i = 2 * m + ((j + k + c) & 1);
+                    if (i < L.nx) rt_[i + L.nx * r] = Q.f[u][c] - cell_sum(L, el, Q, u, c);
+                }
+            }
         __syncthreads();
         const int nc = ncells(C.L);
         for (int cc = t; cc < nc; cc += TAIL_THREADS) {
@@ -1633,10 +1657,19 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         const double fm = block_sum(fv) / (double)n;
         if (t < n) bvec[t] = fm - fv;
         __syncthreads();
+        // M^-1 b by all threads: CPARTS column ranges per row, added in order
         double x = 0.0;
         const double *minv = A.minv + (long)kq * n * n;
-        if (t < n)
-            for (int cc = 0; cc < n; ++cc) x += minv[cc * n + t] * bvec[cc];
+        {
+            const int row = t % CDENSE, part = t / CDENSE, per = (n + CPARTS - 1) / CPARTS;
+            double xp = 0.0;
+            if (row < n)
+                for (int cc = part * per; cc < min((part + 1) * per, n); ++cc) xp += minv[cc * n + row] * bvec[cc];
+            dpart[part][row] = xp;
+            __syncthreads();
+            if (t < n)
+                for (int q = 0; q < CPARTS; ++q) x += dpart[q][t];
+        }
         const double xm = block_sum(t < n ? x : 0.0) / (double)n;
         if (t < n) V.e[V.L.id(i, j, k)] = (T)(x - xm);
         if (A.lds) {
@@ -1654,8 +1687,8 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         const Lay &L = F.L;
         T *el = el_ + A.eoff[a];
         const T *elc = el_ + A.eoff[a + 1];
-        T cf[TAIL_CPT][6], fv[TAIL_CPT];
-        load_regs(F, cf, fv);
+        TailCells<T> Q;
+        load_cells(F, Q);
         const int n = ncells(L);
         for (int c = t; c < n; c += TAIL_THREADS) {
             int i, j, k;
@@ -1664,7 +1697,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
             el[lbox(L, i, j, kl)] += elc[lbox(C.L, i / F.cx, j / F.cy, kl / F.cz)];
         }
         __syncthreads();
-        for (int s = 0; s < F.nu2; ++s) { gs_lds(F, el, cf, fv, 1); gs_lds(F, el, cf, fv, 0); }
+        for (int s = 0; s < F.nu2; ++s) { gs_lds(L, el, Q, 1); gs_lds(L, el, Q, 0); }
         for (int c = t; c < n; c += TAIL_THREADS) {
             int i, j, k;
             cell_coords(L, c, i, j, k);
@@ -2167,7 +2200,7 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
                 const Lay &L = A.lv[q].L;
                 A.eoff[q] = off;
                 off += (L.nx + 2) * (L.ny + 2) * (DIM == 3 ? L.nz + 2 : 1);
-                fit = fit && (long)L.nx * L.ny * (DIM == 3 ? L.nz : 1) <= TAIL_MAX;
+                fit = fit && (long)((L.nx + 1) / 2) * L.ny * (DIM == 3 ? L.nz : 1) <= (long)TAIL_PAIRS * TAIL_THREADS;
             }
             A.lds = fit && off <= TAIL_ELDS ? 1 : 0;
         }
