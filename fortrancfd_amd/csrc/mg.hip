@@ -1146,108 +1146,115 @@ __device__ __forceinline__ void cell_coords_g(const Lay &L, int id, int &i, int 
 }
 
 // Gauss-Jordan inversion without pivoting (M is SPD) by one block of
-// CINV_THREADS threads, the matrix held in registers: thread t owns column
-// t % 128 of the rows t / 128 + NRG q.  Per pivot only the pivot row and
-// column go through LDS; the update of the owned elements is register
-// arithmetic.  Writes M^-1 (symmetric) to minv[n*n].
-constexpr int CINV_THREADS = 1024;
+// CINV_THREADS threads, the matrix held in registers: thread t owns the
+// CINV_T x CINV_T tile (t / CINV_G, t % CINV_G).  Per pivot only the pivot row
+// and column go through LDS (double buffered, one barrier); the update of the
+// owned elements is register arithmetic, 2 CINV_T LDS reads for CINV_T^2
+// elements.  (1024 threads with one column and every eighth row each read 17
+// values for 16 elements: 234 us for 128 cells.)  Writes M^-1 (symmetric) to
+// minv[n*n].
+constexpr int CINV_T = 8, CINV_G = CDENSE / CINV_T, CINV_THREADS = CINV_G * CINV_G;
 template <int DIM>
 __global__ void __launch_bounds__(CINV_THREADS) k_coarse_inv(const double *__restrict__ bx,
                                                              const double *__restrict__ by,
                                                              const double *__restrict__ bz, Lay L, Inv2 ih,
                                                              double *__restrict__ minv) {
-    constexpr int NRG = CINV_THREADS / CDENSE;           // row groups
-    constexpr int NQ = CDENSE * CDENSE / CINV_THREADS;   // owned rows per thread
-    constexpr int NW = CINV_THREADS / WAVE;
-    __shared__ double colg[NRG][NQ], row[CDENSE];
-    __shared__ double sh[NW];
+    static_assert(CDENSE <= CINV_THREADS, "one thread per cell forms the diagonal");
+    __shared__ double col[2][CDENSE], row[2][CDENSE];
+    __shared__ double sh[CINV_THREADS / WAVE];
     const int t = threadIdx.x, n = L.nx * L.ny * L.nz;
-    const int cc = t % CDENSE, rg = t / CDENSE;
+    const int r0 = CINV_T * (t / CINV_G), c0 = CINV_T * (t % CINV_G);
     // a batched 2D stack inverts case blockIdx.x's block (L: one slice)
     const int kq = DIM == 2 ? (int)blockIdx.x : 0;
     minv += (long)kq * n * n;
+    // face coefficients E W N S T B and position of cell c
+    auto faces = [&](int c, double (&cf)[6], int &i, int &j, int &k) {
+        cell_coords(L, c, i, j, k);
+        const long id = L.id(i, j, k + kq);
+        cf[0] = bx[id] * ih.x; cf[1] = bx[id - 1] * ih.x; cf[2] = by[id] * ih.y; cf[3] = by[id - L.sx] * ih.y;
+        cf[4] = DIM == 3 ? bz[id] * ih.z : 0.0;
+        cf[5] = DIM == 3 ? bz[id - L.sxy] * ih.z : 0.0;
+    };
     double dsum = 0.0;
     if (t < n) {
+        double cf[6];
         int i, j, k;
-        cell_coords(L, t, i, j, k);
-        k += kq;
-        const long id = L.id(i, j, k);
-        double d = (bx[id] + bx[id - 1]) * ih.x + (by[id] + by[id - L.sx]) * ih.y;
-        if (DIM == 3) d += (bz[id] + bz[id - L.sxy]) * ih.z;
-        dsum = d;
+        faces(t, cf, i, j, k);
+        dsum = ((cf[0] + cf[1]) + (cf[2] + cf[3])) + (cf[4] + cf[5]);
     }
     // fixed-order block sum: wave butterflies, then the waves in order
     for (int o = 32; o > 0; o >>= 1) dsum += __shfl_xor(dsum, o, WAVE);
     if ((t & (WAVE - 1)) == 0) sh[t / WAVE] = dsum;
     __syncthreads();
     double tot = 0.0;
-    for (int w = 0; w < NW; ++w) tot += sh[w];
+    for (int w = 0; w < CINV_THREADS / WAVE; ++w) tot += sh[w];
     const double sigma = tot / ((double)n * (double)n);
     // M = B + sigma 1 1^T.  B is symmetric (the face coefficient between two
-    // cells is one stored value), so column cc is formed from cell cc's own
-    // faces: the diagonal d(cc) and -c(face) for the neighbour rows.
-    double m[NQ];
-    {
-        int i = 0, j = 0, k = 0;
-        double ce_ = 0.0, cw = 0.0, cn = 0.0, cs = 0.0, ct = 0.0, cb = 0.0, d = 0.0;
-        if (cc < n) {
-            cell_coords(L, cc, i, j, k);
-            k += kq;
-            const long id = L.id(i, j, k);
-            ce_ = bx[id] * ih.x; cw = bx[id - 1] * ih.x; cn = by[id] * ih.y; cs = by[id - L.sx] * ih.y;
-            d = ce_ + cw + cn + cs;
-            if (DIM == 3) {
-                ct = bz[id] * ih.z;
-                cb = bz[id - L.sxy] * ih.z;
-                d += ct + cb;
-            }
-        }
-        const int pz = L.nx * L.ny;
+    // cells is one stored value), so a column is formed from its cell's own
+    // faces: the diagonal and -c(face) for the neighbour rows.
+    double m[CINV_T][CINV_T];
+    const int pz = L.nx * L.ny;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int r = rg + NRG * q;
+    for (int b = 0; b < CINV_T; ++b) {
+        const int cc = c0 + b;
+        double cf[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        int i = 0, j = 0, k = 0;
+        if (cc < n) faces(cc, cf, i, j, k);
+        const double d = ((cf[0] + cf[1]) + (cf[2] + cf[3])) + (cf[4] + cf[5]);
+#pragma unroll
+        for (int a = 0; a < CINV_T; ++a) {
+            const int r = r0 + a;
             double v = sigma;
             if (r == cc) v += d;
-            else if (i < L.nx - 1 && r == cc + 1) v -= ce_;
-            else if (i > 0 && r == cc - 1) v -= cw;
-            else if (j < L.ny - 1 && r == cc + L.nx) v -= cn;
-            else if (j > 0 && r == cc - L.nx) v -= cs;
-            else if (DIM == 3 && k < L.nz - 1 && r == cc + pz) v -= ct;
-            else if (DIM == 3 && k > 0 && r == cc - pz) v -= cb;
-            m[q] = v;
+            else if (i < L.nx - 1 && r == cc + 1) v -= cf[0];
+            else if (i > 0 && r == cc - 1) v -= cf[1];
+            else if (j < L.ny - 1 && r == cc + L.nx) v -= cf[2];
+            else if (j > 0 && r == cc - L.nx) v -= cf[3];
+            else if (DIM == 3 && k < L.nz - 1 && r == cc + pz) v -= cf[4];
+            else if (DIM == 3 && k > 0 && r == cc - pz) v -= cf[5];
+            m[a][b] = v;
         }
     }
-    for (int kk = 0; kk < n; ++kk) {
-        // pivot column (owned by the threads of column kk), stored by row
-        // group so that each thread reads its rows as consecutive words
-        if (cc == kk) {
+    for (int K = 0; K * CINV_T < n; ++K) {
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) colg[rg][q] = m[q];
+        for (int p = 0; p < CINV_T; ++p) {
+            const int kk = K * CINV_T + p, h = kk & 1;
+            if (kk >= n) break;   // uniform
+            if (c0 == K * CINV_T) {
+#pragma unroll
+                for (int a = 0; a < CINV_T; ++a) col[h][r0 + a] = m[a][p];
+            }
+            if (r0 == K * CINV_T) {
+#pragma unroll
+                for (int b = 0; b < CINV_T; ++b) row[h][c0 + b] = m[p][b];
+            }
+            __syncthreads();
+            const double ip = 1.0 / col[h][kk];
+            double cv[CINV_T], rv[CINV_T];
+#pragma unroll
+            for (int a = 0; a < CINV_T; ++a) {
+                cv[a] = col[h][r0 + a];
+                rv[a] = row[h][c0 + a] * ip;   // new pivot row
+            }
+#pragma unroll
+            for (int a = 0; a < CINV_T; ++a)
+#pragma unroll
+                for (int b = 0; b < CINV_T; ++b) m[a][b] -= cv[a] * rv[b];
+            if (c0 == K * CINV_T) {   // pivot column: -c / pivot
+#pragma unroll
+                for (int a = 0; a < CINV_T; ++a) m[a][p] = -cv[a] * ip;
+            }
+            if (r0 == K * CINV_T) {   // pivot row, 1 / pivot on the diagonal
+#pragma unroll
+                for (int b = 0; b < CINV_T; ++b) m[p][b] = (c0 + b == kk) ? ip : rv[b];
+            }
         }
-        if (rg == kk % NRG && cc < n) {
-            double v = 0.0;
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) v = q == kk / NRG ? m[q] : v;
-            row[cc] = v;
-        }
-        __syncthreads();
-        const double piv = colg[kk % NRG][kk / NRG];
-        const double nrow = (cc == kk ? 1.0 : row[cc]) / piv;   // new pivot row, this column
-        double cv[NQ];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) cv[q] = colg[rg][q];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int r = rg + NRG * q;
-            m[q] = r == kk ? nrow : (cc == kk ? 0.0 : m[q]) - cv[q] * nrow;
-        }
-        __syncthreads();
     }
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        const int r = rg + NRG * q;
-        if (r < n && cc < n) minv[r * n + cc] = m[q];
-    }
+    for (int a = 0; a < CINV_T; ++a)
+#pragma unroll
+        for (int b = 0; b < CINV_T; ++b)
+            if (r0 + a < n && c0 + b < n) minv[(long)(r0 + a) * n + c0 + b] = m[a][b];
 }
 
 // e = M^-1 b with b = -(f - mean f), then the zero-mean projection of e;
