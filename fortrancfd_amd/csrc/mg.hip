@@ -756,7 +756,7 @@ __global__ void __launch_bounds__(256) k_sum_stage1(const double *__restrict__ p
 // ended while others of the stack go on: its alpha and beta are 0 from then
 // on, so the x += alpha p still pending from its last iteration is the only
 // update it receives, as at the end of a single solve.
-// The stopping state of each case's solve follows (k_cg_start, k_cg_check):
+// The stopping state of each case's solve follows (k_cg_start, SUM_CG_CHECK):
 // ||f||, the relative residual, its best value, iterations, iterations
 // since the best, a non-finite flag, the starting relative residual (the
 // host reads SC_DONE .. SC_R0), and the solve's tolerance and iteration
@@ -767,18 +767,77 @@ enum {
     SC_NAN = 16, SC_R0 = 17, SC_NST = SC_R0 - SC_DONE + 1, SC_TOL = 18, SC_MAXC = 19
 };
 constexpr int SCS = 64;
-enum { SUM_STORE = 0, SUM_CG_BETA = 1, SUM_CG_ALPHA = 2 };
+enum { SUM_STORE = 0, SUM_CG_BETA = 1, SUM_CG_ALPHA = 2, SUM_CG_CHECK = 3 };
 
-// op SUM_CG_BETA: out = {r.z, r.zold} -> beta = (r.z - r.zold) / rz_old
+// mg_skip[0]: every case's solve has ended; mg_skip[1]: how many have
+// (k_cg_start sets both, the SUM_CG_CHECK step of a case that ends counts it)
+struct CgEnd {
+    int *skip;
+    int nq;           // cases
+    double *status;   // pinned host memory: SC_DONE .. SC_R0 of every case
+};
+
+// The scalar step after a sum, by one thread per case (sc: its scalars).
+// SUM_CG_BETA: out = {r.z, r.zold} -> beta = (r.z - r.zold) / rz_old
 // (0 on the first iteration), rz_old = r.z (Polak-Ribiere);
-// op SUM_CG_ALPHA: out = {p.Ap} -> alpha = rz_old / p.Ap.  A is negative
+// SUM_CG_ALPHA: out = {p.Ap} -> alpha = rz_old / p.Ap.  A is negative
 // definite on the zero-mean space and the cycle approximates its inverse, so
 // r.z < 0 and p.Ap < 0 until round-off; otherwise alpha = 0 and the
 // breakdown flag stops the iteration.
+// SUM_CG_CHECK: out = {||r||^2}, the end of an iteration: a case that has not
+// ended counts it, forms its relative residual sqrt(||r||^2) / ||f||, and ends
+// on a breakdown, on r <= tol, after maxc iterations (both as k_cg_start
+// stored them), or when r has not fallen below 0.9 of its best for 4
+// iterations (the FP64 round-off floor); an ended case is frozen (SC_DONE) for
+// the iterations still queued.  A non-finite r ends the case and is flagged.
+// The case's status goes straight to host memory.
+__device__ __forceinline__ void cg_scalar_step(int op, const double *out, double *sc, int q, const CgEnd &E) {
+    const bool done = sc[SC_DONE] != 0.0;
+    if (op == SUM_CG_BETA) {
+        const double rz = out[0], rzo = out[1];
+        sc[SC_BETA] = (sc[SC_FIRST] != 0.0 || done) ? 0.0 : (rz - rzo) / sc[SC_RZ_OLD];
+        sc[SC_RZ_OLD] = rz;
+        sc[SC_FIRST] = 0.0;
+    } else if (op == SUM_CG_ALPHA) {
+        const double pq = out[0], rz = sc[SC_RZ_OLD];
+        const bool ok = pq < 0.0 && rz < 0.0 && !done;
+        sc[SC_ALPHA] = ok ? rz / pq : 0.0;
+        if (!ok && !done) sc[SC_BREAK] = 1.0;
+    } else if (op == SUM_CG_CHECK) {
+        if (!done) {
+            bool end = sc[SC_BREAK] != 0.0;
+            if (!end) {
+                const double k = sc[SC_K] + 1.0, r = sqrt(out[0]) / sc[SC_FN];
+                sc[SC_K] = k;
+                sc[SC_R] = r;
+                if (!isfinite(r)) {
+                    sc[SC_NAN] = 1.0;
+                    end = true;
+                } else {
+                    if (r < 0.9 * sc[SC_BEST]) {
+                        sc[SC_BEST] = r;
+                        sc[SC_SINCE] = 0.0;
+                    } else {
+                        sc[SC_SINCE] += 1.0;
+                        if (sc[SC_SINCE] >= 4.0) end = true;
+                    }
+                    if (!(r > sc[SC_TOL] && k < sc[SC_MAXC])) end = true;
+                }
+            }
+            if (end) {
+                sc[SC_DONE] = 1.0;
+                if (atomicAdd(&E.skip[1], 1) + 1 == E.nq) E.skip[0] = 1;
+            }
+        }
+        for (int m = 0; m < SC_NST; ++m) E.status[(long)q * SC_NST + m] = sc[SC_DONE + m];
+    }
+}
+
 __global__ void __launch_bounds__(256) k_sum_stage2(const double *__restrict__ partial2, int ns,
-                                                    double *__restrict__ out, int op, double *__restrict__ sc,
-                                                    const int *__restrict__ skip) {
-    if (skip && *skip) return;
+                                                    double *out, int op, double *sc, const int *skip, CgEnd E) {
+    // (the check of another case in this launch may just have set the flag:
+    // every case still reports its status)
+    if (skip && *skip && op != SUM_CG_CHECK) return;
     __shared__ double sh[4];
     const int q = blockIdx.x;   // case
     partial2 += (long)q * ns * 256;
@@ -788,18 +847,7 @@ __global__ void __launch_bounds__(256) k_sum_stage2(const double *__restrict__ p
         double a = block_sum256(partial2[s * 256 + threadIdx.x], sh);
         if (threadIdx.x == 0) out[s] = a;
     }
-    const bool done = sc[SC_DONE] != 0.0;
-    if (threadIdx.x == 0 && op == SUM_CG_BETA) {
-        const double rz = out[0], rzo = out[1];
-        sc[SC_BETA] = (sc[SC_FIRST] != 0.0 || done) ? 0.0 : (rz - rzo) / sc[SC_RZ_OLD];
-        sc[SC_RZ_OLD] = rz;
-        sc[SC_FIRST] = 0.0;
-    } else if (threadIdx.x == 0 && op == SUM_CG_ALPHA) {
-        const double pq = out[0], rz = sc[SC_RZ_OLD];
-        const bool ok = pq < 0.0 && rz < 0.0 && !done;
-        sc[SC_ALPHA] = ok ? rz / pq : 0.0;
-        if (!ok && !done) sc[SC_BREAK] = 1.0;
-    }
+    if (threadIdx.x == 0) cg_scalar_step(op, out, sc, q, E);
 }
 
 // The same sums in one launch: a block of SUM1_T threads per case q sums
@@ -808,9 +856,10 @@ __global__ void __launch_bounds__(256) k_sum_stage2(const double *__restrict__ p
 // k_sum_stage2.  Two dependent launches of ~4.4 us become one.
 constexpr int SUM1_T = 1024;
 __global__ void __launch_bounds__(SUM1_T) k_sum_one(const double *__restrict__ partial, long nbq, int ns,
-                                                   double *__restrict__ out, int op, double *__restrict__ sc,
-                                                   const int *__restrict__ skip) {
-    if (skip && *skip) return;
+                                                   double *out, int op, double *sc, const int *skip, CgEnd E) {
+    // (the check of another case in this launch may just have set the flag:
+    // every case still reports its status)
+    if (skip && *skip && op != SUM_CG_CHECK) return;
     __shared__ double sh[SUM1_T / WAVE];
     const int q = blockIdx.x;   // case
     const long ntot = nbq * gridDim.x;
@@ -838,18 +887,7 @@ __global__ void __launch_bounds__(SUM1_T) k_sum_one(const double *__restrict__ p
         }
         __syncthreads();
     }
-    const bool done = sc[SC_DONE] != 0.0;
-    if (threadIdx.x == 0 && op == SUM_CG_BETA) {
-        const double rz = out[0], rzo = out[1];
-        sc[SC_BETA] = (sc[SC_FIRST] != 0.0 || done) ? 0.0 : (rz - rzo) / sc[SC_RZ_OLD];
-        sc[SC_RZ_OLD] = rz;
-        sc[SC_FIRST] = 0.0;
-    } else if (threadIdx.x == 0 && op == SUM_CG_ALPHA) {
-        const double pq = out[0], rz = sc[SC_RZ_OLD];
-        const bool ok = pq < 0.0 && rz < 0.0 && !done;
-        sc[SC_ALPHA] = ok ? rz / pq : 0.0;
-        if (!ok && !done) sc[SC_BREAK] = 1.0;
-    }
+    if (threadIdx.x == 0) cg_scalar_step(op, out, sc, q, E);
 }
 
 // start of a flexible-CG solve: first iteration, no breakdown (case blockIdx.x)
@@ -866,13 +904,19 @@ __global__ void k_cg_init(double *sc) {
 // freeze case q of a batched solve (see SC_DONE)
 __global__ void k_cg_done(double *sc, int q) { sc[(long)q * SCS + SC_DONE] = 1.0; }
 
-// *skip = every case's solve has ended (one block of CG_THREADS threads)
+// skip[0], skip[1] of CgEnd (one block of CG_THREADS threads)
 constexpr int CG_THREADS = 256;
 __device__ __forceinline__ void cg_all_done(const double *sc, int nq, int *skip) {
-    int done = 1;
-    for (int q = threadIdx.x; q < nq; q += CG_THREADS) done &= sc[(long)q * SCS + SC_DONE] != 0.0;
-    const int all = __syncthreads_and(done);
-    if (threadIdx.x == 0) *skip = all ? 1 : 0;
+    __shared__ int n;
+    if (threadIdx.x == 0) n = 0;
+    __syncthreads();
+    for (int q = threadIdx.x; q < nq; q += CG_THREADS)
+        if (sc[(long)q * SCS + SC_DONE] != 0.0) atomicAdd(&n, 1);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        skip[0] = n == nq ? 1 : 0;
+        skip[1] = n;
+    }
 }
 
 // Stopping state of the flexible-CG solve of every case from the initial
@@ -894,45 +938,6 @@ __global__ void __launch_bounds__(CG_THREADS) k_cg_start(double *sc, int nq, dou
         s[SC_SINCE] = 0.0;
         s[SC_NAN] = isfinite(r) ? 0.0 : 1.0;
         if (!(r > tol && 0 < maxc) || !isfinite(r)) s[SC_DONE] = 1.0;
-    }
-    cg_all_done(sc, nq, skip);
-}
-
-// After an iteration: a case that has not ended counts it, forms its
-// relative residual sqrt(||r||^2) / ||f||, and ends on a breakdown, on
-// r <= tol, after maxc iterations (both as k_cg_start stored them), or when r has not fallen below 0.9 of
-// its best for 4 iterations (the FP64 round-off floor); an ended case is
-// frozen (SC_DONE) for the iterations still queued.  A non-finite r ends
-// the case and is flagged.
-__global__ void __launch_bounds__(CG_THREADS) k_cg_check(double *sc, int nq, int *skip) {
-    if (*skip) return;
-    for (int q = threadIdx.x; q < nq; q += CG_THREADS) {
-        double *s = sc + (long)q * SCS;
-        const double tol = s[SC_TOL], maxc = s[SC_MAXC];
-        if (s[SC_DONE] == 0.0) {
-            if (s[SC_BREAK] != 0.0) {
-                s[SC_DONE] = 1.0;
-            } else {
-                const double k = s[SC_K] + 1.0, r = sqrt(s[SC_RR]) / s[SC_FN];
-                s[SC_K] = k;
-                s[SC_R] = r;
-                bool done = false;
-                if (!isfinite(r)) {
-                    s[SC_NAN] = 1.0;
-                    done = true;
-                } else {
-                    if (r < 0.9 * s[SC_BEST]) {
-                        s[SC_BEST] = r;
-                        s[SC_SINCE] = 0.0;
-                    } else {
-                        s[SC_SINCE] += 1.0;
-                        if (s[SC_SINCE] >= 4.0) done = true;
-                    }
-                    if (!(r > tol && k < maxc)) done = true;
-                }
-                if (done) s[SC_DONE] = 1.0;
-            }
-        }
     }
     cg_all_done(sc, nq, skip);
 }
@@ -1881,7 +1886,7 @@ static int mg_build(fcfd_ctx *c) {
         return FCFD_ERR_ARG;
     }
     FCFD_TRY(alloc0(&c->mg_scalars, SCS * c->nb + c->nb * std::max(6 * ncoarse, ncoarse * ncoarse)));
-    FCFD_TRY(alloc0(&c->mg_skip, 1));
+    FCFD_TRY(alloc0(&c->mg_skip, 2));
     for (auto &e : c->cg_ev)
         if (!e) FCFD_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     return FCFD_OK;
@@ -2415,17 +2420,18 @@ __global__ void __launch_bounds__(256) k_fcg_finish(double *__restrict__ x, cons
 // made the step 1 % slower, while the batched 2D stacks, 128-2048 partials
 // per case, ran 7 % faster in one launch).
 constexpr long SUM1_MAX = 16384;
-static int sum_partials(fcfd_ctx *c, long nb, int ns, double *out, int op = SUM_STORE) {
+static int sum_partials(fcfd_ctx *c, long nb, int ns, double *out, int op = SUM_STORE, double *status = nullptr) {
     const long nbq = nb / c->nb;
+    const CgEnd E{c->mg_skip, c->nb, status};
     if (nbq <= SUM1_MAX) {
         hipLaunchKernelGGL(k_sum_one, dim3(c->nb), dim3(SUM1_T), 0, c->stream, c->red.partial, nbq, ns, out, op,
-                           c->mg_scalars, t_skip);
+                           c->mg_scalars, t_skip, E);
     } else {
         const long chunk = (nbq + 255) / 256;
         hipLaunchKernelGGL(k_sum_stage1, dim3(256, ns, c->nb), dim3(256), 0, c->stream, c->red.partial, nbq, chunk,
                            c->red.partial2, t_skip);
         hipLaunchKernelGGL(k_sum_stage2, dim3(c->nb), dim3(256), 0, c->stream, c->red.partial2, ns, out, op,
-                           c->mg_scalars, t_skip);
+                           c->mg_scalars, t_skip, E);
     }
     FCFD_CHECK(hipGetLastError());
     return FCFD_OK;
@@ -2495,8 +2501,8 @@ static int vcycles(fcfd_ctx *c, int kind, int inner) {
 // One flexible-CG iteration, all on the device: z = V-cycle(s)(r) (kind 1:
 // FP64 z, kind 3: FP32 z) with r.z and r.zold folded into the last sweep,
 // beta; p = z + beta p, q = A z + beta q, z_old = z, p.q; alpha; x += alpha p,
-// r -= alpha q, the next cycle's rhs; ||r||^2; the stopping test of every
-// case (k_cg_check); then the stopping state to host buffer `slot`.
+// r -= alpha q, the next cycle's rhs; ||r||^2 with the stopping test of every
+// case, whose status goes to host buffer `slot`.
 template <int DIM>
 static int fcg_iteration(fcfd_ctx *c, int kind, int inner, int slot) {
     const Geom &G = c->G;
@@ -2540,18 +2546,16 @@ static int fcg_iteration(fcfd_ctx *c, int kind, int inner, int slot) {
                            c->red.partial, DIM);
         FCFD_CHECK(hipGetLastError());
     }
-    FCFD_TRY(sum_partials(c, nb, 1, sc + SC_RR, SUM_STORE));
-    hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(CG_THREADS), 0, c->stream, sc, c->nb, c->mg_skip);
-    FCFD_CHECK(hipGetLastError());
-    // SC_DONE .. SC_NAN of every case, packed
-    FCFD_TRY(gather_to_host(c, c->red.host + (long)slot * SC_NST * c->nb, sc + SC_DONE, SCS, SC_NST, c->nb));
-    return FCFD_OK;
+    // the stopping test and the status of every case with the sum: no check
+    // kernel and no copy node (5 us of an iteration that takes about 75 on a
+    // 64 x 128 grid)
+    return sum_partials(c, nb, 1, sc + SC_RR, SUM_CG_CHECK, c->red.host + (long)slot * SC_NST * c->nb);
 }
 
 // The solve runs the loop of a single system for every case of the context
 // at once (one case unless it is a batched 2D stack).  Each case keeps its
 // own stopping state (on the device for flexible CG: k_cg_start,
-// k_cg_check); once a case's loop would have ended it is frozen on the
+// SUM_CG_CHECK); once a case's loop would have ended it is frozen on the
 // device (SC_DONE; the mixed defect correction skips its update), so its
 // result is that of its own solve.  FP64 plain V-cycles cannot freeze a case
 // and go on improving finished ones until the last case stops.
@@ -2643,7 +2647,7 @@ static int ppe_solve_t(fcfd_ctx *c, double rel_tol, int precision, int *cycles, 
     int it = 0;
     if (krylov && active > 0) {
         // Flexible CG, one graph per iteration, pipelined: while the host
-        // reads iteration it's stopping state (k_cg_check), iteration it + 1
+        // reads iteration it's stopping state (SUM_CG_CHECK), iteration it + 1
         // is already queued, so the device does not wait on the host between
         // iterations.  An iteration queued after the solve has ended finds
         // the skip flag set and all its kernels return at once, but its
