@@ -102,6 +102,7 @@ struct MgLevel {
     int nx, ny, nz;          // cells
     int cx, cy, cz;          // coarsening factor (1|2) to the next level
     double hx, hy, hz;       // spacing
+    double wx = 1, wy = 1, wz = 1;   // width of each axis' last cell / spacing (odd axes: see mg.hip)
     long sx, sxy, ntot;      // layout with one ghost layer (finest uses Geom)
     // FP64 arrays (level >= 1): solution/error, rhs, residual, face coeffs
     double *e64, *f64, *r64, *bx64, *by64, *bz64;

@@ -105,8 +105,27 @@ static Split split_of(const Geom &G) {
     return S;
 }
 
+// 1/h^2 per axis, and what an axis paired from an odd number of cells
+// changes at its far end.  The last aggregate of such an axis has one child:
+// it is w = 1/2 of a cell wide (on coarser levels 1/4 .. 1), and its flux
+// balance per cell volume is that of the full-width one divided by w.  So in
+// its own row the inner face (the only open one of that axis) has the
+// coefficient / w (xl = x / w), its volume is w, and restriction weighs it by
+// that.  The coarse operator times the cell volumes is then symmetric and the
+// piecewise-constant aggregates' Galerkin operator up to the usual factor 2;
+// without it the last cell's correction was twice what it should be, and
+// 75 x 90 x 131 cells took 57 cycles for a first step that 80 x 96 x 128 does
+// in 23.
 struct Inv2 {
-    double x, y, z;  // 1/h^2 per axis
+    double x, y, z, xl, yl, zl;
+    float wx, wy, wz;
+    template <typename T>
+    __device__ __forceinline__ T weight(const Lay &L, int i, int j, int k, int dim) const {
+        T w = i == L.nx - 1 ? (T)wx : (T)1;
+        w *= j == L.ny - 1 ? (T)wy : (T)1;
+        if (dim == 3) w *= k == L.nz - 1 ? (T)wz : (T)1;
+        return w;
+    }
 };
 
 // face coefficient of level 0 between cells with densities a and b.  The
@@ -197,12 +216,12 @@ __device__ __forceinline__ void stencil(const T *__restrict__ e, const T *__rest
         }
     } else {
         ce_ = (T)bx[id] * (T)ih.x;
-        cw = (T)bx[id - 1] * (T)ih.x;
+        cw = (T)bx[id - 1] * (T)(i == L.nx - 1 ? ih.xl : ih.x);
         cn = (T)by[id] * (T)ih.y;
-        cs = (T)by[id - L.sx] * (T)ih.y;
+        cs = (T)by[id - L.sx] * (T)(j == L.ny - 1 ? ih.yl : ih.y);
         if (DIM == 3) {
             ct = (T)bz[id] * (T)ih.z;
-            cb = (T)bz[id - L.sxy] * (T)ih.z;
+            cb = (T)bz[id - L.sxy] * (T)(k == L.nz - 1 ? ih.zl : ih.z);
         }
     }
     sum_c = ce_ + cw + cn + cs;
@@ -234,10 +253,13 @@ __device__ __forceinline__ T apply_A(const T *__restrict__ e, const T *__restric
             acc += face<T>(k > 0, r, rho[id - L.sxy], (T)ih.z) * (e[id - L.sxy] - ep);
         }
     } else {
-        acc = (T)bx[id] * (T)ih.x * (e[id + 1] - ep) + (T)bx[id - 1] * (T)ih.x * (e[id - 1] - ep) +
-              (T)by[id] * (T)ih.y * (e[id + L.sx] - ep) + (T)by[id - L.sx] * (T)ih.y * (e[id - L.sx] - ep);
+        acc = (T)bx[id] * (T)ih.x * (e[id + 1] - ep) +
+              (T)bx[id - 1] * (T)(i == L.nx - 1 ? ih.xl : ih.x) * (e[id - 1] - ep) +
+              (T)by[id] * (T)ih.y * (e[id + L.sx] - ep) +
+              (T)by[id - L.sx] * (T)(j == L.ny - 1 ? ih.yl : ih.y) * (e[id - L.sx] - ep);
         if (DIM == 3)
-            acc += (T)bz[id] * (T)ih.z * (e[id + L.sxy] - ep) + (T)bz[id - L.sxy] * (T)ih.z * (e[id - L.sxy] - ep);
+            acc += (T)bz[id] * (T)ih.z * (e[id + L.sxy] - ep) +
+                   (T)bz[id - L.sxy] * (T)(k == L.nz - 1 ? ih.zl : ih.z) * (e[id - L.sxy] - ep);
     }
     return acc;
 }
@@ -526,6 +548,7 @@ __global__ void __launch_bounds__(FUSED_THREADS) k_smooth_fused(const float *__r
     const int t = threadIdx.x;
     const int i0 = bx_ * TX - H, j0 = by_ * TY - H, k0 = DIM == 3 ? bz_ * TZ - H : bz_;   // 2D: the slice
     const float hx = (float)ih.x, hy = (float)ih.y, hz = (float)ih.z;
+    const float hxl = (float)ih.xl, hyl = (float)ih.yl, hzl = (float)ih.zl;
     // staging: every load of the block's NIT rounds is issued before the
     // first is waited for (a loop with a branch around its loads costs one
     // memory latency per round); positions outside the ghosted array load a
@@ -580,11 +603,12 @@ __global__ void __launch_bounds__(FUSED_THREADS) k_smooth_fused(const float *__r
                 continue;
             const int c = lx + ly * SY + lz * SZ;
             const float ep = se[c];
-            const float ce_ = sbx[c] * hx, cw = sbx[c - 1] * hx, cn = sby[c] * hy, cs = sby[c - SY] * hy;
+            const float ce_ = sbx[c] * hx, cw = sbx[c - 1] * (i == L.nx - 1 ? hxl : hx), cn = sby[c] * hy,
+                        cs = sby[c - SY] * (j == L.ny - 1 ? hyl : hy);
             float sc = ce_ + cw + cn + cs;
             float sce = ce_ * (se[c + 1] - ep) + cw * (se[c - 1] - ep) + cn * (se[c + SY] - ep) + cs * (se[c - SY] - ep);
             if (DIM == 3) {
-                const float ct = sbz[c] * hz, cb = sbz[c - SZ] * hz;
+                const float ct = sbz[c] * hz, cb = sbz[c - SZ] * (k == L.nz - 1 ? hzl : hz);
                 sc += ct + cb;
                 sce += ct * (se[c + SZ] - ep) + cb * (se[c - SZ] - ep);
             }
@@ -617,8 +641,7 @@ __global__ void __launch_bounds__(256) k_resid_restrict(const T *__restrict__ e,
     const int I = bx_ * blockDim.x + threadIdx.x, J = by_ * blockDim.y + threadIdx.y, K = bz_;
     if (I >= C.nx || J >= C.ny) return;
     if (C2) { cx = 2; cy = 2; cz = C2; }
-    T acc = 0;
-    int nch = 0;
+    T acc = 0, wsum = 0;
 #pragma unroll
     for (int kk = 0; kk < (C2 ? C2 : cz); ++kk)
 #pragma unroll
@@ -629,11 +652,13 @@ __global__ void __launch_bounds__(256) k_resid_restrict(const T *__restrict__ e,
                 // the last aggregate of an odd axis has one child
                 if (i >= L.nx || j >= L.ny || (DIM == 3 && k >= L.nz)) continue;
                 long id = L.id(i, j, k);
-                acc += f[id] - apply_A<T, DIM, FINE, CT>(e, rho, bx, by, bz, L, ih, i, j, k, id);
-                ++nch;
+                const T r = f[id] - apply_A<T, DIM, FINE, CT>(e, rho, bx, by, bz, L, ih, i, j, k, id);
+                const T w = FINE ? (T)1 : ih.template weight<T>(L, i, j, k, DIM);
+                acc += w * r;
+                wsum += w;
             }
     const long cid = C.id(I, J, K);
-    fc[cid] = acc / (T)nch;
+    fc[cid] = acc / wsum;
     ec[cid] = (T)0;
 }
 
@@ -658,18 +683,19 @@ template <int DIM, bool FINE>
 __global__ void k_coef_restrict(const double *__restrict__ rho, const double *__restrict__ bxf,
                                 const double *__restrict__ byf, const double *__restrict__ bzf, Lay L,
                                 double *__restrict__ bxc, double *__restrict__ byc, double *__restrict__ bzc, Lay C,
-                                int cx, int cy, int cz) {
+                                int cx, int cy, int cz, Inv2 ih) {
     const int I = blockIdx.x * blockDim.x + threadIdx.x, J = blockIdx.y * blockDim.y + threadIdx.y, K = blockIdx.z;
     if (I >= C.nx || J >= C.ny) return;
     const long cid = C.id(I, J, K);
     // the last aggregate of an odd axis has one child: fine indices past the
-    // level are not children, and each mean runs over the faces that exist
-    // (the +x face of the last coarse cell is the wall either way)
+    // level are not children, and each mean runs over the faces that exist,
+    // by area (the +x face of the last coarse cell is the wall either way)
+    const double wx = ih.wx, wy = ih.wy, wz = ih.wz;
     const int nz_f = DIM == 3 ? L.nz : 1 << 30;
     // x faces at fine i = I*cx + cx - 1
     {
         double s = 0.0;
-        int m = 0;
+        double m = 0.0;
         int i = I * cx + cx - 1;
         for (int kk = 0; kk < cz; ++kk)
             for (int jj = 0; jj < cy; ++jj) {
@@ -679,14 +705,15 @@ __global__ void k_coef_restrict(const double *__restrict__ rho, const double *__
                 double b;
                 if (FINE) b = i < L.nx - 1 ? 2.0 / (rho[id] + rho[id + 1]) : 0.0;
                 else b = bxf[id];
-                s += b;
-                ++m;
+                const double a = (j == L.ny - 1 ? wy : 1.0) * (DIM == 3 && k == L.nz - 1 ? wz : 1.0);
+                s += a * b;
+                m += a;
             }
         bxc[cid] = I < C.nx - 1 ? s / m : 0.0;
     }
     {
         double s = 0.0;
-        int m = 0;
+        double m = 0.0;
         int j = J * cy + cy - 1;
         for (int kk = 0; kk < cz; ++kk)
             for (int ii = 0; ii < cx; ++ii) {
@@ -696,14 +723,15 @@ __global__ void k_coef_restrict(const double *__restrict__ rho, const double *__
                 double b;
                 if (FINE) b = j < L.ny - 1 ? 2.0 / (rho[id] + rho[id + L.sx]) : 0.0;
                 else b = byf[id];
-                s += b;
-                ++m;
+                const double a = (i == L.nx - 1 ? wx : 1.0) * (DIM == 3 && k == L.nz - 1 ? wz : 1.0);
+                s += a * b;
+                m += a;
             }
         byc[cid] = J < C.ny - 1 ? s / m : 0.0;
     }
     if (DIM == 3) {
         double s = 0.0;
-        int m = 0;
+        double m = 0.0;
         int k = K * cz + cz - 1;
         for (int jj = 0; jj < cy; ++jj)
             for (int ii = 0; ii < cx; ++ii) {
@@ -713,8 +741,9 @@ __global__ void k_coef_restrict(const double *__restrict__ rho, const double *__
                 double b;
                 if (FINE) b = k < L.nz - 1 ? 2.0 / (rho[id] + rho[id + L.sxy]) : 0.0;
                 else b = bzf[id];
-                s += b;
-                ++m;
+                const double a = (i == L.nx - 1 ? wx : 1.0) * (j == L.ny - 1 ? wy : 1.0);
+                s += a * b;
+                m += a;
             }
         bzc[cid] = K < C.nz - 1 ? s / m : 0.0;
     }
@@ -1037,12 +1066,15 @@ __global__ void __launch_bounds__(1024) k_coarse_cg(T *__restrict__ eout, const 
         j = (int)(rr % L.ny);
         k = (int)(rr / L.ny) + kq;
     };
-    // Apply -A (positive semi-definite) to v at cell c
+    // Apply -A times the cell volumes (symmetric positive semi-definite) to v
+    // at cell c; wv: the volume of cell (i, j, k)
+    auto wv = [&](int i, int j, int k) { return ih.template weight<double>(L, i, j, k, DIM); };
     auto negA = [&](const double *v, long c) -> double {
         int i, j, k;
         coords(c, i, j, k);
         long id = L.id(i, j, k);
-        double ce_ = bx[id] * ih.x, cw = bx[id - 1] * ih.x, cn = by[id] * ih.y, cs = by[id - L.sx] * ih.y;
+        double ce_ = bx[id] * ih.x, cw = bx[id - 1] * (i == L.nx - 1 ? ih.xl : ih.x), cn = by[id] * ih.y,
+               cs = by[id - L.sx] * (j == L.ny - 1 ? ih.yl : ih.y);
         double sc = ce_ + cw + cn + cs;
         double acc = sc * v[c];
         if (i < L.nx - 1) acc -= ce_ * v[c + 1];
@@ -1050,21 +1082,21 @@ __global__ void __launch_bounds__(1024) k_coarse_cg(T *__restrict__ eout, const 
         if (j < L.ny - 1) acc -= cn * v[c + L.nx];
         if (j > 0) acc -= cs * v[c - L.nx];
         if (DIM == 3) {
-            double ct = bz[id] * ih.z, cb = bz[id - L.sxy] * ih.z;
+            double ct = bz[id] * ih.z, cb = bz[id - L.sxy] * (k == L.nz - 1 ? ih.zl : ih.z);
             long pz = (long)L.nx * L.ny;
             if (k < L.nz - 1) acc -= ct * v[c + pz];
             if (k > 0) acc -= cb * v[c - pz];
             sc += ct + cb;
             acc += (ct + cb) * v[c];
         }
-        return acc;
+        return wv(i, j, k) * acc;
     };
     // rhs mean
     double s = 0.0;
     for (long c = t; c < n; c += nt) {
         int i, j, k;
         coords(c, i, j, k);
-        s += (double)fin[L.id(i, j, k)];
+        s += wv(i, j, k) * (double)fin[L.id(i, j, k)];
     }
     const double mean = block_sum(s) / (double)n;
     double bb = 0.0;
@@ -1072,11 +1104,13 @@ __global__ void __launch_bounds__(1024) k_coarse_cg(T *__restrict__ eout, const 
         int i, j, k;
         coords(c, i, j, k);
         long id = L.id(i, j, k);
-        double b = -((double)fin[id] - mean);   // solve -A x = -f
+        double b = -(wv(i, j, k) * (double)fin[id] - mean);   // solve -A x = -f times the volumes
         x[c] = 0.0;
         r[c] = b;
-        double d = bx[id] * ih.x + bx[id - 1] * ih.x + by[id] * ih.y + by[id - L.sx] * ih.y;
-        if (DIM == 3) d += bz[id] * ih.z + bz[id - L.sxy] * ih.z;
+        double d = bx[id] * ih.x + bx[id - 1] * (i == L.nx - 1 ? ih.xl : ih.x) + by[id] * ih.y +
+                   by[id - L.sx] * (j == L.ny - 1 ? ih.yl : ih.y);
+        if (DIM == 3) d += bz[id] * ih.z + bz[id - L.sxy] * (k == L.nz - 1 ? ih.zl : ih.z);
+        d *= wv(i, j, k);
         dg[c] = d > 0.0 ? 1.0 / d : 0.0;
         bb += b * b;
     }
@@ -1126,7 +1160,8 @@ __global__ void __launch_bounds__(1024) k_coarse_cg(T *__restrict__ eout, const 
 }
 
 // Coarsest levels of at most CDENSE cells are solved exactly with a dense
-// inverse built once per coefficient setup.  The matrix is B = -A (symmetric,
+// inverse built once per coefficient setup.  The matrix is B = -A times the
+// cell volumes (1 but for the last cells of odd axes; symmetric,
 // positive semi-definite, null space = constants) shifted to
 // M = B + sigma 1 1^T, which is positive definite; for a zero-mean rhs b the
 // solution of M x = b has zero mean and solves B x = b.  sigma = mean(diag B)/n
@@ -1172,13 +1207,17 @@ __global__ void __launch_bounds__(CINV_THREADS) k_coarse_inv(const double *__res
     // a batched 2D stack inverts case blockIdx.x's block (L: one slice)
     const int kq = DIM == 2 ? (int)blockIdx.x : 0;
     minv += (long)kq * n * n;
-    // face coefficients E W N S T B and position of cell c
+    // face coefficients E W N S T B times its volume, and position of cell c
     auto faces = [&](int c, double (&cf)[6], int &i, int &j, int &k) {
         cell_coords(L, c, i, j, k);
         const long id = L.id(i, j, k + kq);
-        cf[0] = bx[id] * ih.x; cf[1] = bx[id - 1] * ih.x; cf[2] = by[id] * ih.y; cf[3] = by[id - L.sx] * ih.y;
-        cf[4] = DIM == 3 ? bz[id] * ih.z : 0.0;
-        cf[5] = DIM == 3 ? bz[id - L.sxy] * ih.z : 0.0;
+        const double w = ih.template weight<double>(L, i, j, k, DIM);
+        cf[0] = w * bx[id] * ih.x;
+        cf[1] = w * bx[id - 1] * (i == L.nx - 1 ? ih.xl : ih.x);
+        cf[2] = w * by[id] * ih.y;
+        cf[3] = w * by[id - L.sx] * (j == L.ny - 1 ? ih.yl : ih.y);
+        cf[4] = DIM == 3 ? w * bz[id] * ih.z : 0.0;
+        cf[5] = DIM == 3 ? w * bz[id - L.sxy] * (k == L.nz - 1 ? ih.zl : ih.z) : 0.0;
     };
     double dsum = 0.0;
     if (t < n) {
@@ -1194,8 +1233,8 @@ __global__ void __launch_bounds__(CINV_THREADS) k_coarse_inv(const double *__res
     double tot = 0.0;
     for (int w = 0; w < CINV_THREADS / WAVE; ++w) tot += sh[w];
     const double sigma = tot / ((double)n * (double)n);
-    // M = B + sigma 1 1^T.  B is symmetric (the face coefficient between two
-    // cells is one stored value), so a column is formed from its cell's own
+    // M = B + sigma 1 1^T.  B, times the cell volumes, is symmetric (the face
+    // coefficient between two cells is one stored value), so a column is formed from its cell's own
     // faces: the diagonal and -c(face) for the neighbour rows.
     double m[CINV_T][CINV_T];
     const int pz = L.nx * L.ny;
@@ -1262,11 +1301,11 @@ __global__ void __launch_bounds__(CINV_THREADS) k_coarse_inv(const double *__res
             if (r0 + a < n && c0 + b < n) minv[(long)(r0 + a) * n + c0 + b] = m[a][b];
 }
 
-// e = M^-1 b with b = -(f - mean f), then the zero-mean projection of e;
+// e = M^-1 b with b = -(f - mean f), f times the cell volumes, then the zero-mean projection of e;
 // one block of CDENSE threads, one cell per thread
 template <typename T>
 __global__ void __launch_bounds__(CDENSE) k_coarse_dense(T *__restrict__ eout, const T *__restrict__ fin,
-                                                         const double *__restrict__ minv, Lay L, int dim) {
+                                                         const double *__restrict__ minv, Lay L, Inv2 ih, int dim) {
     if (L.skipped()) return;
     constexpr int NW = CDENSE / WAVE;
     __shared__ double b[CDENSE];
@@ -1278,8 +1317,8 @@ __global__ void __launch_bounds__(CDENSE) k_coarse_dense(T *__restrict__ eout, c
     double f = 0.0;
     if (t < n) {
         cell_coords(L, t, i, j, k);
+        f = ih.template weight<double>(L, i, j, k, dim) * (double)fin[L.id(i, j, k + kq)];
         k += kq;
-        f = (double)fin[L.id(i, j, k)];
     }
     // fixed-order block sum: butterfly per wave (lane 0's order), then waves in order
     auto block_sum = [&](double v) {
@@ -1431,13 +1470,13 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
                 const long id = L.id(min(i, L.nx - 1), j, k + kq);
                 T *cf = Q.cf[u][c];
                 cf[0] = (T)V.bx[id] * (T)V.ih.x;
-                cf[1] = (T)V.bx[id - 1] * (T)V.ih.x;
+                cf[1] = (T)V.bx[id - 1] * (T)(i >= L.nx - 1 ? V.ih.xl : V.ih.x);
                 cf[2] = (T)V.by[id] * (T)V.ih.y;
-                cf[3] = (T)V.by[id - L.sx] * (T)V.ih.y;
+                cf[3] = (T)V.by[id - L.sx] * (T)(j == L.ny - 1 ? V.ih.yl : V.ih.y);
                 T sc = cf[0] + cf[1] + cf[2] + cf[3];
                 if (DIM == 3) {
                     cf[4] = (T)V.bz[id] * (T)V.ih.z;
-                    cf[5] = (T)V.bz[id - L.sxy] * (T)V.ih.z;
+                    cf[5] = (T)V.bz[id - L.sxy] * (T)(k == L.nz - 1 ? V.ih.zl : V.ih.z);
                     sc += cf[4] + cf[5];
                 }
                 Q.f[u][c] = V.f[id];
@@ -1505,12 +1544,19 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         }
         __syncthreads();
     };
-    // global (ghosted) index of slot sl's cell
-    auto top_gid = [&](const TailLevel<T> &F, const TailLevel<T> &C, int sl) -> long {
+    // slot sl's cell (2D: k is the case) and its global (ghosted) index
+    auto top_cell = [&](const TailLevel<T> &C, int sl, int &i, int &j, int &k) {
         const int ch = sl % NCH;
         int I, J, K;
         cell_coords(C.L, t + TAIL_THREADS * (sl / NCH), I, J, K);
-        return F.L.id(2 * I + (ch & 1), 2 * J + ((ch >> 1) & 1), DIM == 3 ? 2 * K + (ch >> 2) : K);
+        i = 2 * I + (ch & 1);
+        j = 2 * J + ((ch >> 1) & 1);
+        k = DIM == 3 ? 2 * K + (ch >> 2) : K;
+    };
+    auto top_gid = [&](const TailLevel<T> &F, const TailLevel<T> &C, int sl) -> long {
+        int i, j, k;
+        top_cell(C, sl, i, j, k);
+        return F.L.id(i, j, k);
     };
     if constexpr (sizeof(T) == 4) {
         __shared__ float es_[TAIL_LDS], fs_[TAIL_TOP];
@@ -1530,12 +1576,14 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
             for (int sl = 0; sl < TAIL_SLOTS; ++sl) {
                 if (t + TAIL_THREADS * (sl / NCH) < nct) {
                     const long id = top_gid(F, C, sl);
+                    int i, j, k;
+                    top_cell(C, sl, i, j, k);
                     tc[sl][0] = F.bx[id] * (float)F.ih.x;
-                    tc[sl][1] = F.bx[id - 1] * (float)F.ih.x;
+                    tc[sl][1] = F.bx[id - 1] * (float)(i == L.nx - 1 ? F.ih.xl : F.ih.x);
                     tc[sl][2] = F.by[id] * (float)F.ih.y;
-                    tc[sl][3] = F.by[id - L.sx] * (float)F.ih.y;
+                    tc[sl][3] = F.by[id - L.sx] * (float)(j == L.ny - 1 ? F.ih.yl : F.ih.y);
                     tc[sl][4] = DIM == 3 ? F.bz[id] * (float)F.ih.z : 0.f;
-                    tc[sl][5] = DIM == 3 ? F.bz[id - L.sxy] * (float)F.ih.z : 0.f;
+                    tc[sl][5] = DIM == 3 ? F.bz[id - L.sxy] * (float)(k == L.nz - 1 ? F.ih.zl : F.ih.z) : 0.f;
                     fs[sl * TAIL_THREADS + t] = F.f[id];
                 } else {
                     for (int q = 0; q < 6; ++q) tc[sl][q] = 0.f;
@@ -1549,7 +1597,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
             for (int g = 0; g < NG; ++g) {
                 const int cc = t + TAIL_THREADS * g;
                 if (cc >= nct) continue;
-                float acc = 0.f;
+                float acc = 0.f, wsum = 0.f;
 #pragma unroll
                 for (int ch = 0; ch < NCH; ++ch) {
                     const int sl = g * NCH + ch, ii = ch & 1, jj = (ch >> 1) & 1, kk = ch >> 2;
@@ -1563,12 +1611,16 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
                         const int ozp = kk ? plane - 4 * stride : 4 * stride, ozm = kk ? -4 * stride : 4 * stride - plane;
                         ae += tc[sl][4] * (es[li + ozp] - ep) + tc[sl][5] * (es[li + ozm] - ep);
                     }
-                    acc += fs[sl * TAIL_THREADS + t] - ae;
+                    int i, j, k;
+                    top_cell(C, sl, i, j, k);
+                    const float w = F.ih.template weight<float>(L, i, j, k, DIM);
+                    acc += w * (fs[sl * TAIL_THREADS + t] - ae);
+                    wsum += w;
                 }
                 int I, J, K;
                 cell_coords(C.L, cc, I, J, K);
                 const long cid = C.L.id(I, J, K);
-                C.f[cid] = acc / (float)NCH;
+                C.f[cid] = acc / wsum;
                 C.e[cid] = 0.f;
             }
             __syncthreads();
@@ -1605,7 +1657,9 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
                     const int i = 2 * m + ((j + k + c) & 1);
-                    if (i < L.nx) rt_[i + L.nx * r] = Q.f[u][c] - cell_sum(L, el, Q, u, c);
+                    if (i < L.nx)
+                        rt_[i + L.nx * r] =
+                            F.ih.template weight<T>(L, i, j, k, DIM) * (Q.f[u][c] - cell_sum(L, el, Q, u, c));
                 }
             }
         __syncthreads();
@@ -1614,18 +1668,17 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
             int I, J, K;
             cell_coords(C.L, cc, I, J, K);
             const int KL = DIM == 3 ? K : 0;
-            T acc = 0;
-            int nch = 0;
+            T acc = 0, wsum = 0;
             for (int kk = 0; kk < F.cz; ++kk)
                 for (int jj = 0; jj < F.cy; ++jj)
                     for (int ii = 0; ii < F.cx; ++ii) {
                         const int i = I * F.cx + ii, j = J * F.cy + jj, k = KL * F.cz + kk;
                         if (i >= L.nx || j >= L.ny || (DIM == 3 && k >= L.nz)) continue;
                         acc += rt_[i + L.nx * (j + L.ny * k)];
-                        ++nch;
+                        wsum += F.ih.template weight<T>(L, i, j, k, DIM);
                     }
             const long cid = C.L.id(I, J, K);
-            C.f[cid] = acc / (T)nch;
+            C.f[cid] = acc / wsum;
             C.e[cid] = (T)0;
         }
         __syncthreads();
@@ -1638,8 +1691,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         for (int cc = t; cc < nc; cc += TAIL_THREADS) {
             int I, J, K;
             cell_coords(C.L, cc, I, J, K);
-            T acc = 0;
-            int nch = 0;
+            T acc = 0, wsum = 0;
             for (int kk = 0; kk < F.cz; ++kk)
                 for (int jj = 0; jj < F.cy; ++jj)
                     for (int ii = 0; ii < F.cx; ++ii) {
@@ -1647,11 +1699,13 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
                         // the last aggregate of an odd axis has one child (2D: k is the case)
                         if (i >= F.L.nx || j >= F.L.ny || (DIM == 3 && k >= F.L.nz)) continue;
                         const long id = F.L.id(i, j, k);
-                        acc += F.f[id] - apply_A<T, DIM, false, T>(F.e, nullptr, F.bx, F.by, F.bz, F.L, F.ih, i, j, k, id);
-                        ++nch;
+                        const T w = F.ih.template weight<T>(F.L, i, j, k, DIM);
+                        acc += w * (F.f[id] -
+                                    apply_A<T, DIM, false, T>(F.e, nullptr, F.bx, F.by, F.bz, F.L, F.ih, i, j, k, id));
+                        wsum += w;
                     }
             const long cid = C.L.id(I, J, K);
-            C.f[cid] = acc / (T)nch;
+            C.f[cid] = acc / wsum;
             C.e[cid] = (T)0;
         }
         __syncthreads();
@@ -1664,7 +1718,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         double fv = 0.0;
         if (t < n) {
             cell_coords(V.L, t, i, j, k);
-            fv = (double)V.f[V.L.id(i, j, k)];
+            fv = V.ih.template weight<double>(V.L, i, j, k, DIM) * (double)V.f[V.L.id(i, j, k)];
         }
         const double fm = block_sum(fv) / (double)n;
         if (t < n) bvec[t] = fm - fv;
@@ -1758,13 +1812,21 @@ static dim3 grd3(int nx, int ny, int nz, dim3 blk) {
     return dim3((nx + blk.x - 1) / blk.x, (ny + blk.y - 1) / blk.y, nz);
 }
 
-static Inv2 inv2(double hx, double hy, double hz) {
+static Inv2 inv2(double hx, double hy, double hz, double wx = 1.0, double wy = 1.0, double wz = 1.0) {
     Inv2 r;
     r.x = 1.0 / (hx * hx);
     r.y = 1.0 / (hy * hy);
     r.z = 1.0 / (hz * hz);
+    r.xl = r.x / wx;
+    r.yl = r.y / wy;
+    r.zl = r.z / wz;
+    r.wx = (float)wx;   // dyadic: exact
+    r.wy = (float)wy;
+    r.wz = (float)wz;
     return r;
 }
+
+static Inv2 inv2(const MgLevel &M) { return inv2(M.hx, M.hy, M.hz, M.wx, M.wy, M.wz); }
 
 int mg_free(fcfd_ctx *c) {
     for (auto &M : c->mg) {
@@ -1846,6 +1908,11 @@ static int mg_build(fcfd_ctx *c) {
         C.nx = (F.nx + cf[0] - 1) / cf[0]; C.ny = (F.ny + cf[1] - 1) / cf[1];
         C.nz = G.dim == 3 ? (F.nz + cf[2] - 1) / cf[2] : F.nz;   // 2D: the cases
         C.hx = F.hx * cf[0]; C.hy = F.hy * cf[1]; C.hz = F.hz * cf[2];
+        // width of the last aggregate: one child on an odd axis
+        auto width = [](int n, int f, double w) { return f == 1 ? w : (n % 2 ? 0.5 * w : 0.5 * (1.0 + w)); };
+        C.wx = width(F.nx, cf[0], F.wx);
+        C.wy = width(F.ny, cf[1], F.wy);
+        C.wz = G.dim == 3 ? width(F.nz, cf[2], F.wz) : 1.0;
         C.sx = C.nx + 2;
         C.sxy = C.sx * (C.ny + 2);
         C.ntot = C.sxy * (C.nz + (G.dim == 3 ? 2 : 0));
@@ -1907,17 +1974,17 @@ int mg_setup(fcfd_ctx *c) {
         if (l == 1) {
             if (G.dim == 3)
                 hipLaunchKernelGGL((k_coef_restrict<3, true>), g, blk, 0, c->stream, c->f[FCFD_RHO], nullptr, nullptr,
-                                   nullptr, LF, C.bx64, C.by64, C.bz64, LC, F.cx, F.cy, F.cz);
+                                   nullptr, LF, C.bx64, C.by64, C.bz64, LC, F.cx, F.cy, F.cz, inv2(F));
             else
                 hipLaunchKernelGGL((k_coef_restrict<2, true>), g, blk, 0, c->stream, c->f[FCFD_RHO], nullptr, nullptr,
-                                   nullptr, LF, C.bx64, C.by64, nullptr, LC, F.cx, F.cy, 1);
+                                   nullptr, LF, C.bx64, C.by64, nullptr, LC, F.cx, F.cy, 1, inv2(F));
         } else {
             if (G.dim == 3)
                 hipLaunchKernelGGL((k_coef_restrict<3, false>), g, blk, 0, c->stream, nullptr, F.bx64, F.by64, F.bz64,
-                                   LF, C.bx64, C.by64, C.bz64, LC, F.cx, F.cy, F.cz);
+                                   LF, C.bx64, C.by64, C.bz64, LC, F.cx, F.cy, F.cz, inv2(F));
             else
                 hipLaunchKernelGGL((k_coef_restrict<2, false>), g, blk, 0, c->stream, nullptr, F.bx64, F.by64,
-                                   nullptr, LF, C.bx64, C.by64, nullptr, LC, F.cx, F.cy, 1);
+                                   nullptr, LF, C.bx64, C.by64, nullptr, LC, F.cx, F.cy, 1, inv2(F));
         }
         FCFD_CHECK(hipGetLastError());
         long n = C.ntot;
@@ -1939,7 +2006,7 @@ int mg_setup(fcfd_ctx *c) {
         const long n = case_cells(M, G.dim);
         if (c->mg.size() > 1 && n <= CDENSE) {
             Lay L = lay_case(M, G.dim);
-            Inv2 ih = inv2(M.hx, M.hy, M.hz);
+            Inv2 ih = inv2(M);
             if (G.dim == 3)
                 hipLaunchKernelGGL(k_coarse_inv<3>, dim3(1), dim3(CINV_THREADS), 0, c->stream, M.bx64, M.by64,
                                    M.bz64, L, ih, coarse_inv(c));
@@ -1979,7 +2046,7 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
                       bool zinit) -> int {
         MgLevel &M = c->mg[lv];
         Lay L = lv == 0 ? lay_of(G) : lay_of(M, G.dim);
-        Inv2 ih = inv2(M.hx, M.hy, M.hz);
+        Inv2 ih = inv2(M);
         T *e; const T *f, *bx, *by, *bz;
         arrays(lv, e, f, bx, by, bz);
         const dim3 blk = tile_rows((M.nx + 1) / 2);   // a thread per cell pair of a row
@@ -2133,7 +2200,7 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
         FCFD_TRY(smooth(lv, sweeps(lv, nu1), false, nullptr, nullptr, zero_init && lv == 0));
         MgLevel &M = c->mg[lv], &C = c->mg[lv + 1];
         Lay L = lv == 0 ? lay_of(G) : lay_of(M, G.dim), LC = lay_of(C, G.dim);
-        Inv2 ih = inv2(M.hx, M.hy, M.hz);
+        Inv2 ih = inv2(M);
         T *e; const T *f, *bx, *by, *bz;
         arrays(lv, e, f, bx, by, bz);
         T *ec; const T *fc_, *a, *b, *cc;
@@ -2198,7 +2265,7 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
             arrays(lv, e, f, bx, by, bz);
             V.e = e; V.f = (T *)f; V.bx = bx; V.by = by; V.bz = bz;
             V.L = lay_case(M, G.dim);
-            V.ih = inv2(M.hx, M.hy, M.hz);
+            V.ih = inv2(M);
             V.cx = M.cx; V.cy = M.cy; V.cz = DIM == 3 ? M.cz : 1;
             V.nu1 = sweeps(lv, nu1);
             V.nu2 = sweeps(lv, nu2);
@@ -2223,14 +2290,14 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
         // coarsest: dense inverse or FP64 CG in one workgroup
         MgLevel &M = c->mg[nl - 1];
         Lay L = lay_of(M, G.dim);
-        Inv2 ih = inv2(M.hx, M.hy, M.hz);
+        Inv2 ih = inv2(M);
         T *e; const T *f, *bx, *by, *bz;
         arrays(nl - 1, e, f, bx, by, bz);
         long n = case_cells(M, G.dim);
         ProfScope ps_(c, R_COARSE);
         if (nl > 1 && n <= CDENSE)
             hipLaunchKernelGGL((k_coarse_dense<T>), dim3(DIM == 2 ? c->nb : 1), dim3(CDENSE), 0, c->stream, e, f,
-                               (const double *)coarse_inv(c), lay_case(M, G.dim), DIM);
+                               (const double *)coarse_inv(c), lay_case(M, G.dim), ih, DIM);
         else   // one workgroup per case
             hipLaunchKernelGGL((k_coarse_cg<T, DIM>), dim3(DIM == 2 ? c->nb : 1), dim3(n >= 1024 ? 1024 : 256), 0,
                                c->stream, e, f, bx, by, bz, M.bx64, M.by64, M.bz64, coarse_inv(c),
