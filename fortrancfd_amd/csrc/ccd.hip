@@ -157,7 +157,7 @@ static void ccd_factor(int kind, int N, double dx, std::vector<double> &pk) {
 // x(a_{s+1})), solve a block-tridiagonal system of 4 x 4 blocks, also fixed
 // by the grid, whose block LU is formed here once.  The solve is then
 //   k_seg_lines<.., false>: per segment, x0 at its two ends;
-//   k_seg_reduce:           per line, the reduced forward / backward sweeps;
+//   k_seg_reduce*:          per line, the reduced forward / backward sweeps;
 //   k_seg_lines<.., true>:  per segment, the segment's own system once more
 //                           with x(a-1) and x(b+1) known, written out.
 // Every line has P threads in each sweep and f is read twice.
@@ -1026,7 +1026,8 @@ __global__ void __launch_bounds__(WAVE) k_seg_lines_x(const double *__restrict__
 // 0 the CCD or up-wind system, 1 the down-wind one): forward d'_s = d_s -
 // m_s d'_{s-1}, backward u_s = Dinv_s (d'_s - U_s u_{s+1}), with d_s =
 // (x0(b_s), x0(a_{s+1})) read from zb and u_s = (x(b_s), x(a_{s+1})) written
-// back over them.
+// back over them.  This form takes lines of any length, at one memory latency
+// an interface and sweep; the two below take all but the longest.
 __global__ void __launch_bounds__(SEGT) k_seg_reduce(double *__restrict__ zb, const double *__restrict__ red_u,
                                                      const double *__restrict__ red_d, long nl, int P) {
     const long t = (long)blockIdx.x * SEGT + threadIdx.x;
@@ -1067,6 +1068,95 @@ __global__ void __launch_bounds__(SEGT) k_seg_reduce(double *__restrict__ zb, co
             un[r] = Di[r * 4 + 0] * w[0] + Di[r * 4 + 1] * w[1] + Di[r * 4 + 2] * w[2] + Di[r * 4 + 3] * w[3];
 #pragma unroll
         for (int k = 0; k < 4; ++k) slot(s, k) = un[k];
+    }
+}
+
+// one of a quad's four values, for all its lanes
+template <int K>
+__device__ __forceinline__ double quad_get(double v) {
+    const unsigned lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, (int)hi, K * 0x55, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, (int)lo, K * 0x55, 0xf, 0xf, true));
+}
+
+// row . (the quad's v)
+__device__ __forceinline__ double quad_row(const double2 &a, const double2 &b, double v) {
+    return a.x * quad_get<0>(v) + a.y * quad_get<1>(v) + b.x * quad_get<2>(v) + b.y * quad_get<3>(v);
+}
+
+// The reduced solve of QL lines a block with the lines' values and the
+// coefficients in LDS: the whole block issues all loads at once, then one
+// wave sweeps, four lanes to a line (a row of each 4 x 4 product each, the
+// vector handed around the quad by DPP), an interface's operands read a step
+// ahead.  The chain of 2 NI products bounds it, about 0.1 us each: 783 and
+// 1037 lines of 64 and 48 interfaces take 17.7 us (k_seg_reduce 51 us; 16
+// interfaces at a time through registers, unrolled, 52 us: 48 KB of code per
+// wave).  Sums are in k_seg_reduce's order, so the results are its bits.
+constexpr int QL = 16, QT = 256;
+constexpr int QRED_LDS = 65536;   // at QL * 4 + NRED doubles an interface: up to 73 interfaces
+// up to this many blocks are resident at once (8 of 256 threads on each of
+// 256 CUs); k_seg_reduce_r has a quarter of the instructions and wins where
+// the lines alone fill the chip: 65536 lines of 16 interfaces 18.3 us against
+// 23.8, 39200 of 9 interfaces 11.3 against 12; 19600 of 17 14.8 against 11.8,
+// 28800 of 9 10.7 against 8.4, 2048 of 16 10.3 against 6.2
+constexpr long QROUND = 2048;
+__global__ void __launch_bounds__(QT) k_seg_reduce_q(double *__restrict__ zb, const double *__restrict__ red_u,
+                                                     const double *__restrict__ red_d, long nl, int P) {
+    extern __shared__ double2 qlds[];
+    const int NI = P - 1, y = blockIdx.y, t = threadIdx.x;
+    double *D = (double *)qlds, *R = D + NI * 4 * QL;
+    const double *Rg = y ? red_d : red_u;
+    const long l0 = (long)blockIdx.x * QL;
+    // slots of interface s: (s, 2), (s, 3), (s + 1, 0), (s + 1, 1), four in a row from the third on
+    const bool live = l0 + (t & (QL - 1)) < nl;
+    double *Z = zb + ((long)y * P * 4 + 2) * nl + (live ? l0 + (t & (QL - 1)) : nl - 1);
+#pragma unroll 8
+    for (int k = t / QL; k < NI * 4; k += QT / QL) D[k * QL + (t & (QL - 1))] = Z[k * nl];
+#pragma unroll 4
+    for (int e = t; e < NI * NRED; e += QT) R[e] = Rg[e];
+    __syncthreads();
+    if (t < 4 * QL) {
+        const int r = t & 3;
+        double *d = D + r * QL + (t >> 2);
+        const double2 *m = (const double2 *)R + r * 2;
+        double v = 0.0;
+        {
+            double dn = d[0];
+            double2 a = m[0], b = m[1];
+            for (int s = 0; s < NI; ++s) {
+                const double dc = dn;
+                const double2 ac = a, bc = b;
+                const int n = min(s + 1, NI - 1);
+                dn = d[n * 4 * QL];
+                a = m[n * (NRED / 2)];
+                b = m[n * (NRED / 2) + 1];
+                v = dc - quad_row(ac, bc, v);
+                d[s * 4 * QL] = v;
+            }
+        }
+        double dn = v;
+        const double2 *di = m + 8, *u = m + 16;
+        double2 a = di[(NI - 1) * (NRED / 2)], b = di[(NI - 1) * (NRED / 2) + 1], e = u[(NI - 1) * (NRED / 2)],
+                f = u[(NI - 1) * (NRED / 2) + 1];
+        v = 0.0;
+        for (int s = NI - 1; s >= 0; --s) {
+            const double dc = dn;
+            const double2 ac = a, bc = b, ec = e, fc = f;
+            const int n = max(s - 1, 0);
+            dn = d[n * 4 * QL];
+            a = di[n * (NRED / 2)];
+            b = di[n * (NRED / 2) + 1];
+            e = u[n * (NRED / 2)];
+            f = u[n * (NRED / 2) + 1];
+            const double w = dc - quad_row(ec, fc, v);
+            v = quad_row(ac, bc, w);
+            d[s * 4 * QL] = v;
+        }
+    }
+    __syncthreads();
+    if (live) {
+#pragma unroll 8
+        for (int k = t / QL; k < NI * 4; k += QT / QL) Z[k * nl] = D[k * QL + (t & (QL - 1))];
     }
 }
 
@@ -1146,9 +1236,14 @@ static int seg_solve(fcfd_ctx *c, int ext, int k0, int k1, const double *f, cons
         else
             hipLaunchKernelGGL((k_seg_ends<DIR, NS>), dim3((unsigned)P, gx), dim3(SEGT), 0, c->stream, f, c->ccd_z,
                                tu + end_off, td + end_off, G, ext, P);
-        if (P - 1 <= SEG_MAXI)
+        const size_t ql = (size_t)(P - 1) * (4 * QL + NRED) * sizeof(double);
+        const long qblocks = (nl + QL - 1) / QL;
+        if (P - 1 <= SEG_MAXI && qblocks * NS > QROUND)
             hipLaunchKernelGGL(k_seg_reduce_r<SEG_MAXI>, dim3(gx, NS), dim3(SEGT), 0, c->stream, c->ccd_z,
                                tu + red_off, td + red_off, nl, P);
+        else if (ql <= QRED_LDS)
+            hipLaunchKernelGGL(k_seg_reduce_q, dim3((unsigned)qblocks, NS), dim3(QT), ql, c->stream,
+                               c->ccd_z, tu + red_off, td + red_off, nl, P);
         else
             hipLaunchKernelGGL(k_seg_reduce, dim3(gx, NS), dim3(SEGT), 0, c->stream, c->ccd_z, tu + red_off,
                                td + red_off, nl, P);
