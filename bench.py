@@ -49,8 +49,10 @@ def region_bytes(case, mixed: bool) -> dict:
     nchild0 = 4 if case.dz > 1.5 * case.dx else 8   # first coarsening: x,y only when dz = 2 dx
     return {
         "ls_adv_stage": 8 * N * 20 / 3,        # R{phi,nu,nv,nw,l1..} W{phi',l} averaged over 3 stages
-        "redis_pass_a": 8 * N * 5,             # R{phi,S0} W{grad,s2,s3}
-        "redis_pass_b": 8 * N * 8,             # R{phi,S0,grad,s2,s3,l1,l2,phi0} W{phi,l} averaged over stages
+        # a whole stage but for the interface band's cells (redis_pass_b, not
+        # modelled): R{phi,S0} W{phi',l1}, R{phi,S0,l1} W{phi',l2},
+        # R{phi,S0,l1,l2,phi0} W{phi',grad}, averaged
+        "redis_pass_a": 8 * N * 16 / 3,
         "ccd_lines": 8 * N * 3,                # one direction per launch: R{f} W{fx,fxx}
         "curv": 8 * N * 10,
         "diff_source": 8 * N * 11,
@@ -82,18 +84,17 @@ FP64_PEAK_TFLOPS = 78.6   # MI355X FP64 vector (every lane an FMA each cycle)
 
 def region_flops(case) -> dict:
     """Algorithmic FP64 flops per launch of the FP64-ALU-bound regions (a
-    divide, square root or sine counts as one flop).  One WENO5-JS
-    reconstruction as the kernels write it: three smoothness indicators
-    (~33), q_k = (EPS + beta_k)^2 (6), the product-form weights (5), their
-    normalisation (3 + 3) and the stencil combination (~25): ~75.
-    WENO stage: 3 faces per cell (each shared by two cells) x 2
-    reconstructions = 450, flux splits 3 x 7, face sums, divergence and the
-    increment-form update ~20: ~490 per cell.  Reinit pass A: 2 one-sided
-    reconstructions per direction = 450, 7 backward differences per
-    direction x 2 = 42, Godunov selection and |grad| ~15, smoothed
-    Heaviside / delta and the lambda terms ~20: ~530 per cell."""
+    divide, square root or sine counts as one flop, an fma as two).  One
+    WENO5-JS value in sample differences: 4 differences, 3 smoothness
+    indicators (24), the product-form weights (8), candidates (9), their sum
+    and normalisation (12): ~57.  WENO stage: 3 faces per cell (each shared
+    by two cells) x 2 reconstructions = 342, flux splits 3 x 7, face sums,
+    divergence and the increment-form update ~20: ~385 per cell.  Reinit
+    stage: 2 one-sided reconstructions per direction = 342, 7 backward
+    differences per direction x 2 = 42, Godunov selection and |grad| ~15,
+    source and update ~10, a few per cent of band cells: ~410 per cell."""
     N = case.nx * case.ny * case.nz
-    return {"ls_adv_stage": N * 490, "redis_pass_a": N * 530}
+    return {"ls_adv_stage": N * 385, "redis_pass_a": N * 410}
 
 
 def profiled_traffic(region: str):
