@@ -65,13 +65,16 @@ __device__ __forceinline__ void clamp_window(double (&d)[W], int lo, int hi) {
 
 // element at a byte offset from a base that is uniform over the wave: the
 // load takes the base from scalar registers and 32 offset bits per lane (an
-// index would be scaled in 64-bit vector arithmetic for every load)
-template <typename T>
-__device__ __forceinline__ T &at_bytes(T *base, unsigned bytes) {
+// index would be scaled in 64-bit vector arithmetic for every load).  A
+// caller's 32-bit offsets must stay below 4 GiB: inside a tile or a row
+// segment, not inside a plane (a 2D plane of 23200 x 23200 cells is larger);
+// 64-bit offsets are plain addresses.
+template <typename T, typename O>
+__device__ __forceinline__ T &at_bytes(T *base, O bytes) {
     return *(T *)((char *)base + bytes);
 }
-template <typename T>
-__device__ __forceinline__ const T &at_bytes(const T *base, unsigned bytes) {
+template <typename T, typename O>
+__device__ __forceinline__ const T &at_bytes(const T *base, O bytes) {
     return *(const T *)((const char *)base + bytes);
 }
 

@@ -380,7 +380,10 @@ int mpls(fcfd_ctx *c) {
 // F = WENO_left(s1 at f-2..f+2) + WENO_right(s2 at f-1..f+3) at clamped
 // positions; L sums F(+1/2) - F(-1/2) per direction.
 // With TX = 64 a wave is one row, so a face's six rows (y) or its row (x)
-// have scalar bases and one vector offset.
+// have scalar bases and one vector offset.  O is the type of a face's byte
+// offsets from the first cell its tile reads, OFF_ROWS rows at most: 32 bits,
+// or 64 bits where that many rows pass 4 GiB (launch_stage).  Every other
+// address is a 64-bit row base and an offset inside the tile's row.
 //
 // What bounds it: a plane is a chain of memory round trips, the faces one
 // after the other and a barrier, about 5 us; a block's planes are serial, so
@@ -388,12 +391,15 @@ int mpls(fcfd_ctx *c) {
 // 256^3 (533 with 256 threads striding over the 580 faces at 64-bit
 // addresses), 54 us at 128^3 (83 with 16 planes a block whatever the grid), 30
 // us in FP32 at 101 x 87 x 117 (90).
+template <int TX>
+constexpr int OFF_ROWS = 256 / TX + 6;   // rows j0 - 3 .. j0 + TY + 2
+
 template <int DIM, typename T, int TX>
 struct StageLds {
     T fx[2][256 / TX][TX + 1], fy[2][256 / TX + 1][TX];
 };
 
-template <int DIM, typename T, int TX>
+template <int DIM, typename T, int TX, typename O>
 __device__ __forceinline__ void ls_adv_stage_body(StageLds<DIM, T, TX> &sh, const T *__restrict__ phi,
                                                   T *__restrict__ phin, const T *__restrict__ nu,
                                                   const T *__restrict__ nv, const T *__restrict__ nw,
@@ -430,13 +436,15 @@ __device__ __forceinline__ void ls_adv_stage_body(StageLds<DIM, T, TX> &sh, cons
         }
         return weno_left(s1[0], s1[1], s1[2], s1[3], s1[4], EPS) + weno_right(s2[1], s2[2], s2[3], s2[4], s2[5], EPS);
     };
-    const unsigned co = (unsigned)(ic + G.g) * (unsigned)sizeof(T);
+    const unsigned co = (unsigned)(ic - i0) * (unsigned)sizeof(T);   // offset of this column from the tile's first
+    // first column and row that the tile's faces read
+    const int cb = max(i0 - 3, xlo), rb = max(j0 - 3, ylo);
     // z window of this column: positions clamp(k - 3 + m), m = 0..6
     T s1z[7], s2z[7], Fl = 0;
     if (DIM == 3) {
 #pragma unroll
         for (int m = 0; m < 7; ++m) {
-            const long row = G.id(0, jc, clampi(k0 - 3 + m, zlo, zhi)) - G.g;
+            const long row = G.id(i0, jc, clampi(k0 - 3 + m, zlo, zhi));
             const T u = vs * at_bytes(nw + row, co), p = at_bytes(phi + row, co);
             s1z[m] = half * (u + fabs(u)) * p;
             s2z[m] = half * (u - fabs(u)) * p;
@@ -447,21 +455,22 @@ __device__ __forceinline__ void ls_adv_stage_body(StageLds<DIM, T, TX> &sh, cons
     for (int k = k0; k < k1; ++k) {
         const int b = k & 1;
         // this cell's operands and the z window's next plane, ahead of the faces
-        const long rc = G.id(0, jc, k) - G.g;
+        const long rc = G.id(i0, jc, k);
         const T pc = at_bytes(phi + rc, co);
         const T l1o = stage >= 1 ? at_bytes(l1 + rc, co) : (T)0, l2o = stage == 2 ? at_bytes(l2 + rc, co) : (T)0;
         T wn = 0, pn = 0;
         if (DIM == 3) {
-            const long row = G.id(0, jc, clampi(k + 4, zlo, zhi)) - G.g;
+            const long row = G.id(i0, jc, clampi(k + 4, zlo, zhi));
             wn = at_bytes(nw + row, co);
             pn = at_bytes(phi + row, co);
         }
         // the x-face and the y-face below the cell, then the tile's last
         // y-face row (first TX threads) and last x-faces (TY threads), one
         // after the other: unrolled, their loads take 198 VGPRs.  A face reads
-        // positions clamp(f - 2 + m) of its line at byte offsets from the
-        // plane's first cell.
-        const long pl = G.id(0, 0, k) - G.g - (long)G.g * G.sx;
+        // positions clamp(f - 2 + m) of its line at byte offsets from cell
+        // (cb, rb) of the plane; o0 may be below it (modulo 2^32 or 2^64), the
+        // sums never are.
+        const long pl = G.id(cb, rb, k);
         const T *pp = phi + pl;
 #pragma unroll 1
         for (int r = 0; r < 3; ++r) {
@@ -471,13 +480,12 @@ __device__ __forceinline__ void ls_adv_stage_body(StageLds<DIM, T, TX> &sh, cons
             const int row = xf ? (last ? min(j0 + t - 128, G.ny - 1) : jc) : 0;
             const int f = xf ? (last ? i0 + TX - 1 : i - 1) : (last ? j0 + TY - 1 : j - 1);
             const int lo = xf ? xlo : ylo, hi = xf ? xhi : yhi;
-            const unsigned st = (xf ? 1u : (unsigned)G.sx) * (unsigned)sizeof(T);
-            const unsigned o0 = xf ? (unsigned)((row + G.g) * (int)G.sx + G.g) * (unsigned)sizeof(T)
-                                   : co + (unsigned)(G.g * (int)G.sx) * (unsigned)sizeof(T);
+            const O st = (xf ? (O)1 : (O)G.sx) * (O)sizeof(T);
+            const O o0 = xf ? ((O)(row - rb) * (O)G.sx - (O)cb) * (O)sizeof(T) : (O)(ic - cb) * (O)sizeof(T) - (O)rb * st;
             T u[6], p[6];
 #pragma unroll
             for (int m = 0; m < 6; ++m) {
-                const unsigned o = o0 + (unsigned)clampi(f - 2 + m, lo, hi) * st;
+                const O o = o0 + (O)clampi(f - 2 + m, lo, hi) * st;
                 u[m] = at_bytes(vp, o);
                 p[m] = at_bytes(pp, o);
             }
@@ -522,7 +530,7 @@ __device__ __forceinline__ void ls_adv_stage_body(StageLds<DIM, T, TX> &sh, cons
     }
 }
 
-template <int DIM, typename T, int TX>
+template <int DIM, typename T, int TX, typename O>
 __global__ void __launch_bounds__(256) k_ls_adv_stage(const T *__restrict__ phi, T *__restrict__ phin,
                                                       const T *__restrict__ nu, const T *__restrict__ nv,
                                                       const T *__restrict__ nw, T *__restrict__ l1,
@@ -530,14 +538,14 @@ __global__ void __launch_bounds__(256) k_ls_adv_stage(const T *__restrict__ phi,
     __shared__ StageLds<DIM, T, TX> sh;
     int bx_, by_, bz_;
     xcd_block(bx_, by_, bz_);
-    ls_adv_stage_body<DIM, T, TX>(sh, phi, phin, nu, nv, nw, l1, l2, G, dt, vs, stage, kc, bx_, by_, bz_);
+    ls_adv_stage_body<DIM, T, TX, O>(sh, phi, phin, nu, nv, nw, l1, l2, G, dt, vs, stage, kc, bx_, by_, bz_);
 }
 
 // the same stage on every block of a multi-block layout in one launch:
 // tab[b] places block b in the stacks; the grid covers the largest block, nz
 // walks per block along z.  (A launch per block of 80 x 75 x 85 cells leaves
 // the chip nearly empty: 75 us each, eight in a row; together 134 us.)
-template <int DIM, int TX>
+template <int DIM, int TX, typename O>
 __global__ void __launch_bounds__(256) k_ls_adv_stage_blocks(const double *__restrict__ phi,
                                                              double *__restrict__ phin,
                                                              const double *__restrict__ nu,
@@ -552,8 +560,8 @@ __global__ void __launch_bounds__(256) k_ls_adv_stage_blocks(const double *__res
     const int b = bz_ / nz;
     const Geom G = tab[b].G;
     const long o = tab[b].off;
-    ls_adv_stage_body<DIM, double, TX>(sh, phi + o, phin + o, nu + o, nv + o, DIM == 3 ? nw + o : nullptr, l1 + o,
-                                       l2 + o, G, dt, 1.0, stage, kc, bx_, by_, bz_ - b * nz);
+    ls_adv_stage_body<DIM, double, TX, O>(sh, phi + o, phin + o, nu + o, nv + o, DIM == 3 ? nw + o : nullptr, l1 + o,
+                                          l2 + o, G, dt, 1.0, stage, kc, bx_, by_, bz_ - b * nz);
 }
 
 // One SSP-RK3 stage with the UCCD source L = -(u phi_x + v phi_y + w phi_z)
@@ -596,19 +604,27 @@ static int stage_planes(long tiles, int nz, int ncu) {
     return kc;
 }
 
+// whether a stage's face offsets fit 32 bits: OFF_ROWS rows of sx elements
+// (rows of up to 53 million cells in FP64 with TX = 64, 38 million with 32)
+static bool stage_off32(const dim3 &blk, long sx, size_t size) {
+    return (double)(blk.x == 64 ? OFF_ROWS<64> : OFF_ROWS<32>) * (double)sx * (double)size < 4294967296.0;
+}
+
 template <int DIM, typename T>
 static int launch_stage(hipStream_t st, int ncu, const Geom &G, const T *phi, T *phin, const T *nu, const T *nv,
                         const T *nw, T *l1, T *l2, T dt, T vs, int stage) {
-    const dim3 blk = tile_rows(G.nx);
+    const bool off32 = stage_off32(tile_rows(G.nx), G.sx, sizeof(T));
+    const dim3 blk = off32 ? tile_rows(G.nx) : dim3(64, 4);
     const dim3 tiles((G.nx + blk.x - 1) / blk.x, (G.ny + blk.y - 1) / blk.y, G.nz);
     const int kc = DIM == 3 ? stage_planes((long)tiles.x * tiles.y, G.nz, ncu) : 1;
     const dim3 grd(tiles.x, tiles.y, (G.nz + kc - 1) / kc);
-    if (blk.x == 64)
-        hipLaunchKernelGGL((k_ls_adv_stage<DIM, T, 64>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, G, dt, vs,
-                           stage, kc);
-    else
-        hipLaunchKernelGGL((k_ls_adv_stage<DIM, T, 32>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, G, dt, vs,
-                           stage, kc);
+#define FCFD_ST(X_, O_)                                                                                             \
+    hipLaunchKernelGGL((k_ls_adv_stage<DIM, T, X_, O_>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, G, dt, vs, \
+                       stage, kc)
+    if (!off32) FCFD_ST(64, unsigned long);
+    else if (blk.x == 64) FCFD_ST(64, unsigned);
+    else FCFD_ST(32, unsigned);
+#undef FCFD_ST
     FCFD_CHECK(hipGetLastError());
     return FCFD_OK;
 }
@@ -627,19 +643,22 @@ int ls_adv_stage(fcfd_ctx *c, const double *phi, double *phin, int stage) {
 int ls_adv_stage_blocks(hipStream_t st, int ncu, const BlockGeom *tab, int nblk, int dim, int nx, int ny, int nz,
                         const double *phi, double *phin, const double *nu, const double *nv, const double *nw,
                         double *l1, double *l2, double dt, int stage) {
-    const dim3 blk = tile_rows(nx);
+    const bool off32 = stage_off32(tile_rows(nx), nx + 6, sizeof(double));   // 3 ghosts a side
+    const dim3 blk = off32 ? tile_rows(nx) : dim3(64, 4);
     const dim3 tiles((nx + blk.x - 1) / blk.x, (ny + blk.y - 1) / blk.y);
     const int kc = dim == 3 ? stage_planes((long)tiles.x * tiles.y * nblk, nz, ncu) : 1, kz = (nz + kc - 1) / kc;
     const dim3 grd(tiles.x, tiles.y, (unsigned)(nblk * kz));
-#define FCFD_SB(D_, X_)                                                                                         \
-    hipLaunchKernelGGL((k_ls_adv_stage_blocks<D_, X_>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, tab, dt, \
+#define FCFD_SB(D_, X_, O_)                                                                                         \
+    hipLaunchKernelGGL((k_ls_adv_stage_blocks<D_, X_, O_>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, tab, dt, \
                        stage, kc, kz)
     if (dim == 3) {
-        if (blk.x == 64) FCFD_SB(3, 64);
-        else FCFD_SB(3, 32);
+        if (!off32) FCFD_SB(3, 64, unsigned long);
+        else if (blk.x == 64) FCFD_SB(3, 64, unsigned);
+        else FCFD_SB(3, 32, unsigned);
     } else {
-        if (blk.x == 64) FCFD_SB(2, 64);
-        else FCFD_SB(2, 32);
+        if (!off32) FCFD_SB(2, 64, unsigned long);
+        else if (blk.x == 64) FCFD_SB(2, 64, unsigned);
+        else FCFD_SB(2, 32, unsigned);
     }
 #undef FCFD_SB
     FCFD_CHECK(hipGetLastError());

@@ -2,8 +2,9 @@
 below, at and above 32 and 64 cells (32- and 64-wide tiles), fewer rows than a
 tile, and planes that do not fill a walk (4 planes a block on small grids),
 against the oracle at the advection's tolerance (1e-12 of the field's max, as
-in test_gpu_parity.py); and the multi-block launch on blocks of unequal
-extents, bit for bit the whole-field step."""
+in test_gpu_parity.py); the multi-block launch on blocks of unequal extents,
+bit for bit the whole-field step; and a plane of more than 4 GiB, which 32-bit
+byte offsets from its first cell do not span."""
 import numpy as np
 import pytest
 import torch   # before the library: both then share one HIP runtime
@@ -67,3 +68,42 @@ def test_blocks_in_one_launch(size, nb):
     B.gather(st, out)
     torch.cuda.synchronize()
     assert np.array_equal(case.interior(out.cpu().numpy()), case.interior(s.pull("phi")))
+
+
+def _repeated(n, m, along):
+    """a level set and a velocity on (m + 6) x (n + 6) cells, ghosts included, that repeat every 1000 along one axis
+    (0: the rows, 1: the row)"""
+    g = torch.Generator().manual_seed(7)
+    x = torch.linspace(0.0, 6.0, m + 6, dtype=torch.float64)
+    y = torch.arange(1000, dtype=torch.float64)[:, None] * (2.0 * np.pi / 1000)
+    base = [torch.sin(40.0 * y + x), torch.cos(30.0 * y - x), torch.sin(20.0 * y) * torch.cos(x)]
+    base = [b + 0.01 * torch.rand(b.shape, generator=g, dtype=torch.float64) for b in base]
+    at = (torch.arange(-3, n + 3) % 1000).cuda()
+    return [(b.cuda() if along == 0 else b.T.contiguous().cuda()).index_select(along, at) for b in base]
+
+
+# 26 and 58 cells a row: the 32- and the 64-wide tiles, a plane of more than
+# 4 GiB; along 1: rows so long that ten of them (what a tile reads) pass
+# 4 GiB, which takes the instance with 64-bit offsets
+@pytest.mark.parametrize("m,along", [(26, 0), (58, 0), (10, 1)])
+def test_plane_over_4gib(m, along):
+    from fortrancfd_amd.blocks import Blocks
+    if torch.cuda.mem_get_info()[0] < 96 << 30:
+        pytest.skip("needs 96 GiB of device memory")
+    full = 2 ** 32 // 80 if along else 2 ** 32 // (8 * (m + 6))   # cells along the axis at the limit
+    out = []
+    for n in (full + 4096, 5000):
+        phi, nu, nv = _repeated(n, m, along)
+        nx, ny = (n, m) if along else (m, n)
+        case = Case(dim=2, nx=nx, ny=ny, nz=1, xend=nx / 32.0, yend=ny / 32.0)
+        B = Blocks(case, 1, 1)
+        assert B.stack_size == phi.numel()
+        B.level_set_rk3_solver(phi, nu, nv)
+        torch.cuda.synchronize()
+        B.close()
+        # 2000 cells past the limit, of the same phase in both, far from the walls
+        r = (1000 if n == 5000 else 1000 * (full // 1000 + 1)) + 3
+        out.append(phi.narrow(along, r, 2000).narrow(1 - along, 3, m).cpu().numpy())
+        del phi, nu, nv
+        torch.cuda.empty_cache()
+    assert np.array_equal(out[0], out[1])
