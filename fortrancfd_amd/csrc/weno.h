@@ -129,7 +129,10 @@ __device__ __forceinline__ float weno_fma(float x, float y, float z) { return fm
 // d(weno_left)/dg_m times vb, into gb[0..4], for the forward's form
 // V = g2 + N r, N = sum a_k c_k, r = 1 / (6 sum a_k): dV/dc_k = a_k r and,
 // with da_k/db_k = -2 a_k / b_k, dV/db_k = -2 a_k r (c_k - 6 N r) / b_k;
-// then back through t, s and c to the differences e and the samples.  T =
+// then back through t, s and c to the differences e and the samples.  The
+// weights a_k r are formed before vb comes in: where the samples are flat
+// (b = EPS / 3) r is 2e-29 in FP32, and vb r would lose the bits of a vb
+// below 6e-10 and vanish below 1e-17.  T =
 // double or float (the weights of that precision's forward).  About 105
 // operations, where differentiating the normalised weights took about 160.
 template <typename T>
@@ -145,11 +148,10 @@ __device__ __forceinline__ void weno_left_adj(const T *g, T EPS, T vb, T *gb) {
     weno_adj_weights(b, a, ib);
     const T r = weno_rcp((T)6 * (a[0] + (a[1] + a[2])));
     const T m = (T)-6 * (weno_fma(a[2], c[2], weno_fma(a[1], c[1], a[0] * c[0])) * r);   // -6 N r
-    const T vr = vb * r;
     T cb[3], tb[3], sb[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        cb[k] = a[k] * vr;
+        cb[k] = (a[k] * r) * vb;
         const T bb = (-two * cb[k]) * ((c[k] + m) * ib[k]);
         tb[k] = ((two * c133) * bb) * t[k];
         sb[k] = (two * bb) * s[k];

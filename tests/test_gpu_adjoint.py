@@ -375,3 +375,48 @@ def test_fp32_gradient_against_fp64():
     m = np.ones(case.shape, dtype=bool)
     m[g:-g, g:-g, g:-g] = False
     assert not g32[m].any()
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+def test_adjoint_step_scales_with_its_cotangent(dtype):
+    """The adjoint step is linear in its cotangent: one smaller by a power of
+    two (2^-50 of O(1), as the gradient tails of a mean over 10^7 cells) gives
+    the same bits scaled, as long as nothing on the way leaves the normal
+    range.  Where the level set and the velocity are constant the weights are
+    the linear ones and every term is of the cotangent's size: exact equality.
+    Elsewhere products of the weights (>= 1e-20 or so) may: 1e-5 of the
+    largest entry, 100 FP32 roundings, covers a cell whose own terms are lost.
+    In the flat part the linear fifth-order weights 0.1, 0.6, 0.3 are also
+    compared with the FP64 step's result (1e-5: sums of about 30 terms)."""
+    case = _case((56, 12, 10))
+    s = _solver(case)
+    tt = getattr(torch, dtype)
+    dev = torch.device("cuda")
+    g = case.ghc
+    x = np.arange(-g, case.nx + g)
+    row = 1.0 + np.where(x < 16, 0.3 * np.sin(0.4 * x) * np.maximum(0, 16 - x) / 16.0, 0.0)
+    phi = np.broadcast_to(row, case.shape)
+    w = _interior_random(case, np.random.default_rng(7)).astype(np.float32).astype(np.float64)
+    vel = [np.full(case.shape, c) for c in (0.5, -0.25, 0.75)]
+    for nm, a in zip(("nu", "nv", "nw"), vel):
+        s.push(nm, a)
+
+    def run(scale, tt):
+        d = lambda a: torch.from_numpy(np.ascontiguousarray(a).reshape(-1)).to(dev, tt)
+        ph, lam, vt = d(phi), d(w * scale), [d(a) for a in vel]
+        bars = [torch.zeros(case.size, dtype=tt, device=dev) for _ in range(3)]
+        torch.cuda.synchronize()
+        ptrs = [ph.data_ptr(), lam.data_ptr(), *(b.data_ptr() for b in bars)]
+        if tt == torch.float64:
+            s.ls_adv_adjoint_step(*ptrs)
+        else:
+            s.ls_adv_adjoint_step_f32(*ptrs, *(v.data_ptr() for v in vt))
+        s.sync()
+        return [a.double().cpu().numpy().reshape(case.shape)[g:-g, g:-g, g:-g] / scale for a in [lam, *bars]]
+
+    small, one, ref = run(2.0 ** -50, tt), run(1.0, tt), run(1.0, torch.float64)
+    # the stages' faces reach 9 cells into the constant part
+    for a, b, r in zip(small, one, ref):
+        assert np.array_equal(a[:, :, 28:], b[:, :, 28:])
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+        assert np.abs(b - r)[:, :, 28:].max() <= 1e-5 * np.abs(r).max()
