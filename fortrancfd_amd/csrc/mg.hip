@@ -1301,73 +1301,58 @@ __global__ void __launch_bounds__(CINV_THREADS) k_coarse_inv(const double *__res
             if (r0 + a < n && c0 + b < n) minv[(long)(r0 + a) * n + c0 + b] = m[a][b];
 }
 
-// e = M^-1 b with b = -(f - mean f), f times the cell volumes, then the zero-mean projection of e;
-// one block of CDENSE threads, one cell per thread
-template <typename T>
-__global__ void __launch_bounds__(CDENSE) k_coarse_dense(T *__restrict__ eout, const T *__restrict__ fin,
-                                                         const double *__restrict__ minv, Lay L, Inv2 ih, int dim) {
-    if (L.skipped()) return;
-    constexpr int NW = CDENSE / WAVE;
-    __shared__ double b[CDENSE];
-    __shared__ double ws[NW];
-    const int t = threadIdx.x, n = L.nx * L.ny * L.nz;
-    const int kq = dim == 2 ? (int)blockIdx.x : 0;   // case of a batched 2D stack (L: one slice)
-    minv += (long)kq * n * n;
-    int i = 0, j = 0, k = kq;
-    double f = 0.0;
-    if (t < n) {
-        cell_coords(L, t, i, j, k);
-        f = ih.template weight<double>(L, i, j, k, dim) * (double)fin[L.id(i, j, k + kq)];
-        k += kq;
-    }
-    // fixed-order block sum: butterfly per wave (lane 0's order), then waves in order
-    auto block_sum = [&](double v) {
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-        if ((t & (WAVE - 1)) == 0) ws[t / WAVE] = v;
-        __syncthreads();
-        double sum = 0.0;
-        for (int w = 0; w < NW; ++w) sum += ws[w];
-        __syncthreads();
-        return sum;
-    };
-    const double fm = block_sum(f) / (double)n;
-    if (t < n) b[t] = fm - f;
-    __syncthreads();
-    double x = 0.0;
-    if (t < n)
-        for (int c = 0; c < n; ++c) x += minv[c * n + t] * b[c];
-    const double xm = block_sum(x) / (double)n;
-    if (t < n) eout[L.id(i, j, k)] = (T)(x - xm);
-}
-
-// Small levels in one workgroup: every level of at most TAIL_MAX cells, down
-// to the dense coarsest solve and back up, runs inside a single launch with
-// barriers between the phases.  On MI355X a dependent launch costs ~4 us
-// however small the grid, and these levels take up to 12 sweeps each; a phase
-// with one cell per thread costs ~1-2 us.  (With 8 cells per thread read from
-// global memory, an 8192-cell level inside the workgroup was slower than
-// separate launches: the sweeps wait on dependent L2 loads.)
+// Small levels in one workgroup: from the first level that fits (tail_fits),
+// down to the dense coarsest solve and back up, the cycle runs inside a
+// single launch with barriers between the phases.  On MI355X a dependent
+// launch costs ~4 us however small the grid, and these levels take up to 12
+// sweeps each; a phase with one cell per thread costs ~1-2 us.  (With 8 cells
+// per thread read from global memory, an 8192-cell level inside the workgroup
+// was slower than separate launches: the sweeps wait on dependent L2 loads.)
 //
 // FP32 cycles may in addition take one fully coarsened "top" level of up to
 // TAIL_TOP cells (8192 = 8 per thread) whose error (TAIL_LDS floats with
 // padding) and rhs live in LDS and whose six face coefficients per cell live
 // in the registers of the thread that owns the cell; a thread owns whole
 // coarse cells with all their children, so the restriction needs no
-// exchange.  FP64 would need twice the registers (spills) and keeps TAIL_MAX.
+// exchange.  FP64 would need twice the registers (spills) and has no top.
 //
-// The levels of at most TAIL_MAX cells keep their error in LDS for the whole
-// cycle (ghosted boxes of TAIL_ELDS elements in all, ghosts 0).  A thread
-// owns pairs of neighbouring cells of a row, one of each colour, so that
-// every thread has one cell per pair in every half-sweep; it holds their LDS
-// positions, face coefficients, reciprocal diagonals and rhs in registers,
-// loaded from global memory once per down and once per up phase.  A
-// half-sweep is then seven LDS reads, the update and a barrier.  (With cells
-// dealt out in memory order half of the threads were idle in a half-sweep,
-// and every one recomputed its cells' positions.)  Each level's error is
-// written back at the end of its up phase.
+// The levels below the top, of at most TAIL_MAX cells, keep their error in
+// LDS for the whole cycle (ghosted boxes of TAIL_ELDS elements in all, ghosts
+// 0).  A thread owns pairs of neighbouring cells of a row, one of each
+// colour, so that every thread has one cell per pair in every half-sweep; it
+// holds their LDS positions, face coefficients, reciprocal diagonals and rhs
+// in registers, loaded from global memory once per down and once per up
+// phase.  A half-sweep is then seven LDS reads, the update and a barrier.
+// (With cells dealt out in memory order half of the threads were idle in a
+// half-sweep, and every one recomputed its cells' positions.)  Each level's
+// error is written back at the end of its up phase.
 constexpr int TAIL_MAX = 4096, TAIL_THREADS = 1024, TAIL_LEVELS = 8, TAIL_PAIRS = TAIL_MAX / (2 * TAIL_THREADS);
 constexpr int TAIL_TOP = 8192, TAIL_LDS = 12288, TAIL_SLOTS = TAIL_TOP / TAIL_THREADS;
 constexpr int TAIL_ELDS = 8192;
+
+// elements of a level's ghosted box
+template <int DIM>
+__host__ __device__ __forceinline__ int tail_box(const Lay &L) {
+    return (L.nx + 2) * (L.ny + 2) * (DIM == 3 ? L.nz + 2 : 1);
+}
+
+// Whether the levels from lv on can be resident: every one's pairs have an
+// owner and their boxes share TAIL_ELDS.  A row of odd length has a pair more
+// than half its cells, so a level of fewer than TAIL_MAX cells may not fit
+// (13 x 15 x 20: 3900 cells, 2100 pairs); the tail then starts a level lower.
+// (Run from global memory by the one workgroup instead, the FP64 step of
+// 100 x 120 x 160 cells took 15.3 ms and that of 60 x 64 x 68 8.2 ms; 12.6
+// and 5.5 ms this way.)
+static bool tail_fits(const fcfd_ctx *c, int lv) {
+    long boxes = 0;
+    for (size_t q = lv; q < c->mg.size(); ++q) {
+        const Lay L = lay_case(c->mg[q], c->G.dim);
+        if ((long)((L.nx + 1) / 2) * L.ny * L.nz > TAIL_PAIRS * TAIL_THREADS) return false;
+        boxes += c->G.dim == 3 ? tail_box<3>(L) : tail_box<2>(L);
+        if (boxes > TAIL_ELDS) return false;
+    }
+    return true;
+}
 
 template <typename T>
 struct TailLevel {
@@ -1386,8 +1371,7 @@ struct TailArgs {
     int n;                 // levels in the tail; the last is solved densely
     int top;               // lv[0] is an LDS/register top level (FP32 only)
     const double *minv;    // dense inverse of the last level (k_coarse_inv)
-    int lds;               // levels from lv[top] on keep their error in LDS
-    int eoff[TAIL_LEVELS]; // offset of each such level's ghosted box
+    int eoff[TAIL_LEVELS]; // offset of the ghosted box of each level from lv[top] on
 };
 
 // 1 / sc of a Gauss-Seidel update in the cycle's precision (0 off the grid)
@@ -1419,21 +1403,6 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         k += kq;
     };
     auto ncells = [](const Lay &L) { return L.nx * L.ny * L.nz; };
-    auto gs = [&](const TailLevel<T> &V, int color) {
-        const Lay &L = V.L;
-        const int n = ncells(L);
-        const Prol<T> P0{nullptr, Lay{}, 0, 0, 0};
-        for (int c = t; c < n; c += TAIL_THREADS) {
-            int i, j, k;
-            cell_coords(L, c, i, j, k);
-            if (((i + j + (DIM == 3 ? k : 0)) & 1) != color) continue;   // 2D: k is the case
-            const long id = L.id(i, j, k);
-            T sc, sce, ep;
-            stencil<T, DIM, false, 0, T>(V.e, nullptr, V.bx, V.by, V.bz, L, V.ih, i, j, k, id, P0, sc, sce, ep);
-            V.e[id] = sc > (T)0 ? ep + gs_step<T>(sce - V.f[id], sc) : ep;
-        }
-        __syncthreads();
-    };
     // fixed-order sum over the block: wave butterflies, then the waves in order
     auto block_sum = [&](double v) {
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
@@ -1445,13 +1414,12 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         return s;
     };
     const int nl = A.n;
-    // ---- LDS-resident levels (A.lds): error in a ghosted box per level
+    // ---- levels below the top: error in a ghosted box of LDS per level
     __shared__ T el_[TAIL_ELDS];
     __shared__ T rt_[TAIL_MAX];
     auto lbox = [](const Lay &L, int i, int j, int k) {   // k: 0 in 2D
         return (i + 1) + (L.nx + 2) * ((j + 1) + (DIM == 3 ? (L.ny + 2) * (k + 1) : 0));
     };
-    auto boxn = [](const Lay &L) { return (L.nx + 2) * (L.ny + 2) * (DIM == 3 ? L.nz + 2 : 1); };
     // this thread's pairs of a level: pair q = t + u TAIL_THREADS covers cells
     // 2m, 2m + 1 of a row; the cell of colour c is i = 2m + ((j + k + c) & 1)
     auto load_cells = [&](const TailLevel<T> &V, TailCells<T> &Q) {
@@ -1627,13 +1595,13 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         }
     }
     // down: smooth, restrict the residual, clear the coarse error
-    for (int a = a0; a < nl - 1 && A.lds; ++a) {
+    for (int a = a0; a < nl - 1; ++a) {
         const TailLevel<T> &F = A.lv[a];
         const TailLevel<T> &C = A.lv[a + 1];
         const Lay &L = F.L;
         T *el = el_ + A.eoff[a];
         TailCells<T> Q;
-        for (int q = t; q < boxn(L); q += TAIL_THREADS) el[q] = (T)0;
+        for (int q = t; q < tail_box<DIM>(L); q += TAIL_THREADS) el[q] = (T)0;
         load_cells(F, Q);
         __syncthreads();
         const int n = ncells(L);
@@ -1683,33 +1651,6 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         }
         __syncthreads();
     }
-    for (int a = a0; a < nl - 1 && !A.lds; ++a) {
-        const TailLevel<T> &F = A.lv[a];
-        const TailLevel<T> &C = A.lv[a + 1];
-        for (int s = 0; s < F.nu1; ++s) { gs(F, 0); gs(F, 1); }
-        const int nc = ncells(C.L);
-        for (int cc = t; cc < nc; cc += TAIL_THREADS) {
-            int I, J, K;
-            cell_coords(C.L, cc, I, J, K);
-            T acc = 0, wsum = 0;
-            for (int kk = 0; kk < F.cz; ++kk)
-                for (int jj = 0; jj < F.cy; ++jj)
-                    for (int ii = 0; ii < F.cx; ++ii) {
-                        const int i = I * F.cx + ii, j = J * F.cy + jj, k = K * F.cz + kk;
-                        // the last aggregate of an odd axis has one child (2D: k is the case)
-                        if (i >= F.L.nx || j >= F.L.ny || (DIM == 3 && k >= F.L.nz)) continue;
-                        const long id = F.L.id(i, j, k);
-                        const T w = F.ih.template weight<T>(F.L, i, j, k, DIM);
-                        acc += w * (F.f[id] -
-                                    apply_A<T, DIM, false, T>(F.e, nullptr, F.bx, F.by, F.bz, F.L, F.ih, i, j, k, id));
-                        wsum += w;
-                    }
-            const long cid = C.L.id(I, J, K);
-            C.f[cid] = acc / wsum;
-            C.e[cid] = (T)0;
-        }
-        __syncthreads();
-    }
     // coarsest: e = M^-1 b, b = -(f - mean f), zero-mean result
     {
         const TailLevel<T> &V = A.lv[nl - 1];
@@ -1738,16 +1679,14 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
         }
         const double xm = block_sum(t < n ? x : 0.0) / (double)n;
         if (t < n) V.e[V.L.id(i, j, k)] = (T)(x - xm);
-        if (A.lds) {
-            T *el = el_ + A.eoff[nl - 1];
-            for (int q = t; q < boxn(V.L); q += TAIL_THREADS) el[q] = (T)0;
-            __syncthreads();
-            if (t < n) el[lbox(V.L, i, j, DIM == 3 ? k : 0)] = (T)(x - xm);
-        }
+        T *el = el_ + A.eoff[nl - 1];
+        for (int q = t; q < tail_box<DIM>(V.L); q += TAIL_THREADS) el[q] = (T)0;
+        __syncthreads();
+        if (t < n) el[lbox(V.L, i, j, DIM == 3 ? k : 0)] = (T)(x - xm);
         __syncthreads();
     }
     // up: prolong (piecewise constant), smooth; LDS levels write their error back
-    for (int a = nl - 2; a >= a0 && A.lds; --a) {
+    for (int a = nl - 2; a >= a0; --a) {
         const TailLevel<T> &F = A.lv[a];
         const TailLevel<T> &C = A.lv[a + 1];
         const Lay &L = F.L;
@@ -1770,18 +1709,6 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(TailArgs<T> A) {
             F.e[L.id(i, j, k)] = el[lbox(L, i, j, DIM == 3 ? k : 0)];
         }
         __syncthreads();
-    }
-    for (int a = nl - 2; a >= a0 && !A.lds; --a) {
-        const TailLevel<T> &F = A.lv[a];
-        const TailLevel<T> &C = A.lv[a + 1];
-        const int n = ncells(F.L);
-        for (int c = t; c < n; c += TAIL_THREADS) {
-            int i, j, k;
-            cell_coords(F.L, c, i, j, k);
-            F.e[F.L.id(i, j, k)] += C.e[C.L.id(i / F.cx, j / F.cy, k / F.cz)];
-        }
-        __syncthreads();
-        for (int s = 0; s < F.nu2; ++s) { gs(F, 1); gs(F, 0); }
     }
     if constexpr (sizeof(T) == 4) {
         if (A.top) {
@@ -2173,12 +2100,12 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
         return 32L * M.nx * M.ny * M.nz <= n0 ? nuc : nu;
     };
     // levels [lt, nl) run inside one single-workgroup launch (k_mg_tail) when
-    // they are all small and the coarsest has a dense inverse; else lt = nl
+    // the coarsest has a dense inverse (it then fits by itself); else lt = nl
     int lt = nl, top = 0;
     auto ncell_of = [&](int lv) { return case_cells(c->mg[lv], G.dim); };   // per case
     if (nl > 1 && ncell_of(nl - 1) <= CDENSE) {
-        for (int lv = std::max(l, 1); lv < nl; ++lv)
-            if (ncell_of(lv) <= TAIL_MAX) { lt = lv; break; }
+        for (int lv = std::max(l, 1); lv < nl && lt == nl; ++lv)
+            if (nl - lv <= TAIL_LEVELS && tail_fits(c, lv)) lt = lv;
         // FP32: one more level above, resident in LDS and registers
         if constexpr (sizeof(T) == 4) {
             const int lv = lt - 1;
@@ -2186,13 +2113,12 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
             const int nch = DIM == 3 ? 8 : 4;
             const bool full = F.cx == 2 && F.cy == 2 && (DIM == 2 || F.cz == 2) && F.nx % 2 == 0 &&
                               F.ny % 2 == 0 && (DIM == 2 || F.nz % 2 == 0);
-            if (lt < nl && lv >= std::max(l, 1) && full && ncell_of(lv) <= TAIL_TOP) {
+            if (nl - lv <= TAIL_LEVELS && lv >= std::max(l, 1) && full && ncell_of(lv) <= TAIL_TOP) {
                 const MgLevel &C = c->mg[lv + 1];
                 const long plane = DIM == 3 ? (long)C.nx * C.ny : C.nx;
                 if (nch * (ncell_of(lv + 1) + 2 * plane) <= TAIL_LDS) { lt = lv; top = 1; }
             }
         }
-        if (nl - lt > TAIL_LEVELS) { lt = nl; top = 0; }
     }
     const int ldown = lt < nl ? lt : nl - 1;   // levels smoothed by separate launches: [l, ldown)
     // down
@@ -2270,24 +2196,15 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
             V.nu1 = sweeps(lv, nu1);
             V.nu2 = sweeps(lv, nu2);
         }
-        // the levels below the top keep their error in LDS when their
-        // ghosted boxes fit
-        {
-            int off = 0;
-            bool fit = true;
-            for (int q = A.top; q < A.n; ++q) {
-                const Lay &L = A.lv[q].L;
-                A.eoff[q] = off;
-                off += (L.nx + 2) * (L.ny + 2) * (DIM == 3 ? L.nz + 2 : 1);
-                fit = fit && (long)((L.nx + 1) / 2) * L.ny * (DIM == 3 ? L.nz : 1) <= (long)TAIL_PAIRS * TAIL_THREADS;
-            }
-            A.lds = fit && off <= TAIL_ELDS ? 1 : 0;
+        for (int q = A.top, off = 0; q < A.n; ++q) {
+            A.eoff[q] = off;
+            off += tail_box<DIM>(A.lv[q].L);
         }
         ProfScope ps_(c, R_COARSE);
         hipLaunchKernelGGL((k_mg_tail<T, DIM>), dim3(DIM == 2 ? c->nb : 1), dim3(TAIL_THREADS), 0, c->stream, A);
         FCFD_CHECK(hipGetLastError());
     } else {
-        // coarsest: dense inverse or FP64 CG in one workgroup
+        // coarsest level without a dense inverse: FP64 CG, one workgroup per case
         MgLevel &M = c->mg[nl - 1];
         Lay L = lay_of(M, G.dim);
         Inv2 ih = inv2(M);
@@ -2295,13 +2212,9 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
         arrays(nl - 1, e, f, bx, by, bz);
         long n = case_cells(M, G.dim);
         ProfScope ps_(c, R_COARSE);
-        if (nl > 1 && n <= CDENSE)
-            hipLaunchKernelGGL((k_coarse_dense<T>), dim3(DIM == 2 ? c->nb : 1), dim3(CDENSE), 0, c->stream, e, f,
-                               (const double *)coarse_inv(c), lay_case(M, G.dim), ih, DIM);
-        else   // one workgroup per case
-            hipLaunchKernelGGL((k_coarse_cg<T, DIM>), dim3(DIM == 2 ? c->nb : 1), dim3(n >= 1024 ? 1024 : 256), 0,
-                               c->stream, e, f, bx, by, bz, M.bx64, M.by64, M.bz64, coarse_inv(c),
-                               lay_case(M, G.dim), ih, (int)std::min<long>(n, 96), 0.0);
+        hipLaunchKernelGGL((k_coarse_cg<T, DIM>), dim3(DIM == 2 ? c->nb : 1), dim3(n >= 1024 ? 1024 : 256), 0,
+                           c->stream, e, f, bx, by, bz, M.bx64, M.by64, M.bz64, coarse_inv(c),
+                           lay_case(M, G.dim), ih, (int)std::min<long>(n, 96), 0.0);
         FCFD_CHECK(hipGetLastError());
     }
     // up

@@ -90,3 +90,39 @@ def test_every_tuner_schedule_reaches_the_same_pressure():
         else:
             d = np.abs(p - ref).max() / np.abs(ref).max()
             assert d <= 1e-8, (sched, d)
+
+
+# (grid, separate coarse levels in the FP64 and in the FP32 cycle): 16 x 16 x
+# 16 fits the tail; 15 x 16 x 17 has fewer cells but 2176 pairs for 2048
+# places; 4 x 16 x 64 fits by pairs but its box and the next level's do not
+# share the LDS (the FP32 cycle takes it as its top level); 2D likewise
+TAILS = [((32, 32, 32), 0, 0), ((30, 32, 34), 1, 1), ((8, 32, 128), 1, 0), ((128, 128, 1), 0, 0), ((122, 134, 1), 1, 1)]
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("size,sep64,sep32", TAILS)
+def test_tail_starts_at_a_level_that_fits(size, sep64, sep32, precision):
+    from fortrancfd_amd import Solver
+    from fortrancfd_amd.types import Case
+    from test_gpu_odd_axes import TOL, _solve
+    nx, ny, nz = size
+    case = Case(dim=2 if nz == 1 else 3, nx=nx, ny=ny, nz=nz, xend=1.0, yend=ny / nx, zend=nz / nx,
+                ppe_precision=precision)
+    s = Solver(case)
+    f = np.random.default_rng(3).standard_normal(case.shape)
+    case.interior(f)[...] -= case.interior(f).mean()
+    s.push("rho", np.ones(case.shape))
+    s.push("ppe_src", f)
+    s.push("p", np.zeros(case.shape))
+    s.ppe_sor_init()
+    s.prof_enable(True)
+    _, rel = s.ppe_solve_rhs(TOL, precision)
+    launches = {k: n for k, (_, n) in s.prof_read().items()}
+    assert rel <= TOL
+    assert (launches["mg_smooth_coarse"] > 0) == bool((sep64, sep32)[precision]), launches
+    # and the cycle is as good as on a grid whose levels all fit
+    cyc, rel, res = _solve(size, precision)
+    ref, _, _ = _solve((32, 32, 32) if nz > 1 else (128, 128, 1), precision)
+    print(size, cyc, "reference", ref, "rel", rel, "recomputed", res)
+    assert rel <= TOL and res <= 2 * TOL
+    assert cyc <= ref + 3, (cyc, ref)
