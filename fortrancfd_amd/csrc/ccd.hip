@@ -17,6 +17,7 @@
 // stages them through LDS tiles so that the wave's loads and stores are row
 // segments (measured at 256^3: ~0.35 ms per x sweep, from ~0.88 ms with
 // per-lane strided access; y or z ~0.19 ms).
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
@@ -1027,7 +1028,7 @@ __global__ void __launch_bounds__(WAVE) k_seg_lines_x(const double *__restrict__
 // m_s d'_{s-1}, backward u_s = Dinv_s (d'_s - U_s u_{s+1}), with d_s =
 // (x0(b_s), x0(a_{s+1})) read from zb and u_s = (x(b_s), x(a_{s+1})) written
 // back over them.  This form takes lines of any length, at one memory latency
-// an interface and sweep; the two below take all but the longest.
+// an interface and sweep; the two below take shorter ones (reduce_form).
 __global__ void __launch_bounds__(SEGT) k_seg_reduce(double *__restrict__ zb, const double *__restrict__ red_u,
                                                      const double *__restrict__ red_d, long nl, int P) {
     const long t = (long)blockIdx.x * SEGT + threadIdx.x;
@@ -1094,12 +1095,6 @@ __device__ __forceinline__ double quad_row(const double2 &a, const double2 &b, d
 // wave).  Sums are in k_seg_reduce's order, so the results are its bits.
 constexpr int QL = 16, QT = 256;
 constexpr int QRED_LDS = 65536;   // at QL * 4 + NRED doubles an interface: up to 73 interfaces
-// up to this many blocks are resident at once (8 of 256 threads on each of
-// 256 CUs); k_seg_reduce_r has a quarter of the instructions and wins where
-// the lines alone fill the chip: 65536 lines of 16 interfaces 18.3 us against
-// 23.8, 39200 of 9 interfaces 11.3 against 12; 19600 of 17 14.8 against 11.8,
-// 28800 of 9 10.7 against 8.4, 2048 of 16 10.3 against 6.2
-constexpr long QROUND = 2048;
 __global__ void __launch_bounds__(QT) k_seg_reduce_q(double *__restrict__ zb, const double *__restrict__ red_u,
                                                      const double *__restrict__ red_d, long nl, int P) {
     extern __shared__ double2 qlds[];
@@ -1215,6 +1210,28 @@ __global__ void __launch_bounds__(SEGT) k_seg_reduce_r(double *__restrict__ zb, 
         }
 }
 
+// Which form takes the reduced solve of nl lines of ni interfaces in ns
+// systems.  One wave of k_seg_reduce_q's four sweeps, so it wins while its
+// blocks are resident in a few rounds, and the forms with a line per thread
+// win where the lines alone fill the chip.  At most SEG_MAXI interfaces: one
+// round (8 blocks a CU) against k_seg_reduce_r, which has a quarter of the
+// instructions: 65536 lines of 16 interfaces 23.8 us against 18.3, 39200 of 9
+// interfaces 12 against 11.3; 19600 of 17 11.8 against 14.8, 28800 of 9 8.4
+// against 10.7, 2048 of 16 6.2 against 10.3.  More: three rounds of what LDS
+// holds (8 blocks of 21 interfaces a CU, 5 of 31, 4 of 43, 2 of 68) against
+// k_seg_reduce, in us at lines x systems:
+//   21 interfaces:  67600 35 / 39, 135200 60 / 61, 250000 110 / 106
+//   31:             40000 37 / 47,  80000 64 / 67, 172000 138 / 105
+//   43:             22500 42 / 61,  45000 67 / 75,  90000 107 / 90
+//   68:             10000 40 / 83,  20000 64 / 91,  48400 130 / 112, 96800 246 / 151
+enum { RED_ANY, RED_REG, RED_LDS };
+static int reduce_form(int ni, long nl, int ns, int ncu) {
+    const long blocks = (nl + QL - 1) / QL * ns, lds = (long)ni * (4 * QL + NRED) * (long)sizeof(double);
+    if (ni <= SEG_MAXI) return blocks > 8L * ncu ? RED_REG : RED_LDS;
+    const long resident = std::min(8L, 163840 / lds) * ncu;   // 160 KB of LDS a CU
+    return lds <= QRED_LDS && blocks <= 3 * resident ? RED_LDS : RED_ANY;
+}
+
 // the partitioned solve of the y (dir 1) or z (dir 2) lines: NS = 1 CCD
 // with table k0, NS = 2 UCCD with tables k0 (up) and k1 (down)
 // the partitioned solve of the lines along DIR: NS = 1 CCD with table k0,
@@ -1236,14 +1253,14 @@ static int seg_solve(fcfd_ctx *c, int ext, int k0, int k1, const double *f, cons
         else
             hipLaunchKernelGGL((k_seg_ends<DIR, NS>), dim3((unsigned)P, gx), dim3(SEGT), 0, c->stream, f, c->ccd_z,
                                tu + end_off, td + end_off, G, ext, P);
-        const size_t ql = (size_t)(P - 1) * (4 * QL + NRED) * sizeof(double);
-        const long qblocks = (nl + QL - 1) / QL;
-        if (P - 1 <= SEG_MAXI && qblocks * NS > QROUND)
+        const int form = reduce_form(P - 1, nl, NS, c->ncu);
+        if (form == RED_REG)
             hipLaunchKernelGGL(k_seg_reduce_r<SEG_MAXI>, dim3(gx, NS), dim3(SEGT), 0, c->stream, c->ccd_z,
                                tu + red_off, td + red_off, nl, P);
-        else if (ql <= QRED_LDS)
-            hipLaunchKernelGGL(k_seg_reduce_q, dim3((unsigned)qblocks, NS), dim3(QT), ql, c->stream,
-                               c->ccd_z, tu + red_off, td + red_off, nl, P);
+        else if (form == RED_LDS)
+            hipLaunchKernelGGL(k_seg_reduce_q, dim3((unsigned)((nl + QL - 1) / QL), NS), dim3(QT),
+                               (size_t)(P - 1) * (4 * QL + NRED) * sizeof(double), c->stream, c->ccd_z, tu + red_off,
+                               td + red_off, nl, P);
         else
             hipLaunchKernelGGL(k_seg_reduce, dim3(gx, NS), dim3(SEGT), 0, c->stream, c->ccd_z, tu + red_off,
                                td + red_off, nl, P);
