@@ -82,10 +82,10 @@ def _repeated(n, m, along):
     return [(b.cuda() if along == 0 else b.T.contiguous().cuda()).index_select(along, at) for b in base]
 
 
-# 26 and 58 cells a row: the 32- and the 64-wide tiles, a plane of more than
-# 4 GiB; along 1: rows so long that ten of them (what a tile reads) pass
+# rows of 16010 and 16058 cells (the 32- and the 64-wide tiles), a plane of
+# more than 4 GiB; along 1: rows so long that ten of them (what a tile reads) pass
 # 4 GiB, which takes the instance with 64-bit offsets
-@pytest.mark.parametrize("m,along", [(26, 0), (58, 0), (10, 1)])
+@pytest.mark.parametrize("m,along", [(16010, 0), (16058, 0), (10, 1)])
 def test_plane_over_4gib(m, along):
     from fortrancfd_amd.blocks import Blocks
     if torch.cuda.mem_get_info()[0] < 96 << 30:
@@ -103,7 +103,7 @@ def test_plane_over_4gib(m, along):
         B.close()
         # 2000 cells past the limit, of the same phase in both, far from the walls
         r = (1000 if n == 5000 else 1000 * (full // 1000 + 1)) + 3
-        out.append(phi.narrow(along, r, 2000).narrow(1 - along, 3, m).cpu().numpy())
+        out.append(phi.narrow(along, r, 2000).narrow(1 - along, 3, m).clone())
         del phi, nu, nv
         torch.cuda.empty_cache()
-    assert np.array_equal(out[0], out[1])
+    assert torch.equal(out[0], out[1])
