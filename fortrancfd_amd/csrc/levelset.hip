@@ -646,7 +646,10 @@ int ls_adv_stage_blocks(hipStream_t st, int ncu, const BlockGeom *tab, int nblk,
     const bool off32 = stage_off32(tile_rows(nx), nx + 6, sizeof(double));   // 3 ghosts a side
     const dim3 blk = off32 ? tile_rows(nx) : dim3(64, 4);
     const dim3 tiles((nx + blk.x - 1) / blk.x, (ny + blk.y - 1) / blk.y);
-    const int kc = dim == 3 ? stage_planes((long)tiles.x * tiles.y * nblk, nz, ncu) : 1, kz = (nz + kc - 1) / kc;
+    int kc = dim == 3 ? stage_planes((long)tiles.x * tiles.y * nblk, nz, ncu) : 1;
+    // the blocks' walks share grid.z, whose limit is 65536 (up to 4096 blocks)
+    while ((long)nblk * ((nz + kc - 1) / kc) > 65535) kc *= 2;
+    const int kz = (nz + kc - 1) / kc;
     const dim3 grd(tiles.x, tiles.y, (unsigned)(nblk * kz));
 #define FCFD_SB(D_, X_, O_)                                                                                         \
     hipLaunchKernelGGL((k_ls_adv_stage_blocks<D_, X_, O_>), grd, blk, 0, st, phi, phin, nu, nv, nw, l1, l2, tab, dt, \

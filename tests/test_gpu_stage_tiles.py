@@ -41,7 +41,8 @@ def test_stage_tiles(size):
     assert r <= 1e-12, r
 
 
-@pytest.mark.parametrize("size,nb", [((67, 11, 13), (2, 2, 3)), ((129, 10, 9), (2, 3, 2)), ((70, 31, 1), (3, 4, 1))])
+@pytest.mark.parametrize("size,nb", [((67, 11, 13), (2, 2, 3)), ((129, 10, 9), (2, 3, 2)), ((70, 31, 1), (3, 4, 1)),
+                                     ((48, 48, 4112), (16, 16, 16))])   # walks longer than 16 planes (grid.z)
 def test_blocks_in_one_launch(size, nb):
     from fortrancfd_amd import Solver
     from fortrancfd_amd.blocks import Blocks
