@@ -236,11 +236,7 @@ static int adj_planes(long tiles, int n, int ncu) {
 }
 
 static int adj_scratch(fcfd_ctx *c) {
-    if (c->adj[0]) return FCFD_OK;
-    for (int q = 0; q < 5; ++q) {
-        if (hipMalloc((void **)&c->adj[q], sizeof(double) * c->G.ntot) != hipSuccess) return FCFD_ERR_HIP;
-        if (hipMemsetAsync(c->adj[q], 0, sizeof(double) * c->G.ntot, c->stream) != hipSuccess) return FCFD_ERR_HIP;
-    }
+    for (auto &p : c->adj) FCFD_TRY(alloc_once(&p, c->G.ntot, true, c->stream));
     return FCFD_OK;
 }
 
@@ -304,11 +300,7 @@ int ls_adv_adjoint_step(fcfd_ctx *c, const double *phi, double *lambda, double *
 int ls_adv_adjoint_step_f32(fcfd_ctx *c, const float *phi, float *lambda, float *ub, float *vb, float *wb,
                             const float *nu, const float *nv, const float *nw) {
     const Geom &G = c->G;
-    if (!c->adj32[0])
-        for (int q = 0; q < 7; ++q) {
-            FCFD_CHECK(hipMalloc((void **)&c->adj32[q], sizeof(float) * G.ntot));
-            FCFD_CHECK(hipMemsetAsync(c->adj32[q], 0, sizeof(float) * G.ntot, c->stream));
-        }
+    for (auto &p : c->adj32) FCFD_TRY(alloc_once(&p, G.ntot, true, c->stream));
     float *phi1 = c->adj32[0], *phi2 = c->adj32[1], *lam1 = c->adj32[2], *lam2 = c->adj32[3], *w = c->adj32[4];
     float *l1 = c->adj32[5], *l2 = c->adj32[6];
     ProfScope ps_(c, R_LS_ADV);

@@ -265,12 +265,15 @@ int stack_scratch(fcfd_blocks *B) {
                     h.push_back(g);
                 }
         FCFD_CHECK(hipDeviceGetAttribute(&B->ncu, hipDeviceAttributeMultiprocessorCount, B->device));
-        FCFD_CHECK(hipMalloc((void **)&B->tab, sizeof(BlockGeom) * h.size()));
-        FCFD_CHECK(hipMemcpy(B->tab, h.data(), sizeof(BlockGeom) * h.size(), hipMemcpyHostToDevice));
+        BlockGeom *tab = nullptr;
+        FCFD_CHECK(hipMalloc((void **)&tab, sizeof(BlockGeom) * h.size()));
+        if (hipMemcpy(tab, h.data(), sizeof(BlockGeom) * h.size(), hipMemcpyHostToDevice) != hipSuccess) {
+            hipFree(tab);
+            return FCFD_ERR_HIP;
+        }
+        B->tab = tab;
     }
-    if (B->a) return FCFD_OK;
-    for (double **p : {&B->a, &B->b, &B->l1, &B->l2})
-        FCFD_CHECK(hipMalloc((void **)p, sizeof(double) * B->total));
+    for (double **p : {&B->a, &B->b, &B->l1, &B->l2}) FCFD_TRY(alloc_once(p, B->total));
     return FCFD_OK;
 }
 
@@ -394,10 +397,8 @@ extern "C" int fcfd_blocks_check_per(fcfd_blocks *B, const double *stack, double
     if (!B || !stack || !err) return FCFD_ERR_ARG;
     const dim3 grd = blk_grid(B);
     const long np = (long)grd.x * grd.y;
-    if (!B->part) {
-        FCFD_CHECK(hipMalloc((void **)&B->part, sizeof(double) * np));
-        B->part_host.resize(np);
-    }
+    FCFD_TRY(alloc_once(&B->part, np));
+    B->part_host.resize(np);
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(k_blocks_check_per, grd, dim3(256), 0, st, stack, B->part, B->D);
     FCFD_CHECK(hipGetLastError());

@@ -392,6 +392,22 @@ constexpr int RES_STRIDE = 16, RES_LAMBDA = 8, RES_VDIV = 9, DIAG_W = 11;
 template <int DIM>
 __device__ __forceinline__ int case_of(int k) { return DIM == 2 ? k : 0; }
 
+// n elements on first use, cleared on st where asked.  *p stays null unless
+// all of it succeeded, so that a call after one that ran out of memory asks
+// again: each array of a set is tested by itself, never the set by its first.
+template <typename T>
+inline int alloc_once(T **p, long n, bool clear = false, hipStream_t st = nullptr) {
+    if (*p) return FCFD_OK;
+    T *q = nullptr;
+    FCFD_CHECK(hipMalloc((void **)&q, sizeof(T) * n));
+    if (clear && hipMemsetAsync(q, 0, sizeof(T) * n, st) != hipSuccess) {
+        (void)hipFree(q);
+        return FCFD_ERR_HIP;
+    }
+    *p = q;
+    return FCFD_OK;
+}
+
 // launch helpers --------------------------------------------------------
 // 256-thread block for rows of w threads: 64 x 4, or 32 x 8 where that
 // leaves fewer lanes idle past the row end (140 cells: 160 instead of 192

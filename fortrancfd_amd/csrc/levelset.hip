@@ -730,8 +730,7 @@ int ls_adv_stage_f32(fcfd_ctx *c, const float *phi, float *phin, const float *nu
 // array, no ghosts), then the zero-gradient ghost copy as in ls_advect.
 int ls_advect_f32(fcfd_ctx *c, float *phi, const float *nu, const float *nv, const float *nw) {
     const Geom &G = c->G;
-    if (!c->adv32[0])
-        for (int q = 0; q < 4; ++q) FCFD_CHECK(hipMalloc((void **)&c->adv32[q], sizeof(float) * G.ntot));
+    for (auto &p : c->adv32) FCFD_TRY(alloc_once(&p, G.ntot));
     float *B = c->adv32[0], *Cb = c->adv32[1], *l1 = c->adv32[2], *l2 = c->adv32[3];
     float *in[3] = {phi, B, Cb}, *out[3] = {B, Cb, phi};
     for (int s = 0; s < 3; ++s) {

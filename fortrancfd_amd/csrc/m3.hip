@@ -524,10 +524,7 @@ int m3_fields(fcfd_ctx *c) {
     // the kernels number the interior cells in 32 bits (grid_flat)
     if (c->G.dim != 3 || !flat_fits(c->G)) return FCFD_ERR_ARG;
     for (int f : {FCFD_PHI1, FCFD_PHI2, FCFD_RHO_OLD, FCFD_MU_OLD})
-        if (!c->f[f]) {
-            FCFD_CHECK(hipMalloc((void **)&c->f[f], sizeof(double) * c->G.ntot));
-            FCFD_CHECK(hipMemsetAsync(c->f[f], 0, sizeof(double) * c->G.ntot, c->stream));
-        }
+        FCFD_TRY(alloc_once(&c->f[f], c->G.ntot, true, c->stream));
     return FCFD_OK;
 }
 
