@@ -107,8 +107,10 @@ static Split split_of(const Geom &G) {
 
 // 1/h^2 per axis, and what an axis paired from an odd number of cells
 // changes at its far end.  The last aggregate of such an axis has one child:
-// it is w = 1/2 of a cell wide (on coarser levels 1/4 .. 1), and its flux
-// balance per cell volume is that of the full-width one divided by w.  So in
+// it is half as wide as that child, w of a cell, and stays narrow further
+// down: w = 2^-m after m odd levels in a row (an axis of 129 cells reaches
+// 1/64 at 3 cells), (1 + w) / 2 below an even one.  Its flux balance per cell
+// volume is that of the full-width one divided by w.  So in
 // its own row the inner face (the only open one of that axis) has the
 // coefficient / w (xl = x / w), its volume is w, and restriction weighs it by
 // that.  The coarse operator times the cell volumes is then symmetric and the
