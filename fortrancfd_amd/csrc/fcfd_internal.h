@@ -302,7 +302,7 @@ __device__ __forceinline__ double block_max256(double v, double *sh4) {
 struct BandList {
     unsigned *cnt;    // [3 stages][NXCD]
     unsigned *tile;   // [NXCD][cap]
-    unsigned cap;
+    unsigned cap, ncu;
     // list the calling block's tile when any of its threads holds a band cell
     __device__ __forceinline__ void append(int stage, int hold, unsigned id) const {
         hold = __syncthreads_or(hold);
@@ -337,12 +337,20 @@ struct BandList {
     }
 };
 
-// the band cells of up to BAND_TILES listed tiles (entries first .. of
-// `total`), collected by a 256-thread block so that it can work on them with
-// full waves: cell[0 .. n) = slot * 256 + thread slot within the tile.
+// the band cells of `per` listed tiles (entries first .. of `total`, at most
+// BAND_TILES), collected by a 256-thread block so that it can work on them
+// with full waves: cell[0 .. n) = slot * 256 + thread slot within the tile.
 // cell_of(tile, thread slot, i, j, k) places a cell (false: none there),
-// inside(phi) is the band test.
+// inside(phi) is the band test.  A block takes no more tiles than give every
+// CU a block, so that a short list is spread over the chip: with 8 whatever
+// the list, 64 x 128 cells that all lie in the band were 4 blocks, and a
+// pseudo step took 82 us instead of 43 (384 x 768, 4 % of the cells: 77
+// instead of 53).
 constexpr int BAND_TILES = 8;
+__device__ __forceinline__ int band_per(const BandList &band, unsigned total) {
+    const unsigned n = (total + band.ncu - 1) / band.ncu;
+    return n < 1 ? 1 : (n > BAND_TILES ? BAND_TILES : (int)n);
+}
 struct BandCells {
     unsigned tile[BAND_TILES];
     unsigned short cell[BAND_TILES * 256];
@@ -350,10 +358,10 @@ struct BandCells {
 };
 template <typename CellOf, typename Inside>
 __device__ __forceinline__ void band_collect(BandCells &sh, const BandList &band, int stage, unsigned first,
-                                             unsigned total, const double *__restrict__ phi, const Geom &G,
+                                             unsigned total, int per, const double *__restrict__ phi, const Geom &G,
                                              CellOf cell_of, Inside inside) {
     const int t = threadIdx.x + threadIdx.y * blockDim.x;
-    if (t < BAND_TILES) sh.tile[t] = band.entry(stage, first + t);
+    if (t < BAND_TILES) sh.tile[t] = t < per ? band.entry(stage, first + t) : 0u;
     if (t == 0) sh.n = 0;
     __syncthreads();
     double p[BAND_TILES];
@@ -361,7 +369,7 @@ __device__ __forceinline__ void band_collect(BandCells &sh, const BandList &band
 #pragma unroll
     for (int s = 0; s < BAND_TILES; ++s) {
         int i, j, k;
-        const bool in = cell_of(sh.tile[s], t, i, j, k) && first + s < total;
+        const bool in = cell_of(sh.tile[s], t, i, j, k) && s < per && first + s < total;
         p[s] = phi[in ? G.id(i, j, k) : G.id(0, 0, 0)];
         have |= in ? 1u << s : 0u;
     }
@@ -481,12 +489,13 @@ inline dim3 grid_interior(const Geom &G, dim3 blk) {
 // the band lists of a launch of ntiles 256-thread blocks (the context holds
 // room for the larger of its tiled and its flat launch over the interior)
 inline BandList band_lists(const fcfd_ctx *c, long ntiles) {
-    return BandList{c->band, c->band + 3 * NXCD, (unsigned)((ntiles + NXCD - 1) / NXCD)};
+    return BandList{c->band, c->band + 3 * NXCD, (unsigned)((ntiles + NXCD - 1) / NXCD), (unsigned)c->ncu};
 }
-// blocks that share the listed tiles: up to 4 per CU
+// blocks that share the listed tiles: one per tile up to one per CU, then as
+// many as BAND_TILES each take, up to 4 per CU
 inline dim3 band_grid(const fcfd_ctx *c, long ntiles) {
-    const long n = (ntiles + BAND_TILES - 1) / BAND_TILES, most = 4L * c->ncu;
-    return dim3((unsigned)(n < most ? n : most));
+    const long few = ntiles < c->ncu ? ntiles : c->ncu, n = (ntiles + BAND_TILES - 1) / BAND_TILES, most = 4L * c->ncu;
+    return dim3((unsigned)(n < few ? few : (n < most ? n : most)));
 }
 
 // kernels implemented in the .hip files (host wrappers)

@@ -880,7 +880,7 @@ __global__ void __launch_bounds__(256) k_redis_stage(const double *__restrict__ 
 // correction (redis_lambda :385-408), source and update as in k_redis_stage.
 // A term outside the band is 0 (its delta is) and is not stored: it is read
 // all the same and not selected, so that the loads of a plane issue together.
-// A block takes BAND_TILES listed tiles at a time (tiles of gx x gy blocks a
+// A block takes up to BAND_TILES listed tiles at a time (tiles of gx x gy blocks a
 // plane) and works on their band cells with full waves (band_collect): a
 // band is a few cells thick, so about a tenth of a listed tile's lanes hold
 // one.  18 us at 160 x 144 x 200.  One column of 16 planes per thread, tangent to the band,
@@ -906,9 +906,10 @@ __global__ void __launch_bounds__(256) k_redis_band(const double *__restrict__ p
         k = (int)k_;
         return i < G.nx && j < G.ny;
     };
-    for (unsigned g = blockIdx.x * BAND_TILES; g < total; g += gridDim.x * BAND_TILES) {
+    const int per = band_per(band, total);
+    for (unsigned g = blockIdx.x * per; g < total; g += gridDim.x * per) {
         if (t < BAND_TILES) s_err[t] = 0ull;
-        band_collect(sh, band, STAGE, g, total, phi, G, cell_of, [&](double p) { return in_band(p, iw); });
+        band_collect(sh, band, STAGE, g, total, per, phi, G, cell_of, [&](double p) { return in_band(p, iw); });
         for (int c = t; c < sh.n; c += 256) {
             const int slot = sh.cell[c] / 256;
             int i, j, k;
@@ -961,7 +962,7 @@ __global__ void __launch_bounds__(256) k_redis_band(const double *__restrict__ p
                 atomicMax(&s_err[slot], (unsigned long long)__double_as_longlong(fabs(pst - pn)));
         }
         __syncthreads();
-        if (STAGE == 2 && t < BAND_TILES && g + t < total) {
+        if (STAGE == 2 && t < per && g + t < total) {
             const int q = case_of<DIM>((int)(sh.tile[t] / gx / gy));
             atomicMax(&flags[(long)q * FLAG_STRIDE + FLAG_SHARD0 + sh.tile[t] % NSHARD], s_err[t]);
         }

@@ -224,8 +224,9 @@ __global__ void __launch_bounds__(M3_BT) k_m3_redis_band(const double *__restric
         k = (int)kk;
         return t < n;
     };
-    for (unsigned first = blockIdx.x * BAND_TILES; first < total; first += gridDim.x * BAND_TILES) {
-        band_collect(sh, band, STAGE, first, total, T, G, cell_of, [&](double p) { return m3_in_band(p, w); });
+    const int per = band_per(band, total);
+    for (unsigned first = blockIdx.x * per; first < total; first += gridDim.x * per) {
+        band_collect(sh, band, STAGE, first, total, per, T, G, cell_of, [&](double p) { return m3_in_band(p, w); });
         for (int c = threadIdx.x; c < sh.n; c += M3_BT) {
             int i, j, k;
             cell_of(sh.tile[sh.cell[c] / 256], sh.cell[c] % 256, i, j, k);

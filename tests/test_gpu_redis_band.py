@@ -35,6 +35,25 @@ def _phi(case, kind):
     return np.ascontiguousarray(sum(X) - 2.0 * case.dx)
 
 
+@pytest.mark.parametrize("size,per", [((40, 40, 80), 4), ((8, 8, 1900), 8)])
+def test_redis_band_tiles_per_block(size, per):
+    """lists of 800 and 1900 tiles, so 4 and 8 tiles a block on 256 CUs (the
+    grids above: 1), with a band that holds every cell"""
+    from fortrancfd_amd import Solver
+    nx, ny, nz = size
+    case = case3d(nx, ls_w=8000.0)
+    case.ny, case.nz, case.zend = ny, nz, nz * case.dx
+    phi = bubble(case, 0.3, 1)
+    s, o = Solver(case), Oracle(case)
+    Oracle.threads(8)
+    s.push("phi", phi)
+    o.set("phi", phi)
+    assert s.level_set_rk3_redis(1) > 0
+    o.call("level_set_rk3_redis", 1)
+    Oracle.threads(1)
+    assert max_rel(s.pull("phi"), o.get("phi")) <= 1e-11
+
+
 @pytest.mark.parametrize("tag,mk", GRIDS)
 @pytest.mark.parametrize("kind", ["thin", "none", "all", "ghosts", "corner"])
 def test_redis_band(tag, mk, kind):
