@@ -298,13 +298,16 @@ __device__ __forceinline__ double block_max256(double v, double *sh4) {
 // block appending to list (block id % NXCD), with a counter per stage and
 // list (one counter would serialise the appends).  A list can hold every
 // block that appends to it.  The order of a list does not matter: every band
-// cell is independent of the others.
+// cell is independent of the others.  A grid of no more tiles than CUs is not
+// listed: all tiles are taken (all > 0), which saves the append and two
+// memory latencies of the band pass.
 struct BandList {
     unsigned *cnt;    // [3 stages][NXCD]
     unsigned *tile;   // [NXCD][cap]
-    unsigned cap, ncu;
+    unsigned cap, ncu, all;
     // list the calling block's tile when any of its threads holds a band cell
     __device__ __forceinline__ void append(int stage, int hold, unsigned id) const {
+        if (all) return;
         hold = __syncthreads_or(hold);
         if (hold && threadIdx.x + threadIdx.y == 0) {
             const unsigned q = (blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)) % NXCD;
@@ -312,6 +315,7 @@ struct BandList {
         }
     }
     __device__ __forceinline__ unsigned total(int stage) const {
+        if (all) return all;
         unsigned n = 0;
 #pragma unroll
         for (unsigned q = 0; q < NXCD; ++q) n += cnt[stage * NXCD + q];
@@ -319,6 +323,7 @@ struct BandList {
     }
     // entry `at` of the lists taken end to end
     __device__ __forceinline__ unsigned entry(int stage, unsigned at) const {
+        if (all) return at;
         for (unsigned q = 0; q < NXCD; ++q) {
             const unsigned n = cnt[stage * NXCD + q];
             if (at < n) return tile[q * cap + at];
@@ -489,7 +494,8 @@ inline dim3 grid_interior(const Geom &G, dim3 blk) {
 // the band lists of a launch of ntiles 256-thread blocks (the context holds
 // room for the larger of its tiled and its flat launch over the interior)
 inline BandList band_lists(const fcfd_ctx *c, long ntiles) {
-    return BandList{c->band, c->band + 3 * NXCD, (unsigned)((ntiles + NXCD - 1) / NXCD), (unsigned)c->ncu};
+    return BandList{c->band, c->band + 3 * NXCD, (unsigned)((ntiles + NXCD - 1) / NXCD), (unsigned)c->ncu,
+                    ntiles <= c->ncu ? (unsigned)ntiles : 0u};
 }
 // blocks that share the listed tiles: one per tile up to one per CU, then as
 // many as BAND_TILES each take, up to 4 per CU

@@ -35,23 +35,49 @@ def _phi(case, kind):
     return np.ascontiguousarray(sum(X) - 2.0 * case.dx)
 
 
-@pytest.mark.parametrize("size,per", [((40, 40, 80), 4), ((8, 8, 1900), 8)])
-def test_redis_band_tiles_per_block(size, per):
-    """lists of 800 and 1900 tiles, so 4 and 8 tiles a block on 256 CUs (the
-    grids above: 1), with a band that holds every cell"""
+# The grids above have no more tiles than CUs and are not listed; these have
+# 512, 800 and 1900 tiles.  "all": every cell in the band (2, 4 and 8 tiles a
+# block on 256 CUs).
+LISTED = [(256, 512, 1), (40, 40, 80), (8, 8, 1900)]
+
+
+@pytest.mark.parametrize("kind", ["thin", "none", "all"])
+@pytest.mark.parametrize("size", LISTED)
+def test_redis_band_lists(size, kind):
     from fortrancfd_amd import Solver
     nx, ny, nz = size
-    case = case3d(nx, ls_w=8000.0)
-    case.ny, case.nz, case.zend = ny, nz, nz * case.dx
-    phi = bubble(case, 0.3, 1)
+    kw = {"ls_w": 8000.0} if kind == "all" else {}
+    case = case2d(nx, **kw) if nz == 1 else case3d(nx, **kw)
+    if nz > 1:
+        case.ny, case.nz, case.zend = ny, nz, nz * case.dx
+    phi = _phi(case, kind)
     s, o = Solver(case), Oracle(case)
     Oracle.threads(8)
     s.push("phi", phi)
     o.set("phi", phi)
-    assert s.level_set_rk3_redis(1) > 0
+    it = s.level_set_rk3_redis(1)
     o.call("level_set_rk3_redis", 1)
+    assert it == o.diag()["redis_iters"]
     Oracle.threads(1)
     assert max_rel(s.pull("phi"), o.get("phi")) <= 1e-11
+
+
+def test_redis_band_lists_of_a_batch():
+    """six cases of 75 x 150 cells have 342 tiles and are listed, one alone has
+    57 and is not: bit for bit the same"""
+    from fortrancfd_amd import Solver
+    from fortrancfd_amd.solver import BatchSolver
+    case = case2d(75, name="batch")
+    phis = [bubble(case, 0.1 * q, q) for q in range(6)]
+    b = BatchSolver([case2d(75, name="batch") for _ in phis])
+    b.push("phi", np.stack(phis))
+    b.level_set_rk3_redis(1)
+    got = b.pull("phi")
+    for q, phi in enumerate(phis):
+        s = Solver(case)
+        s.push("phi", phi)
+        s.level_set_rk3_redis(1)
+        assert np.array_equal(got[q], s.pull("phi").reshape(case.shape)), q
 
 
 @pytest.mark.parametrize("tag,mk", GRIDS)
