@@ -2108,18 +2108,21 @@ static int vcycle(fcfd_ctx *c, int l, T *e0, const T *f0, const T *rho0, int nu1
     if (nl > 1 && ncell_of(nl - 1) <= CDENSE) {
         for (int lv = std::max(l, 1); lv < nl && lt == nl; ++lv)
             if (nl - lv <= TAIL_LEVELS && tail_fits(c, lv)) lt = lv;
-        // FP32: one more level above, resident in LDS and registers
+        // FP32: one more level above, resident in LDS and registers; or the
+        // first level itself where it would have two pairs a thread (24 x 24
+        // x 48 cells: 0.74 ms a solve by pairs, 0.69 this way; 32^3 0.76 and
+        // 0.68; 128 x 128 0.73 and 0.66)
         if constexpr (sizeof(T) == 4) {
-            const int lv = lt - 1;
-            const MgLevel &F = c->mg[lv];
-            const int nch = DIM == 3 ? 8 : 4;
-            const bool full = F.cx == 2 && F.cy == 2 && (DIM == 2 || F.cz == 2) && F.nx % 2 == 0 &&
-                              F.ny % 2 == 0 && (DIM == 2 || F.nz % 2 == 0);
-            if (nl - lv <= TAIL_LEVELS && lv >= std::max(l, 1) && full && ncell_of(lv) <= TAIL_TOP) {
-                const MgLevel &C = c->mg[lv + 1];
-                const long plane = DIM == 3 ? (long)C.nx * C.ny : C.nx;
-                if (nch * (ncell_of(lv + 1) + 2 * plane) <= TAIL_LDS) { lt = lv; top = 1; }
-            }
+            auto can_top = [&](int lv) {
+                if (lv < std::max(l, 1) || lv + 1 >= nl || nl - lv > TAIL_LEVELS) return false;
+                const MgLevel &F = c->mg[lv], &C = c->mg[lv + 1];
+                const long nch = DIM == 3 ? 8 : 4, plane = DIM == 3 ? (long)C.nx * C.ny : C.nx;
+                const bool full = F.cx == 2 && F.cy == 2 && (DIM == 2 || F.cz == 2) && F.nx % 2 == 0 &&
+                                  F.ny % 2 == 0 && (DIM == 2 || F.nz % 2 == 0);
+                return full && ncell_of(lv) <= TAIL_TOP && nch * (ncell_of(lv + 1) + 2 * plane) <= TAIL_LDS;
+            };
+            if (can_top(lt - 1)) { lt -= 1; top = 1; }
+            else if (ncell_of(lt) > TAIL_MAX / 2 && can_top(lt)) top = 1;
         }
     }
     const int ldown = lt < nl ? lt : nl - 1;   // levels smoothed by separate launches: [l, ldown)

@@ -95,8 +95,10 @@ def test_every_tuner_schedule_reaches_the_same_pressure():
 # (grid, separate coarse levels in the FP64 and in the FP32 cycle): 16 x 16 x
 # 16 fits the tail; 15 x 16 x 17 has fewer cells but 2176 pairs for 2048
 # places; 4 x 16 x 64 fits by pairs but its box and the next level's do not
-# share the LDS (the FP32 cycle takes it as its top level); 2D likewise
-TAILS = [((32, 32, 32), 0, 0), ((30, 32, 34), 1, 1), ((8, 32, 128), 1, 0), ((128, 128, 1), 0, 0), ((122, 134, 1), 1, 1)]
+# share the LDS (the FP32 cycle takes it as its top level); 2D likewise.  14 x
+# 15 x 18 fits with two pairs a thread in both precisions, 16 x 16 x 16 is the
+# FP32 cycle's top level
+TAILS = [((32, 32, 32), 0, 0), ((28, 30, 36), 0, 0), ((30, 32, 34), 1, 1), ((8, 32, 128), 1, 0), ((128, 128, 1), 0, 0), ((122, 134, 1), 1, 1)]
 
 
 @pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
