@@ -1782,7 +1782,14 @@ int mg_free(fcfd_ctx *c) {
     return mg_drop_graphs(c);
 }
 
+// A solve returns with its last iteration, or one queued ahead in vain, still
+// in flight: its graph is destroyed only once the stream has run it.
 int mg_drop_graphs(fcfd_ctx *c) {
+    bool any = false;
+    for (auto &s : c->vgraph)
+        for (auto &a : s)
+            for (hipGraphExec_t g : a) any = any || g;
+    if (any) FCFD_CHECK(hipStreamSynchronize(c->stream));
     for (int a = 0; a < 4; ++a)
         for (int b = 0; b < 5; ++b) {
             for (int s = 0; s < 2; ++s) {

@@ -4,48 +4,14 @@ a stand-in that counts them and fails one on request).  A call that runs out
 of memory reports it and launches nothing; the next one allocates what is
 missing before it launches."""
 import os
-import subprocess
-import sys
 
 import pytest
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-LIB = os.path.join(ROOT, "fortrancfd_amd", "libfcfd.so")
+import hip_standin
 
-STANDIN = r"""
-#include <stddef.h>
-#include <stdlib.h>
-static int calls, fail_at, live, launches;
-static int hit(void) { return ++calls == fail_at; }
-void standin_reset(int n) { calls = live = launches = 0; fail_at = n; }
-int standin_live(void) { return live; }
-int standin_launches(void) { return launches; }
-int hipMalloc(void **p, size_t n) { (void)n; if (hit()) return 2; *p = malloc(16); ++live; return 0; }
-int hipMemcpy(void *d, const void *s, size_t n, int k) { (void)d; (void)s; (void)n; (void)k; return hit() ? 1 : 0; }
-int hipFree(void *p) { free(p); --live; return 0; }
-int hipGetDevice(int *d) { *d = 0; return 0; }
-int hipDeviceGetAttribute(int *v, int a, int d) { (void)a; (void)d; *v = 256; return 0; }
-int hipGetLastError(void) { return 0; }
-const char *hipGetErrorString(int e) { (void)e; return "stand-in"; }
-typedef struct { unsigned x, y, z; } d3;
-int __hipPushCallConfiguration(d3 g, d3 b, size_t s, void *st) { (void)g; (void)b; (void)s; (void)st; return 0; }
-int __hipPopCallConfiguration(d3 *g, d3 *b, size_t *s, void **st) { d3 o = {1, 1, 1}; *g = *b = o; *s = 0; *st = 0; return 0; }
-int hipLaunchKernel(const void *f, d3 g, d3 b, void **a, size_t s, void *st) {
-    (void)f; (void)g; (void)b; (void)a; (void)s; (void)st;
-    ++launches;
-    return 0;
-}
-"""
-
-DRIVER = r"""
-import ctypes as C, sys
-sys.path.insert(0, sys.argv[1])
-hip = C.CDLL(sys.argv[2], mode=C.RTLD_GLOBAL)   # ahead of the library's own HIP runtime
-lib = C.CDLL(sys.argv[3])
-from fortrancfd_amd.types import Case
+BODY = r"""
 case = Case(dim=3, nx=12, ny=12, nz=12)
 grid, params = case.grid_struct(), case.param_struct()
-vp = C.c_void_p
 lib.fcfd_blocks_create.argtypes = [vp, vp] + [C.c_int] * 6 + [vp]
 lib.fcfd_blocks_level_set_rk3_solver.argtypes = [vp] * 6
 lib.fcfd_blocks_destroy.argtypes = [vp]
@@ -65,10 +31,6 @@ print("done")
 """
 
 
-@pytest.mark.skipif(not os.path.exists(LIB), reason="libfcfd.so not built (fortrancfd_amd/build.py)")
+@pytest.mark.skipif(not os.path.exists(hip_standin.LIB), reason="libfcfd.so not built (fortrancfd_amd/build.py)")
 def test_blocks_step_after_a_failed_allocation(tmp_path):
-    src, so = tmp_path / "standin.c", tmp_path / "standin.so"
-    src.write_text(STANDIN)
-    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", str(so), str(src)], check=True)
-    r = subprocess.run([sys.executable, "-c", DRIVER, ROOT, str(so), LIB], capture_output=True, text=True)
-    assert r.returncode == 0 and r.stdout.strip() == "done", r.stdout + r.stderr
+    hip_standin.run(tmp_path, BODY)
