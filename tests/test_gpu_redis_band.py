@@ -1,5 +1,6 @@
 """The reinitialisation's split into cells outside the interface band (finished
-by the stage kernel) and band cells (collected from listed tiles), against the
+by the stage kernel) and band cells (collected from the tiles, which are listed
+on grids of more tiles than CUs), against the
 oracle: grids whose tiles are cut off, level sets whose band is empty, thin,
 the whole box or one tile, and ghosts that are no copies of the boundary cells
 (the first stage reads phi(-1)).
