@@ -1,9 +1,8 @@
 """The reinitialisation's split into cells outside the interface band (finished
 by the stage kernel) and band cells (collected from the tiles, which are listed
-on grids of more tiles than CUs), against the
-oracle: grids whose tiles are cut off, level sets whose band is empty, thin,
-the whole box or one tile, and ghosts that are no copies of the boundary cells
-(the first stage reads phi(-1)).
+on grids of more tiles than CUs), against the oracle: grids whose tiles are cut
+off, level sets whose band is empty, thin, the whole box or one tile, and
+ghosts that are no copies of the boundary cells (the first stage reads phi(-1)).
 
 Tolerance 1e-11 of the field's max, as for the reinitialisation tests of
 test_gpu_parity.py (31 pseudo-steps of WENO5 with sin/cos of another library).
